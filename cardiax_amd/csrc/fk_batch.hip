@@ -49,6 +49,7 @@ struct SimDesc {
   Coef c;
   const float* D;
   float* buf[2][3];  // ping-pong state: [parity][v, w, u]
+  float* user[3];    // the caller's state buffers
   int H, W;
   int n_stim;
   float dt, inv_dx2;
@@ -187,18 +188,47 @@ k_batch_step_t(const SimDesc* __restrict__ sims, const TileItem* __restrict__ it
 #undef FK_BT2
 }
 
+// n floats from src to dst, blocks [blk, blk + stride, ...) of 1024: 16-byte
+// moves where both pointers allow them.
+__device__ __forceinline__ void copy_cells(float* __restrict__ dst, const float* __restrict__ src,
+                                           size_t n, size_t blk, size_t stride) {
+  const bool wide = (((uintptr_t)dst | (uintptr_t)src) & 15) == 0;
+  const size_t n4 = wide ? n / 4 : 0;
+  for (size_t i = blk * 256 + threadIdx.x; i < n4; i += stride * 256)
+    ((float4*)dst)[i] = ((const float4*)src)[i];
+  for (size_t i = 4 * n4 + blk * 256 + threadIdx.x; i < n; i += stride * 256) dst[i] = src[i];
+}
+
+// The whole batch's state between the callers' buffers and a pool, one launch
+// in place of one copy per field (768 copies of 2.4 us for 256 simulations,
+// 1.85 ms; 26.1 M cells now take 0.15 ms). blockIdx.y strides over the
+// fields: LOAD callers -> pool 0 and resets the step counter; else pool
+// `parity` -> callers and moves every simulation's time on by n_steps.
+constexpr int kCopyBlocks = 16;  // blocks per field and launch row
+
+template <bool LOAD>
+__global__ void __launch_bounds__(256)
+k_batch_copy(SimDesc* __restrict__ sims, int n, int parity, int64_t* __restrict__ step_base,
+             int64_t n_steps) {
+  for (int64_t y = blockIdx.y; y < 3 * (int64_t)n; y += gridDim.y) {
+    SimDesc& S = sims[y / 3];
+    const int f = (int)(y % 3);
+    const size_t cells = (size_t)S.H * S.W;
+    if (LOAD)
+      copy_cells(S.buf[0][f], S.user[f], cells, blockIdx.x, kCopyBlocks);
+    else
+      copy_cells(S.user[f], S.buf[parity][f], cells, blockIdx.x, kCopyBlocks);
+    if (!LOAD && f == 0 && blockIdx.x == 0 && threadIdx.x == 0) S.t0 += (double)n_steps;
+  }
+  if (LOAD && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *step_base = 0;
+}
+
 __global__ void k_batch_bump(int64_t* step_base, int64_t by) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *step_base += by;
 }
 
 __global__ void k_batch_set(int64_t* step_base, int64_t value) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *step_base = value;
-}
-
-// After a run: every simulation's next first step is n_steps later.
-__global__ void k_batch_advance(SimDesc* sims, int n, int64_t n_steps) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) sims[i].t0 += (double)n_steps;
 }
 
 }  // namespace fk
@@ -346,6 +376,9 @@ int32_t fk_batch_create(const fk_sim* sims, int32_t n, fk_batch** out) {
     const size_t cells = (size_t)s.H * s.W;
     for (int p = 0; p < 2; ++p)
       for (int f = 0; f < 3; ++f) d.buf[p][f] = b->pool[p] + 3 * b->offset[i] + f * cells;
+    d.user[0] = s.v;
+    d.user[1] = s.w;
+    d.user[2] = s.u;
     d.H = s.H;
     d.W = s.W;
     d.n_stim = s.n_stimuli;
@@ -528,16 +561,8 @@ int32_t fk_batch_run(fk_batch* b, int64_t n_steps, int32_t use_graph, void* stre
   for (int i = 0; i < b->n_sims; ++i)
     if (!check_time(b->host_sims[i].t, b->host_sims[i].t + (double)n_steps)) return last_code();
   hipStream_t s = (hipStream_t)stream;
-  // state in: caller buffers -> pool 0
-  for (int i = 0; i < b->n_sims; ++i) {
-    const fk_sim& sm = b->host_sims[i];
-    const size_t cells = (size_t)sm.H * sm.W;
-    float* dst = b->pool[0] + 3 * b->offset[i];
-    HIP_CHECK(hipMemcpyAsync(dst, sm.v, cells * 4, hipMemcpyDeviceToDevice, s));
-    HIP_CHECK(hipMemcpyAsync(dst + cells, sm.w, cells * 4, hipMemcpyDeviceToDevice, s));
-    HIP_CHECK(hipMemcpyAsync(dst + 2 * cells, sm.u, cells * 4, hipMemcpyDeviceToDevice, s));
-  }
-  k_batch_set<<<1, 64, 0, s>>>(b->d_step, 0);
+  const dim3 cg(kCopyBlocks, (unsigned)std::min<int64_t>(3 * (int64_t)b->n_sims, 65535));
+  k_batch_copy<true><<<cg, 256, 0, s>>>(b->d_sims, b->n_sims, 0, b->d_step, 0);
   HIP_CHECK(hipGetLastError());
   int64_t k = 0;
   int parity = 0;
@@ -555,19 +580,10 @@ int32_t fk_batch_run(fk_batch* b, int64_t n_steps, int32_t use_graph, void* stre
     HIP_CHECK(batch_chunk(b, b->opt, n, &parity, s));
     k += n;
   }
-  // state out: final pool -> caller buffers
-  for (int i = 0; i < b->n_sims; ++i) {
-    const fk_sim& sm = b->host_sims[i];
-    const size_t cells = (size_t)sm.H * sm.W;
-    const float* src = b->pool[parity] + 3 * b->offset[i];
-    HIP_CHECK(hipMemcpyAsync(sm.v, src, cells * 4, hipMemcpyDeviceToDevice, s));
-    HIP_CHECK(hipMemcpyAsync(sm.w, src + cells, cells * 4, hipMemcpyDeviceToDevice, s));
-    HIP_CHECK(hipMemcpyAsync(sm.u, src + 2 * cells, cells * 4, hipMemcpyDeviceToDevice, s));
-  }
+  k_batch_copy<false><<<cg, 256, 0, s>>>(b->d_sims, b->n_sims, parity, b->d_step, n_steps);
+  HIP_CHECK(hipGetLastError());
   // the simulations' times advance by n_steps for a later run
   for (auto& sm : b->host_sims) sm.t += (double)n_steps;
-  k_batch_advance<<<(b->n_sims + 255) / 256, 256, 0, s>>>(b->d_sims, b->n_sims, n_steps);
-  HIP_CHECK(hipGetLastError());
   return FK_OK;
 }
 
