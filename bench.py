@@ -286,7 +286,7 @@ def bench_adjoint(seed, size=256, n_steps=2000, frame_every=50, reps=2):
                                 "achieved": round(fwd_adj, 1),
                                 "frac": round(fwd_adj / HBM_PEAK_GBS, 4)},
             "roofline": dict(leg_roofline(ADJ_BWD_BYTES * size * size, per_step,
-                                          "k_adj_main<true>", "%dx%d" % shape),
+                                          "k_adj_rev<2>", "%dx%d" % shape),
                              design_bytes_per_launch=ADJ_BWD_DESIGN_BYTES * size * size),
             "grad_finite": bool(torch.isfinite(D.grad).all().item())}
 
@@ -297,14 +297,13 @@ def bench_adjoint(seed, size=256, n_steps=2000, frame_every=50, reps=2):
 # and its recompute from the checkpoints (28).
 ADJ_BWD_BYTES = 48
 ADJ_FWD_BWD_BYTES = 104
-# What the fused reverse kernel moves by construction per cell: it also reads
-# the derived fields of its step (28), lam_v/lam_w, v, w, u, D, dL/dD and the
-# previous u (32 more in all) and writes the next step's derived fields (28).
-ADJ_BWD_DESIGN_BYTES = 104
+# What the reverse kernel moves by construction per cell: nothing more, beside
+# the halo rows and columns of its windows of u, D and lam_u.
+ADJ_BWD_DESIGN_BYTES = 48
 
 
 def adjoint_step_seconds(st, prm, D, stims, shape, t_mid, n_short=10, n_long=40):
-    """Time of one reverse step (k_adj_main<true>) on the stream it runs on:
+    """Time of one reverse step (k_adj_rev<2>) on the stream it runs on:
     fk_adjoint_segment over n_long and n_short steps of a trajectory from the
     middle of the rollout, HIP events around each; the difference cancels the
     segment's fixed launches."""

@@ -1,29 +1,55 @@
-// Device side of the adjoint of one forward-Euler step (the reverse step, its
-// derived fields and the boundary tables of the transposed operators), shared
-// by the per-grid kernels (fk_adjoint.hip) and the batched rollout
-// (fk_rollout_batch.hip): one code path, so both give identical bits.
-// The mathematics is described at the top of fk_adjoint.hip.
+// Device side of the adjoint of one forward-Euler step, shared by the per-grid
+// kernel (fk_adjoint.hip) and the batched rollout (fk_rollout_batch.hip): one
+// code path, so both give identical bits. The mathematics is described at the
+// top of fk_adjoint.hip.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
-#include "fk_device.h"
+#include <type_traits>
+
+#include "fk_stream.h"
 
 namespace fk {
 
-constexpr int kAdjB = 8;       // tabulated rows at each edge
-constexpr int kAdjSlots = 16;  // 2 * kAdjB
-constexpr int kAdjBand = 5;    // |column - row| <= 5 in A1, A2
+// The per-axis operators A1 = crop G pad and A2 = crop G G pad of an axis of N
+// cells (G: the gradient rule of cardiax/solve.py:230-250, one-sided on the two
+// outermost padded entries of each side). Away from the edges their rows are
+// central stencils. The rows of the kAdjB cells nearest each edge, and the
+// transposed rows of the kAdjT cells nearest it, come from a table.
+constexpr int kAdjB = 8, kAdjT = 13;
+constexpr int kA1 = 3, kA2 = 5;  // |column - row| <= 3 in A1, <= 5 in A2
+constexpr int kAdjSlots = 2 * kAdjT;
 
-// Tables of one axis: row slot -> A1[row][row + d], A2[row][row + d], d in [-5, 5].
-struct AdjAxisTab {
-  float a1[kAdjSlots][2 * kAdjBand + 1];
-  float a2[kAdjSlots][2 * kAdjBand + 1];
+struct AdjRow {
+  float a1[8], a2[12];  // A[i][i + d], d = -3 .. 3 and -5 .. 5 (and padding)
+  float t1[8], t2[12];  // A[i - d][i]
+};
+struct alignas(16) AdjAxisTab {
+  AdjRow r[kAdjSlots];
 };
 
-// Gradient rule of cardiax/solve.py:230-250 as a matrix on n padded entries:
-// the coefficient of entry q in row p.
-__device__ __forceinline__ double g_coef(int p, int q, int n) {
+// Whether cell i lies within B of an edge (of a short axis: any cell).
+__host__ __device__ inline bool adj_near(int i, int N, int B) {
+  return N <= 2 * B || i < B || i >= N - B;
+}
+// Table row of a cell within kAdjT of an edge.
+__host__ __device__ inline int adj_slot(int i, int N) {
+  return N <= kAdjSlots || i < kAdjT ? i : i - (N - kAdjSlots);
+}
+
+// Central rows of A1 (d = -2..2) and A2 (d = -4..4).
+#define FK_A1(d) ((d) == -2 ? 1.0f / 12.0f : (d) == -1 ? -2.0f / 3.0f : (d) == 1 ? 2.0f / 3.0f : (d) == 2 ? -1.0f / 12.0f : 0.0f)
+#define FK_A2(d)                                                                          \
+  ((d) == 0 ? -65.0f / 72.0f                                                              \
+            : ((d) == 1 || (d) == -1) ? 1.0f / 9.0f                                       \
+            : ((d) == 2 || (d) == -2) ? 4.0f / 9.0f                                       \
+            : ((d) == 3 || (d) == -3) ? -1.0f / 9.0f                                      \
+            : ((d) == 4 || (d) == -4) ? 1.0f / 144.0f : 0.0f)
+
+// Gradient rule as a matrix on n padded entries: the coefficient of entry q in
+// row p.
+__host__ __device__ inline double g_coef(int p, int q, int n) {
   const int d = q - p;
   if (p <= 1) {
     const double c[4] = {-11.0 / 6.0, 3.0, -1.5, 1.0 / 3.0};
@@ -38,238 +64,98 @@ __device__ __forceinline__ double g_coef(int p, int q, int n) {
 }
 
 // Edge padding as a matrix: padded entry q takes original cell clamp(q-1).
-__device__ __forceinline__ double pad_coef(int q, int i, int N) {
+__host__ __device__ inline double pad_coef(int q, int i, int N) {
   int s = q - 1;
   s = s < 0 ? 0 : (s > N - 1 ? N - 1 : s);
   return s == i ? 1.0 : 0.0;
 }
 
-__device__ __forceinline__ int adj_slot(int i, int N) {
-  if (N <= kAdjSlots) return i;
-  if (i < kAdjB) return i;
-  if (i >= N - kAdjB) return i - (N - kAdjSlots);
-  return -1;
-}
-
-// A1[j][j + d] and A2[j][j + d] (0 outside the band or the grid).
-struct AxisOps {
-  const AdjAxisTab* T;
-  int N;
-  __device__ float a1(int j, int d) const {
-    const int s = adj_slot(j, N);
-    if (s >= 0) return T->a1[s][d + kAdjBand];
-    const float c[5] = {1.0f / 12.0f, -2.0f / 3.0f, 0.0f, 2.0f / 3.0f, -1.0f / 12.0f};
-    return (d >= -2 && d <= 2) ? c[d + 2] : 0.0f;
+// A1[j][i] and A2[j][i] (0 off the axis): the rules composed exactly for the
+// rows near an edge, the central stencils elsewhere.
+__host__ __device__ inline void adj_coef(int j, int i, int N, float& a1, float& a2) {
+  a1 = a2 = 0.0f;
+  if (j < 0 || j >= N || i < 0 || i >= N) return;
+  const int d = i - j;
+  if (!adj_near(j, N, kAdjB)) {
+    a1 = FK_A1(d);
+    a2 = FK_A2(d);
+    return;
   }
-  __device__ float a2(int j, int d) const {
-    const int s = adj_slot(j, N);
-    if (s >= 0) return T->a2[s][d + kAdjBand];
-    const float c[9] = {1.0f / 144.0f, -1.0f / 9.0f, 4.0f / 9.0f, 1.0f / 9.0f, -65.0f / 72.0f,
-                        1.0f / 9.0f,   4.0f / 9.0f,  -1.0f / 9.0f, 1.0f / 144.0f};
-    return (d >= -4 && d <= 4) ? c[d + 4] : 0.0f;
+  const int n = N + 2, pj = j + 1;  // padded row of original j
+  double s1 = 0.0, s2 = 0.0;
+  for (int q = pj - 3; q <= pj + 3; ++q) {
+    if (q < 0 || q >= n) continue;
+    const double gq = g_coef(pj, q, n);
+    if (gq == 0.0) continue;
+    s1 += gq * pad_coef(q, i, N);
+    double gp = 0.0;  // A2 = crop G G pad: row pj of G times column i of G pad
+    for (int s = q - 3; s <= q + 3; ++s)
+      if (s >= 0 && s < n) gp += g_coef(q, s, n) * pad_coef(s, i, N);
+    s2 += gq * gp;
   }
-};
-
-
-constexpr int kAdjThreads = 256;
-
-// Central stencils of the untabulated rows: A1 = G (d = -2..2) and A2 = G G
-// (d = -4..4).
-#define FK_A1(d) ((d) == -2 ? 1.0f / 12.0f : (d) == -1 ? -2.0f / 3.0f : (d) == 1 ? 2.0f / 3.0f : (d) == 2 ? -1.0f / 12.0f : 0.0f)
-#define FK_A2(d)                                                                          \
-  ((d) == 0 ? -65.0f / 72.0f                                                              \
-            : ((d) == 1 || (d) == -1) ? 1.0f / 9.0f                                       \
-            : ((d) == 2 || (d) == -2) ? 4.0f / 9.0f                                       \
-            : ((d) == 3 || (d) == -3) ? -1.0f / 9.0f                                      \
-            : ((d) == 4 || (d) == -4) ? 1.0f / 144.0f : 0.0f)
-
-// A1[j][j + d] and A2[j][j + d] without branches on the memory path: the
-// table entry is always loaded (slot clamped into range) and then selected,
-// so unrolled loops issue every load up front. Zero when j is off the axis.
-__device__ __forceinline__ void band_coef(const AdjAxisTab& T, int j, int d, int N, float& a1,
-                                          float& a2) {
-  const bool on = j >= 0 && j < N;
-  const int s = adj_slot(on ? j : 0, N);
-  const int sc = s < 0 ? 0 : s;
-  const float t1 = T.a1[sc][d + kAdjBand], t2 = T.a2[sc][d + kAdjBand];
-  a1 = !on ? 0.0f : (s >= 0 ? t1 : FK_A1(d));
-  a2 = !on ? 0.0f : (s >= 0 ? t2 : FK_A2(d));
+  a1 = (float)s1;
+  a2 = (float)s2;
 }
 
-// Row j of an axis of N cells uses the central stencils (not a table row).
-__device__ __forceinline__ bool central_row(int j, int N) { return adj_slot(j, N) < 0; }
-// Every row within the band of j is central, so (A^T q)(j) uses the
-// transposed central stencils only.
-__device__ __forceinline__ bool central_cone(int j, int N) {
-  return N > kAdjSlots && j >= kAdjB + kAdjBand && j < N - kAdjB - kAdjBand;
+// Sums of taps in the order of d. dL/dD adds L A2 u and A1^T (L A1 u), which
+// nearly cancel, so it carries the rounding of these sums many times over: two
+// differences of differences in their place take fewer operations, but moved
+// dL/dD by 7e-5 over 500 steps and gained under 2 us of 29.
+// sum_d A1(d) x[s d], x[0] the centre; s = -1 the transposed row.
+template <int s>
+__device__ __forceinline__ float a1_sum(const float* x) {
+  float g = FK_A1(-2) * x[-2 * s];
+  g = fmaf(FK_A1(-1), x[-s], g);
+  g = fmaf(FK_A1(1), x[s], g);
+  return fmaf(FK_A1(2), x[2 * s], g);
 }
 
-// Fields the reverse step derives from u and the incoming cotangent before
-// applying the transposed operators: L = lam_u (+ injected cotangent),
-// lap = A2x u + A2y u, Q2 = D L, Q1x = D_x L, Px = L (A1x u), Q1y = D_y L,
-// Py = L (A1y u). Fields read together are stored as pairs.
-struct AdjPre {
-  float2* Llap;  // (L, lap)
-  float2* QPx;   // (Q1x, Px)
-  float2* QPy;   // (Q1y, Py)
-  float* Q2;
-};
-
-// Inputs of the derived fields of one cell: u at offsets -5..5 along both
-// axes (clamped into the grid; the coefficients there are 0), D, D_x, D_y.
-struct PreIn {
-  float xs[2 * kAdjBand + 1], ys[2 * kAdjBand + 1];
-  float D, Dx, Dy;
-};
-
-__device__ __forceinline__ void pre_load(const float* __restrict__ u,
-                                         const float* __restrict__ D,
-                                         const float* __restrict__ Dx,
-                                         const float* __restrict__ Dy, int i, int c, int H,
-                                         int W, PreIn& in) {
-  const size_t idx = (size_t)i * W + c;
+__device__ __forceinline__ float a2_sum(const float* x) {
+  float g = FK_A2(-4) * x[-4];
 #pragma unroll
-  for (int d = -kAdjBand; d <= kAdjBand; ++d) {
-    in.xs[d + kAdjBand] = u[(size_t)clampi(i + d, 0, H - 1) * W + c];
-    in.ys[d + kAdjBand] = u[(size_t)i * W + clampi(c + d, 0, W - 1)];
+  for (int d = -3; d <= 4; ++d) g = fmaf(FK_A2(d), x[d], g);
+  return g;
+}
+
+// The same with a table row, each product rounded.
+__device__ __forceinline__ float tab_sum(const float* t, const float* x, int n) {
+#pragma clang fp contract(off)
+  float g = 0.0f;
+#pragma unroll
+  for (int d = -n; d <= n; ++d) g = g + t[d + n] * x[d];
+  return g;
+}
+
+// sum_d A2(d) y2[-d] + A1(d) y1[-d]: the transposed diffusion operators.
+__device__ __forceinline__ float at_sum(const float* y2, const float* y1) {
+  float g = 0.0f;
+#pragma unroll
+  for (int d = -4; d <= 4; ++d) {
+    g = fmaf(FK_A2(d), y2[-d], g);
+    if (d >= -2 && d <= 2 && d != 0) g = fmaf(FK_A1(d), y1[-d], g);
   }
-  in.D = D[idx];
-  in.Dx = Dx[idx];
-  in.Dy = Dy[idx];
+  return g;
 }
 
-// The derived fields of one cell, given its cotangent L (lam_u plus any
-// injected cotangent) and the loaded inputs. lap is the axis-0 sum plus the
-// axis-1 sum, the order k_adj_main uses too.
-// Per-axis pieces of the derived fields of the previous step: A1 u and A2 u
-// at position i of an axis of N cells, from u at offsets -5..5 along the axis
-// (clamped into the grid; the coefficients there are 0).
-__device__ __forceinline__ void axis_pre(const float* __restrict__ xs, int i, int N,
-                                         const AdjAxisTab& T, float& g, float& lap) {
-  g = 0.0f;
-  lap = 0.0f;
-  if (central_row(i, N)) {
+// A value and its neighbours up to n columns away: x[n + d] is column + d.
+template <int n>
+__device__ __forceinline__ void lane_window(float y, float x[2 * n + 1]) {
+  x[n] = y;
 #pragma unroll
-    for (int d = -4; d <= 4; ++d) {
-      lap += FK_A2(d) * xs[d + kAdjBand];
-      g += FK_A1(d) * xs[d + kAdjBand];
-    }
-  } else {
-#pragma unroll
-    for (int d = -kAdjBand; d <= kAdjBand; ++d) {
-      float a1, a2;
-      band_coef(T, i, d, N, a1, a2);
-      const bool on = i + d >= 0 && i + d < N;
-      g += on ? a1 * xs[d + kAdjBand] : 0.0f;
-      lap += on ? a2 * xs[d + kAdjBand] : 0.0f;
-    }
+  for (int d = 1; d <= n; ++d) {
+    x[n + d] = from_right(x[n + d - 1]);
+    x[n - d] = from_left(x[n - d + 1]);
   }
 }
 
+constexpr int kRevOut = 54;   // output columns per wave: 5 halo lanes on each side
+constexpr int kRevHalo = 5;   // what an edge's rules reach (4 away from the edges)
 
-__device__ __forceinline__ void pre_store(const PreIn& in, float L, int i, int c, int H, int W,
-                                          const AdjAxisTab* tab, const AdjPre& o) {
-  const size_t idx = (size_t)i * W + c;
-  float gx, lapx, gy, lapy;
-  axis_pre(in.xs, i, H, tab[0], gx, lapx);
-  axis_pre(in.ys, c, W, tab[1], gy, lapy);
-  o.Llap[idx] = make_float2(L, lapx + lapy);
-  o.QPx[idx] = make_float2(in.Dx * L, L * gx);
-  o.QPy[idx] = make_float2(in.Dy * L, L * gy);
-  o.Q2[idx] = in.D * L;
-}
-
-// The boundary tables of both axes staged in LDS by the whole block (one
-// barrier) when the block holds a cell within 13 cells of an edge: the edge
-// paths then read coefficients from LDS and only their field loads go to
-// memory, all independent of each other. Interior blocks (the condition is
-// block-uniform) skip the staging and never read the tables.
-__device__ __forceinline__ void stage_tables(const AdjAxisTab* __restrict__ tab, int H, int W,
-                                             int rows, AdjAxisTab* s_tab, int bx, int by) {
-  const int r0 = by * rows, c0 = bx * 64;
-  const bool interior = central_cone(r0, H) && central_cone(r0 + rows - 1, H) &&
-                        central_cone(c0, W) && central_cone(c0 + 63, W);
-  if (interior) return;
-  const float* src = (const float*)tab;
-  float* dst = (float*)s_tab;
-  constexpr int n = (int)(2 * sizeof(AdjAxisTab) / sizeof(float));
-  for (int k = threadIdx.x; k < n; k += blockDim.x) dst[k] = src[k];
-  __syncthreads();
-}
-
-// The derived fields of one cell of the block at (bx, by) of k_adj_pre's grid
-// (64 columns x 4 rows): L = lam_u (+ injected cotangent) and the fields of
-// pre_store. `tab` is the block's LDS.
-__device__ __forceinline__ void adj_pre_tile(const float* __restrict__ u,
-                                             const float* __restrict__ D,
-                                             const float* __restrict__ Dx,
-                                             const float* __restrict__ Dy,
-                                             const float* __restrict__ lu,
-                                             const float* __restrict__ inj, int H, int W,
-                                             const AdjAxisTab* __restrict__ tab_g,
-                                             const AdjPre& o, int bx, int by, AdjAxisTab* tab) {
-  stage_tables(tab_g, H, W, 4, tab, bx, by);
-  const int c = bx * 64 + (threadIdx.x & 63);
-  const int i = by * 4 + (threadIdx.x >> 6);
-  if (i >= H || c >= W) return;
-  const size_t idx = (size_t)i * W + c;
-  PreIn in;
-  pre_load(u, D, Dx, Dy, i, c, H, W, in);
-  pre_store(in, inj ? lu[idx] + inj[idx] : lu[idx], i, c, H, W, tab, o);
-}
-
-// What the reverse step of t+k-1 needs from the step of t+k: the state
-// x_{t+k-1}'s u and the cotangent injected into x_{t+k} (may be null).
-struct AdjNext {
-  const float* u_prev;
-  const float* inj;
-  const float *D, *Dx, *Dy;
-  AdjPre pre;
-};
-
-// Transposed operators along one axis at position i (stride between
-// neighbours `step` elements, base index `idx` of position i):
-// s = A2^T(Q2) + A1^T(Q1), e = A1^T(P), with (Q1, P) stored as pairs.
-__device__ __forceinline__ void axis_transpose(const float* __restrict__ Q2,
-                                               const float2* __restrict__ QP, size_t idx,
-                                               ptrdiff_t step, int i, int N, const AdjAxisTab& T,
-                                               float& sv, float& ev) {
-  sv = 0.0f;
-  ev = 0.0f;
-  if (central_cone(i, N)) {
-#pragma unroll
-    for (int d = -4; d <= 4; ++d) {
-      const size_t j = idx - (ptrdiff_t)d * step;
-      sv += FK_A2(d) * Q2[j];
-      if (d >= -2 && d <= 2 && d != 0) {
-        const float2 q = QP[j];
-        sv += FK_A1(d) * q.x;
-        ev += FK_A1(d) * q.y;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int d = -kAdjBand; d <= kAdjBand; ++d) {
-      const int jr = i - d;
-      float a1, a2;
-      band_coef(T, jr, d, N, a1, a2);  // 0 when jr is off the axis
-      const size_t j = idx + (ptrdiff_t)(clampi(jr, 0, N - 1) - i) * step;
-      const float2 q = QP[j];
-      sv += a2 * Q2[j] + a1 * q.x;
-      ev += a1 * q.y;
-    }
-  }
-}
-
-// Index of x wave `xw` (0 or 1) of the block at (bx, by) of k_adj_main's grid
-// (gx blocks wide) among all x waves of the grid: one tau accumulator each.
-__device__ __forceinline__ size_t adj_wave_index(int bx, int by, int gx, int xw) {
-  return ((size_t)by * gx + bx) * 2 + (size_t)xw;
-}
-
-// Number of x waves (tau accumulators) of k_adj_main on an H x W grid.
-__host__ __device__ inline size_t adj_n_waves(int H, int W) {
-  return (size_t)((W + 63) / 64) * (size_t)((H + 1) / 2) * 2;
+// Tau accumulators: one triple of doubles per strip and pair of rows, so that
+// the sums do not depend on the band height.
+__host__ __device__ inline int adj_strips(int W) { return (W + kRevOut - 1) / kRevOut; }
+__host__ __device__ inline size_t adj_n_groups(int H, int W) {
+  return (size_t)adj_strips(W) * (size_t)((H + 1) / 2);
 }
 
 // Stimulus fields of one step as an active list (count(), on(m), field(m)).
@@ -280,152 +166,291 @@ struct AdjStimList {
   __device__ const float* field(int m) const { return sa.f[m]; }
 };
 
-// One reverse step from the derived fields, two threads per cell in
-// different waves of a block of 64 columns x 2 rows: the "x" thread loads and
-// applies the transposed operators along axis 0, evaluates the reaction's
-// adjoint and writes every output; the "y" thread applies those along axis 1
-// (and, with NEXT, derives the axis-1 part of the previous step's fields) and
-// hands its 4 results over through LDS (one barrier). Twice the waves and half
-// the dependency chain per wave: the step is latency-bound on small grids.
-// The tau-gradient contributions of the 64 cells of an x wave are summed
-// across the wave (a fixed butterfly) and lane 0 adds the three sums to the
-// wave's own double accumulator g_tau[wave]: 24 bytes per 64 cells per step,
-// deterministic (each accumulator is touched by one wave, in step order).
-// NEXT: also write the derived fields of the previous step's reverse (they
-// depend on the new cotangent only at the same cell), so a segment needs one
-// launch per step.
-// The block at (bx, by) of a grid gx blocks wide; `tab` and `xch` are the
-// block's LDS. Every thread of the block calls it (one barrier inside).
-template <bool NEXT, class SV>
-__device__ __forceinline__ void adj_main_tile(
-    const Coef& c, const float* __restrict__ v, const float* __restrict__ w,
-    const float* __restrict__ u, int H, int W, const SV& sv, float dt, float inv_dx2,
-    const float* __restrict__ lv, const float* __restrict__ lw, const AdjPre& pre,
-    float* __restrict__ lv_o, float* __restrict__ lw_o, float* __restrict__ lu_o,
-    float* __restrict__ gD, double* __restrict__ g_tau, const AdjAxisTab* __restrict__ tab_g,
-    const AdjNext& nx, int bx, int by, int gx, AdjAxisTab* tab, float4* xch) {
-  stage_tables(tab_g, H, W, 2, tab, bx, by);
-  const bool ythread = threadIdx.x >= kAdjThreads / 2;  // wave-uniform
-  const int q = threadIdx.x & (kAdjThreads / 2 - 1);
-  const int col = bx * 64 + (q & 63);
-  const int i = by * 2 + (q >> 6);
-  const bool in = i < H && col < W;
-  const size_t idx = in ? (size_t)i * W + col : 0;
+// Sum over the wave's 64 lanes, valid in lane 63: a fixed tree of DPP moves
+// (no LDS). The lanes without a source add 0.
+__device__ __forceinline__ float wave_sum63(float x) {
+  auto add = [](float a, auto ctrl, auto rows) {
+    const int m = __builtin_amdgcn_update_dpp(0, __float_as_int(a), decltype(ctrl)::value,
+                                              decltype(rows)::value, 0xf, false);
+    return a + __int_as_float(m);
+  };
+  using std::integral_constant;
+  x = add(x, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr:1
+  x = add(x, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});  // row_shr:2
+  x = add(x, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});  // row_shr:4
+  x = add(x, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});  // row_shr:8
+  x = add(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row_bcast:15
+  x = add(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row_bcast:31
+  return x;
+}
 
-  // x-thread state (kept across the barrier)
-  float xs[2 * kAdjBand + 1];
-  float nD = 0.0f, nDx = 0.0f, nDy = 0.0f, inj = 0.0f;
-  float vv = 0.0f, ww = 0.0f, uu = 0.0f, lvv = 0.0f, lww = 0.0f, L = 0.0f, lap = 0.0f;
-  float sx = 0.0f, ex = 0.0f, gx_n = 0.0f, lapx_n = 0.0f;
-  float gd = 0.0f;
-  bool stim = false;
-  if (ythread) {
-    float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (in) {
-      float ys[2 * kAdjBand + 1];
-      if (NEXT) {
-        const float* urow = nx.u_prev + (size_t)i * W;
+struct AdjArgs {
+  const float *v, *w, *u, *D;        // the state of the step, the D-map
+  const float *lv, *lw, *lu, *inj;   // cotangent of the next state; inj (may be null) adds to lu
+  float *lv_o, *lw_o, *lu_o, *gD;    // cotangent of this state; dL/dD (accumulated)
+  double* g_tau;                     // tau accumulators
+  const AdjAxisTab* tab;             // rows, columns
+};
+
+// One reverse step of the band of R rows (even) at rs of the strip at cs: one
+// wave, lane l on column cs - 5 + l, rows walked as the forward streaming tile
+// walks them: windows of u, D and the cotangent L = lu + inj in registers,
+// column neighbours by DPP, no LDS. The fields that the transposed operators
+// read (D L, D_x L, L u_x and the same along y) are formed from those windows,
+// so a reverse step reads and writes only what it must (state 12 bytes,
+// cotangent 12 in and 12 out, D 4, dL/dD 8: 48 per cell, and the windows' halo
+// rows). It replaced a kernel that kept seven derived fields in memory (104
+// bytes by design, 121-142 measured), two threads per cell:
+// 59.1 us before, 28.9 now per step of 12 problems of 128^2 to 512^2 (1.26 M
+// cells); 61 us for 3.84 M cells (3.0 TB/s of the 48 bytes); 7.05 and 7.0 at
+// 256^2, where a launch and an edge wave's own instructions bound both.
+// XG, YG: a row within 13 of an edge, a column within 13 of a side. In such a
+// band each row, and in such a strip each lane, takes the table or the central
+// taps by itself, so neither the band height nor the strip changes a bit.
+// tab: the wave's LDS copy of the tables, filled here where they are used (read
+// from memory one row after another they were most of an edge wave's time: a
+// dozen dependent scalar loads, 33 us in place of 29 for the 12 problems).
+template <int R, bool XG, bool YG, class SV>
+__device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H, int W,
+                                         const SV& sv, float dt, float inv_dx2, int rs, int cs,
+                                         AdjAxisTab* tab) {
+#pragma clang fp contract(off)
+  static_assert(R % 2 == 0, "tau groups are pairs of rows");
+  constexpr int E = XG ? kRevHalo : 4;  // window rows above and below the band
+  constexpr int NW = R + 2 * E, NG = NW - 4;  // window; its first differences
+  const int lane = threadIdx.x & 63;
+  const int col = cs - kRevHalo + lane;
+  const bool in_col = col >= 0 && col < W;
+  // the lane's cell near a side, and its table row
+  const bool nearB = YG && in_col && adj_near(col, W, kAdjB);
+  const bool nearT = YG && in_col && adj_near(col, W, kAdjT);
+  const int tslot = nearT ? adj_slot(col, W) : 0;
+  const uint32_t off = (uint32_t)(YG ? clampi(col, 0, W - 1) : col) * 4u;
+  auto at = [&](const float* f, int r) {
+    return ld(f + (size_t)(XG ? clampi(r, 0, H - 1) : r) * (size_t)W, off);
+  };
+
+  constexpr int kTab4 = (int)(sizeof(AdjAxisTab) / sizeof(f32x4)), kTabN = (kTab4 + 63) / 64;
+  f32x4 tx[XG ? kTabN : 1], ty[YG ? kTabN : 1];
 #pragma unroll
-        for (int d = -kAdjBand; d <= kAdjBand; ++d)
-          ys[d + kAdjBand] = urow[clampi(col + d, 0, W - 1)];
-      }
-      axis_transpose(pre.Q2, pre.QPy, idx, 1, col, W, tab[1], r.x, r.y);
-      if (NEXT) axis_pre(ys, col, W, tab[1], r.z, r.w);
-    }
-    xch[q] = r;
-  } else if (in) {
-    // x thread: everything that does not need the y results
-    if (NEXT) {  // issued first: independent of everything below
-#pragma unroll
-      for (int d = -kAdjBand; d <= kAdjBand; ++d)
-        xs[d + kAdjBand] = nx.u_prev[(size_t)clampi(i + d, 0, H - 1) * W + col];
-      nD = nx.D[idx];
-      nDx = nx.Dx[idx];
-      nDy = nx.Dy[idx];
-      if (nx.inj) inj = nx.inj[idx];
-    }
-    vv = v[idx];
-    ww = w[idx];
-    uu = u[idx];
-    const float2 Llap = pre.Llap[idx];
-    L = Llap.x;
-    lap = Llap.y;
-    lvv = lv[idx];
-    lww = lw[idx];
-    gd = gD[idx];
-    for (int k = 0; k < sv.count(); ++k) stim = stim || (sv.on(k) && sv.field(k)[idx] != 0.0f);
-    axis_transpose(pre.Q2, pre.QPx, idx, W, i, H, tab[0], sx, ex);
-    if (NEXT) axis_pre(xs, i, H, tab[0], gx_n, lapx_n);
+  for (int k = 0; k < kTabN; ++k) {
+    const uint32_t o = (uint32_t)min(64 * k + lane, kTab4 - 1);
+    if constexpr (XG) tx[k] = ((const f32x4 __attribute__((address_space(1)))*)(gcbytes)a.tab)[o];
+    if constexpr (YG)
+      ty[k] = ((const f32x4 __attribute__((address_space(1)))*)(gcbytes)(a.tab + 1))[o];
   }
-  __syncthreads();  // every thread of the block passes this one barrier
-  if (ythread) return;  // whole waves: the x waves stay complete for the tau sums
-  float t_d = 0.0f, t_r = 0.0f, t_si = 0.0f;  // this cell's tau-gradient terms
-  if (in) {
-    const float4 yr = xch[q];
-    const float sy = yr.x, ey = yr.y;
+  float uu[NW], dd[NW], LL[NW];
+#pragma unroll
+  for (int k = 0; k < NW; ++k) uu[k] = at(a.u, rs - E + k);
+#pragma unroll
+  for (int k = 0; k < NW; ++k) LL[k] = at(a.lu, rs - E + k);
+#pragma unroll
+  for (int k = 0; k < NW; ++k) dd[k] = at(a.D, rs - E + k);
+  if (a.inj) {
+#pragma unroll
+    for (int k = 0; k < NW; ++k) LL[k] = LL[k] + at(a.inj, rs - E + k);
+  }
+  float vv[R], ww[R], lvv[R], lww[R], gd[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    vv[k] = at(a.v, rs + k);
+    ww[k] = at(a.w, rs + k);
+    lvv[k] = at(a.lv, rs + k);
+    lww[k] = at(a.lw, rs + k);
+    gd[k] = at(a.gD, rs + k);
+  }
+  if constexpr (XG || YG) {
+#pragma unroll
+    for (int k = 0; k < kTabN; ++k) {
+      const int o = min(64 * k + lane, kTab4 - 1);
+      if constexpr (XG) ((f32x4*)&tab[0])[o] = tx[k];
+      if constexpr (YG) ((f32x4*)&tab[1])[o] = ty[k];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // read by this wave only
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (XG || YG) {  // no cotangent beyond the grid
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+      const int i = rs - E + k;
+      LL[k] = (!XG || (i >= 0 && i < H)) && (!YG || in_col) ? LL[k] : 0.0f;
+    }
+  }
 
-    // --- reaction, gates as fixed masks -----------------------------------
-    const bool p = uu >= c.V_c;
-    const float inv_tvm = (uu >= c.V_v) ? c.inv_tv2m : c.inv_tv1m;
-    const float dfv_dv = p ? -c.inv_tvp : -inv_tvm;
-    const float dfw_dw = p ? -c.inv_twp : -c.inv_twm;
-    const float S = half_one_plus_tanh(c, uu);  // (1 + tanh(k (u - V_csi))) / 2
+  // A1 of a window at its entry m, row r; `fused`: of the D-map
+  auto slope = [&](const float* x, int m, int r, bool fused) {
+    if (XG && r >= 0 && r < H && adj_near(r, H, kAdjB)) {
+      const float* t = tab[0].r[adj_slot(r, H)].a1;
+      float g = 0.0f;
+#pragma unroll
+      for (int d = -kA1; d <= kA1; ++d)
+        if (m + d >= 0 && m + d < NW) {  // taps beyond the window are 0
+          const float y = x[m + d];
+          g = fused ? fmaf(t[d + kA1], y, g) : g + t[d + kA1] * y;
+        }
+      return g;
+    }
+    return a1_sum<1>(x + m);
+  };
+  // Q2 = D L; u_x, P = L u_x and Q1 = D_x L
+  float q2[NW], pp[NG], q1[NG];
+#pragma unroll
+  for (int k = 0; k < NW; ++k) q2[k] = dd[k] * LL[k];
+#pragma unroll
+  for (int k = 0; k < NG; ++k) {
+    const int m = k + 2, r = rs - E + m;
+    pp[k] = LL[m] * slope(uu, m, r, false);
+    q1[k] = slope(dd, m, r, true) * LL[m];
+  }
+
+  float ts[3];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int i = rs + k, m = k + E, mf = m - 2;  // row, its entries in the windows
+    const float uc = uu[m], L = LL[m];
+    // along the rows: A2 u, s = A2^T Q2 + A1^T Q1, e = A1^T P
+    float lapx, sx, ex;
+    if (XG && i < H && adj_near(i, H, kAdjB))
+      lapx = tab_sum(tab[0].r[adj_slot(i, H)].a2, uu + m, kA2);
+    else
+      lapx = a2_sum(uu + m);
+    if (XG && i < H && adj_near(i, H, kAdjT)) {
+      const AdjRow& t = tab[0].r[adj_slot(i, H)];
+      sx = ex = 0.0f;
+#pragma unroll
+      for (int d = -kA2; d <= kA2; ++d) {
+        if (d >= -kA1 && d <= kA1) {
+          sx = fmaf(t.t1[d + kA1], q1[mf - d], sx);
+          ex = fmaf(t.t1[d + kA1], pp[mf - d], ex);
+        }
+        sx = fmaf(t.t2[d + kA2], q2[m - d], sx);
+      }
+    } else {
+      sx = at_sum(q2 + m, q1 + mf);
+      ex = a1_sum<-1>(pp + mf);
+    }
+    // along the columns
+    float lapy, sy, ey;
+    if constexpr (!YG) {
+      float x[9], z[5], y2[9], y1[5], yp[5];
+      lane_window<4>(uc, x);
+      lane_window<2>(dd[m], z);
+      lapy = a2_sum(x + 4);
+      lane_window<4>(q2[m], y2);
+      lane_window<2>(a1_sum<1>(z + 2) * L, y1);
+      lane_window<2>(L * a1_sum<1>(x + 4), yp);
+      sy = at_sum(y2 + 4, y1 + 2);
+      ey = a1_sum<-1>(yp + 2);
+    } else {
+      // the lane's table row, loaded anew for each row of the band: kept, it
+      // would hold 40 registers (lane shifts are evaluated by the whole wave,
+      // then selected)
+      int slot = tslot;
+      asm volatile("" : "+v"(slot));
+      const AdjRow& t = tab[1].r[slot];
+      float x[11], z[7], y2[11], y1[7], yp[7];
+      lane_window<5>(uc, x);
+      lane_window<3>(dd[m], z);
+      const float lt = tab_sum(t.a2, x + 5, kA2), gt = tab_sum(t.a1, x + 5, kA1);
+      float ft = 0.0f;
+#pragma unroll
+      for (int d = -kA1; d <= kA1; ++d) ft = fmaf(t.a1[d + kA1], z[d + 3], ft);
+      const float lc = a2_sum(x + 5), gc = a1_sum<1>(x + 5), fc = a1_sum<1>(z + 3);
+      lapy = nearB ? lt : lc;
+      lane_window<5>(q2[m], y2);
+      lane_window<3>((nearB ? ft : fc) * L, y1);
+      lane_window<3>(L * (nearB ? gt : gc), yp);
+      float s = 0.0f, e = 0.0f;
+#pragma unroll
+      for (int d = -kA2; d <= kA2; ++d) {
+        if (d >= -kA1 && d <= kA1) {
+          s = fmaf(t.t1[d + kA1], y1[3 - d], s);
+          e = fmaf(t.t1[d + kA1], yp[3 - d], e);
+        }
+        s = fmaf(t.t2[d + kA2], y2[5 - d], s);
+      }
+      const float sc = at_sum(y2 + 5, y1 + 3), ec = a1_sum<-1>(yp + 3);
+      sy = nearT ? s : sc;
+      ey = nearT ? e : ec;
+    }
+    const float lap = lapx + lapy;
+    // reaction, gates as fixed masks
+    const bool q = uc >= c.V_c;
+    const float inv_tvm = (uc >= c.V_v) ? c.inv_tv2m : c.inv_tv1m;
+    const float dfv_dv = q ? -c.inv_tvp : -inv_tvm;
+    const float dfw_dw = q ? -c.inv_twp : -c.inv_twm;
+    const float S = half_one_plus_tanh(c, uc);  // (1 + tanh(k (u - V_csi))) / 2
     // dS/du = 2k S (1 - S); kk = -2 k log2(e)
     const float dS = -c.kk * 0.69314718055994531f * S * (1.0f - S);
     // j_ion = -(j_fi + j_so + j_si) / Cm
-    const float djdv = p ? (uu - c.V_c) * (1.0f - uu) * c.inv_td * c.inv_cm : 0.0f;
+    const float a1 = (uc - c.V_c) * (1.0f - uc) * c.inv_td * c.inv_cm;
+    const float djdv = q ? a1 : 0.0f;
     const float djdw = S * c.inv_tsi * c.inv_cm;
-    const float djdu =
-        -((p ? -vv * (1.0f + c.V_c - 2.0f * uu) * c.inv_td : 0.0f) + (p ? 0.0f : c.inv_t0) -
-          ww * dS * c.inv_tsi) *
-        c.inv_cm;
-    // stimulus replaces j_ion: no cotangent reaches it where active
+    const float a0 = q ? -vv[k] * fmaf(-2.0f, uc, 1.0f + c.V_c) * c.inv_td : c.inv_t0;
+    const float djdu = -fmaf(-(ww[k] * dS), c.inv_tsi, a0) * c.inv_cm;
+    // a stimulus replaces j_ion: no cotangent reaches it where one is active
+    bool stim = false;
+    for (int f = 0; f < sv.count(); ++f)
+      if (sv.on(f)) stim = stim || at(sv.field(f), i) != 0.0f;
     const float lus = stim ? 0.0f : L;
-
-    lv_o[idx] = lvv + dt * (dfv_dv * lvv + djdv * lus);
-    lw_o[idx] = lww + dt * (dfw_dw * lww + djdw * lus);
-    const float lu_new = L + dt * (djdu * lus + (sx + sy) * inv_dx2);
-    lu_o[idx] = lu_new;
-    gD[idx] = gd + dt * (L * lap + ex + ey) * inv_dx2;
+    const bool out = lane >= kRevHalo && lane < kRevHalo + kRevOut && col < W && (!XG || i < H);
+    if (out) {
+      const size_t ro = (size_t)i * (size_t)W;
+      st(a.lv_o + ro, off, fmaf(dt, fmaf(dfv_dv, lvv[k], djdv * lus), lvv[k]));
+      st(a.lw_o + ro, off, fmaf(dt, fmaf(dfw_dw, lww[k], djdw * lus), lww[k]));
+      st(a.lu_o + ro, off, fmaf(dt, fmaf(djdu, lus, (sx + sy) * inv_dx2), L));
+      st(a.gD + ro, off, fmaf(dt * (fmaf(L, lap, ex) + ey), inv_dx2, gd[k]));
+    }
     // tau gradients: d j_ion / d tau
-    const float djd_td = p ? -vv * (uu - c.V_c) * (1.0f - uu) * c.inv_td * c.inv_td * c.inv_cm
-                           : 0.0f;
-    const float djd_tr = p ? c.inv_tr * c.inv_tr * c.inv_cm : 0.0f;
-    const float djd_tsi = -ww * S * c.inv_tsi * c.inv_tsi * c.inv_cm;
-    t_d = dt * djd_td * lus;
-    t_r = dt * djd_tr * lus;
-    t_si = dt * djd_tsi * lus;
-    if (NEXT) {  // derived fields of the previous step, at this cell
-      const float Ln = lu_new + inj;
-      nx.pre.Llap[idx] = make_float2(Ln, lapx_n + yr.w);
-      nx.pre.QPx[idx] = make_float2(nDx * Ln, Ln * gx_n);
-      nx.pre.QPy[idx] = make_float2(nDy * Ln, Ln * yr.z);
-      nx.pre.Q2[idx] = nD * Ln;
+    const float lt = out ? lus * dt : 0.0f;
+    const float t_d = (q ? -vv[k] * a1 * c.inv_td : 0.0f) * lt;
+    const float t_r = (q ? c.inv_tr * c.inv_tr * c.inv_cm : 0.0f) * lt;
+    const float t_si = (-ww[k] * S * c.inv_tsi * c.inv_tsi * c.inv_cm) * lt;
+    if (k % 2 == 0) {
+      ts[0] = t_d;
+      ts[1] = t_r;
+      ts[2] = t_si;
+    } else {
+      const float r0 = wave_sum63(ts[0] + t_d), r1 = wave_sum63(ts[1] + t_r),
+                  r2 = wave_sum63(ts[2] + t_si);
+      if (lane == 63 && (!XG || i - 1 < H)) {
+        double* g = a.g_tau + 3 * ((size_t)(cs / kRevOut) * ((H + 1) / 2) + (i - 1) / 2);
+        g[0] += (double)r0;
+        g[1] += (double)r1;
+        g[2] += (double)r2;
+      }
     }
   }
-  // every lane of the x wave takes part; lanes off the grid add 0
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    t_d += __shfl_xor(t_d, o, 64);
-    t_r += __shfl_xor(t_r, o, 64);
-    t_si += __shfl_xor(t_si, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    double* a = g_tau + 3 * adj_wave_index(bx, by, gx, threadIdx.x >> 6);
-    a[0] += (double)t_d;
-    a[1] += (double)t_r;
-    a[2] += (double)t_si;
+}
+
+// Whether the band of R rows at rs, the strip at cs take the edge rules.
+__host__ __device__ inline bool adj_edge_band(int rs, int R, int H) {
+  return rs < kAdjT || rs + R + kAdjT > H;
+}
+__host__ __device__ inline bool adj_edge_strip(int cs, int W) {
+  return cs < kAdjT || cs + kRevOut + kAdjT > W;
+}
+
+// adj_tile with its edge flags (bit 0 band, bit 1 strip).
+template <int R, class SV>
+__device__ __forceinline__ void adj_tile_any(const Coef& c, const AdjArgs& a, int H, int W,
+                                             const SV& sv, float dt, float inv_dx2, int rs, int cs,
+                                             int flags, AdjAxisTab* tab) {
+  switch (flags) {
+    case 0: adj_tile<R, false, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
+    case 1: adj_tile<R, true, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
+    case 2: adj_tile<R, false, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
+    default: adj_tile<R, true, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
   }
 }
 
 // Blocks of the first pass of the tau reduction (k_adj_reduce).
 constexpr int kRedBlocks = 512;
 
-// Workspace layout: [tables (2 axes)][Dx][Dy][tau accumulators: 3 doubles per x wave of
-// k_adj_main][cotangent ping-pong: 3 fields][derived fields: 2 sets of 7 (8 floats per
-// cell)][tau block sums]
+// Workspace layout: [tables (2 axes)][tau accumulators: 3 doubles per group]
+// [cotangent ping-pong: 3 fields][tau block sums]
 struct AdjLayout {
-  size_t tab, dx, dy, part, lam, pre, red, total;
+  size_t tab, part, lam, red, total;
 };
 
 inline AdjLayout adj_layout(int H, int W) {
@@ -438,21 +463,11 @@ inline AdjLayout adj_layout(int H, int W) {
     return at;
   };
   L.tab = take(2 * sizeof(AdjAxisTab));
-  L.dx = take(cells * sizeof(float));
-  L.dy = take(cells * sizeof(float));
-  L.part = take(3 * adj_n_waves(H, W) * sizeof(double));
+  L.part = take(3 * adj_n_groups(H, W) * sizeof(double));
   L.lam = take(3 * cells * sizeof(float));
-  L.pre = take(2 * 8 * cells * sizeof(float));
   L.red = take(3 * kRedBlocks * sizeof(double));
   L.total = o;
   return L;
-}
-
-// Set `set` of the derived fields: three float2 fields, then Q2 (the pairs
-// stay 8-byte aligned for any n).
-inline AdjPre pre_fields(const AdjLayout& L, char* wk, int set, size_t n) {
-  float* pf = (float*)(wk + L.pre) + (size_t)set * 8 * n;
-  return AdjPre{(float2*)pf, (float2*)(pf + 2 * n), (float2*)(pf + 4 * n), pf + 6 * n};
 }
 
 }  // namespace fk

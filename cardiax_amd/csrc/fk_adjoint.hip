@@ -18,9 +18,10 @@
 //   g_tau += dt sum(dJ/dtau lam_u*)            (tau_d, tau_r, tau_si)
 // with lam_u* = lam_u outside active stimulus cells and 0 inside.
 //
-// The operators' entries away from the edges are the central stencils; the 8
-// rows nearest each edge are tabulated per call by k_adj_tables, which
-// composes the reference's gradient rules exactly (any N >= 3).
+// The operators' rows away from the edges are the central stencils; those near
+// an edge are tabulated per call by k_adj_tables, which composes the
+// reference's gradient rules exactly (any N >= 3). One launch reverses one step
+// (adj_tile).
 #include <hip/hip_runtime.h>
 
 #include "cardiax_amd.h"
@@ -30,81 +31,45 @@
 
 namespace fk {
 
-// A1[j][i] and A2[j][i] for the tabulated rows of both axes.
+// Band rows of a reverse step on one grid: a small grid's step takes as long as
+// its slowest wave (256^2: 7.0 us with 2 rows, 8.9 with 4, 13.9 with 8); the
+// halo rows of short bands cost less (1120^2: 24.7, 23.9 and 29.8).
+constexpr int kRevRows = 2;
+
+// The table rows of both axes, one d = -5 .. 5 per thread.
 __global__ void k_adj_tables(int H, int W, AdjAxisTab* tab) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int per_axis = kAdjSlots * (2 * kAdjBand + 1);
+  constexpr int per_axis = kAdjSlots * 12;
   if (t >= 2 * per_axis) return;
-  const int axis = t / per_axis, r = t % per_axis;
-  const int slot = r / (2 * kAdjBand + 1), d = r % (2 * kAdjBand + 1) - kAdjBand;
-  const int N = axis == 0 ? H : W, n = N + 2;
-  // row j of the slot
-  int j;
-  if (N <= kAdjSlots) j = slot;
-  else j = slot < kAdjB ? slot : N - kAdjSlots + slot;
-  double a1 = 0.0, a2 = 0.0;
-  const int i = j + d;
-  if (j < N && i >= 0 && i < N) {
-    const int pj = j + 1;  // padded row of original j
-    for (int q = pj - 3; q <= pj + 3; ++q) {
-      if (q < 0 || q >= n) continue;
-      const double gq = g_coef(pj, q, n);
-      if (gq == 0.0) continue;
-      a1 += gq * pad_coef(q, i, N);
-      // A2 = crop G G pad: row pj of G times column i of G pad
-      double gp = 0.0;
-      for (int s = q - 3; s <= q + 3; ++s)
-        if (s >= 0 && s < n) gp += g_coef(q, s, n) * pad_coef(s, i, N);
-      a2 += gq * gp;
-    }
-  }
-  AdjAxisTab& T = tab[axis];
-  if (slot < kAdjSlots) {
-    T.a1[slot][d + kAdjBand] = (float)a1;
-    T.a2[slot][d + kAdjBand] = (float)a2;
+  const int axis = t / per_axis, slot = t % per_axis / 12, d = t % 12 - kA2;
+  const int N = axis == 0 ? H : W;
+  const int i = N <= kAdjSlots || slot < kAdjT ? slot : slot + (N - kAdjSlots);
+  float a1, a2, t1, t2;  // 0 for d = 6 and for cells off a short axis
+  adj_coef(i, d <= kA2 ? i + d : -1, N, a1, a2);
+  adj_coef(d <= kA2 ? i - d : -1, i, N, t1, t2);
+  AdjRow& r = tab[axis].r[slot];
+  r.a2[d + kA2] = a2;
+  r.t2[d + kA2] = t2;
+  if (d >= -kA1 && d <= kA1 + 1) {
+    r.a1[d + kA1] = d <= kA1 ? a1 : 0.0f;
+    r.t1[d + kA1] = d <= kA1 ? t1 : 0.0f;
   }
 }
 
-// Static first derivatives of D: (A1x D, A1y D).
-__global__ void k_adj_dgrad(const float* __restrict__ D, int H, int W,
-                            const AdjAxisTab* __restrict__ tab, float* __restrict__ Dx,
-                            float* __restrict__ Dy) {
-  const int c = blockIdx.x * 64 + threadIdx.x, i = blockIdx.y * 4 + threadIdx.y;
-  if (i >= H || c >= W) return;
-  const AxisOps ox{&tab[0], H}, oy{&tab[1], W};
-  float sx = 0.0f, sy = 0.0f;
-  for (int d = -kAdjBand; d <= kAdjBand; ++d) {
-    if (i + d >= 0 && i + d < H) sx += ox.a1(i, d) * D[(size_t)(i + d) * W + c];
-    if (c + d >= 0 && c + d < W) sy += oy.a1(c, d) * D[(size_t)i * W + c + d];
-  }
-  Dx[(size_t)i * W + c] = sx;
-  Dy[(size_t)i * W + c] = sy;
-}
-
-
-__global__ void __launch_bounds__(kAdjThreads)
-k_adj_pre(const float* __restrict__ u, const float* __restrict__ D,
-          const float* __restrict__ Dx, const float* __restrict__ Dy,
-          const float* __restrict__ lu, const float* __restrict__ inj, int H, int W,
-          const AdjAxisTab* __restrict__ tab_g, AdjPre o) {
-  __shared__ AdjAxisTab tab[2];
-  adj_pre_tile(u, D, Dx, Dy, lu, inj, H, W, tab_g, o, blockIdx.x, blockIdx.y, tab);
-}
-
-// One reverse step (adj_main_tile) per block of 64 columns x 2 rows.
-template <bool NEXT>
-__global__ void __launch_bounds__(kAdjThreads)
-k_adj_main(Coef c, const float* __restrict__ v, const float* __restrict__ w,
-           const float* __restrict__ u, int H, int W, StimArgs sa, float dt, float inv_dx2,
-           const float* __restrict__ lv, const float* __restrict__ lw, AdjPre pre,
-           float* __restrict__ lv_o, float* __restrict__ lw_o, float* __restrict__ lu_o,
-           float* __restrict__ gD, double* __restrict__ g_tau,
-           const AdjAxisTab* __restrict__ tab_g, AdjNext nx) {
-  __shared__ AdjAxisTab tab[2];
-  __shared__ float4 xch[kAdjThreads / 2];  // y thread -> x thread of each cell
+// One reverse step: a wave per (strip, band of R rows), four per block.
+template <int R>
+__global__ void __launch_bounds__(256)
+k_adj_rev(Coef c, AdjArgs a, int H, int W, StimArgs sa, float dt, float inv_dx2, int n_bands,
+          int n_tiles) {
+  __shared__ AdjAxisTab tab[4][2];
+  const int tile = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x >> 6));
+  if (tile >= n_tiles) return;  // whole wave leaves; the kernel has no barrier
+  const int strip = tile / n_bands, band = tile - strip * n_bands;
+  const int rs = R * band, cs = kRevOut * strip;
   const AdjStimList sv{sa};
-  adj_main_tile<NEXT>(c, v, w, u, H, W, sv, dt, inv_dx2, lv, lw, pre, lv_o, lw_o, lu_o, gD,
-                      g_tau, tab_g, nx, blockIdx.x, blockIdx.y, gridDim.x, tab, xch);
+  adj_tile_any<R>(c, a, H, W, sv, dt, inv_dx2, rs, cs,
+                  (adj_edge_band(rs, R, H) ? 1 : 0) | (adj_edge_strip(cs, W) ? 2 : 0),
+                  tab[threadIdx.x >> 6]);
 }
 
 __global__ void k_adj_zero(float* a, size_t n) {
@@ -114,7 +79,7 @@ __global__ void k_adj_zero(float* a, size_t n) {
 }
 
 
-// Sums of the three per-wave tau accumulators (n triples of doubles): each
+// Sums of the three tau accumulators (n triples of doubles): each
 // block reduces a grid-stride slice into part[block][0..2] (k_adj_reduce),
 // then one block adds the block sums (k_adj_reduce_final). Fixed order:
 // deterministic.
@@ -159,39 +124,18 @@ k_adj_reduce_final(const double* __restrict__ part, int n_part, float* g_tau) {
     for (int k = 0; k < 3; ++k) g_tau[k] = (float)s[k][0];
 }
 
-static hipError_t launch_pre(const AdjLayout& L, char* wk, const float* D, const float* u,
-                             int H, int W, const float* lu, const float* inj, int set,
-                             hipStream_t s) {
-  const size_t n = (size_t)H * W;
-  const dim3 grid((W + 63) / 64, (H + 3) / 4);
-  k_adj_pre<<<grid, kAdjThreads, 0, s>>>(u, D, (const float*)(wk + L.dx),
-                                         (const float*)(wk + L.dy), lu, inj, H, W,
-                                         (const AdjAxisTab*)(wk + L.tab),
-                                         pre_fields(L, wk, set, n));
-  return hipGetLastError();
-}
-
-// Reverse step from derived-field set `set`: cotangents lam_in (v, w; u comes
-// from the fields) -> lam_out. With u_prev, also writes set 1 - set for the
-// step before (u_prev = that step's state u, inj = its injected cotangent).
-static hipError_t launch_main(const AdjLayout& L, char* wk, const Coef& c, const float* D,
-                              const float* v, const float* w, const float* u, int H, int W,
-                              const StimArgs& sa, float dt, float inv_dx2,
-                              const float* const lam_in[3], float* const lam_out[3], float* gD,
-                              int set, const float* u_prev, const float* inj, hipStream_t s) {
-  const size_t n = (size_t)H * W;
-  const AdjAxisTab* tab = (const AdjAxisTab*)(wk + L.tab);
-  const dim3 grid((W + 63) / 64, (H + 1) / 2);  // 64 x 2 cells, two threads each
-  const AdjNext nx{u_prev, inj, D, (const float*)(wk + L.dx), (const float*)(wk + L.dy),
-                   pre_fields(L, wk, 1 - set, n)};
-  if (u_prev)
-    k_adj_main<true><<<grid, kAdjThreads, 0, s>>>(
-        c, v, w, u, H, W, sa, dt, inv_dx2, lam_in[0], lam_in[1], pre_fields(L, wk, set, n),
-        lam_out[0], lam_out[1], lam_out[2], gD, (double*)(wk + L.part), tab, nx);
-  else
-    k_adj_main<false><<<grid, kAdjThreads, 0, s>>>(
-        c, v, w, u, H, W, sa, dt, inv_dx2, lam_in[0], lam_in[1], pre_fields(L, wk, set, n),
-        lam_out[0], lam_out[1], lam_out[2], gD, (double*)(wk + L.part), tab, nx);
+// Reverse step: cotangents lam_in (v, w, u; inj, if not null, adds to u) ->
+// lam_out.
+static hipError_t launch_rev(const AdjLayout& L, char* wk, const Coef& c, const float* D,
+                             const float* v, const float* w, const float* u, int H, int W,
+                             const StimArgs& sa, float dt, float inv_dx2,
+                             const float* const lam_in[3], const float* inj,
+                             float* const lam_out[3], float* gD, hipStream_t s) {
+  const AdjArgs a{v, w, u, D, lam_in[0], lam_in[1], lam_in[2], inj, lam_out[0], lam_out[1],
+                  lam_out[2], gD, (double*)(wk + L.part), (const AdjAxisTab*)(wk + L.tab)};
+  const int strips = adj_strips(W), bands = (H + kRevRows - 1) / kRevRows;
+  const int tiles = strips * bands;
+  k_adj_rev<kRevRows><<<(tiles + 3) / 4, 256, 0, s>>>(c, a, H, W, sa, dt, inv_dx2, bands, tiles);
   return hipGetLastError();
 }
 
@@ -217,13 +161,10 @@ int32_t fk_adjoint_prepare(const float* D, int32_t H, int32_t W, void* work, siz
   hipStream_t s = (hipStream_t)stream;
   char* wk = (char*)work;
   AdjAxisTab* tab = (AdjAxisTab*)(wk + L.tab);
-  const int n_tab = 2 * kAdjSlots * (2 * kAdjBand + 1);
+  const int n_tab = 2 * kAdjSlots * 12;
   k_adj_tables<<<(n_tab + 255) / 256, 256, 0, s>>>(H, W, tab);
   HIP_CHECK(hipGetLastError());
-  const dim3 block(64, 4), grid((W + 63) / 64, (H + 3) / 4);
-  k_adj_dgrad<<<grid, block, 0, s>>>(D, H, W, tab, (float*)(wk + L.dx), (float*)(wk + L.dy));
-  HIP_CHECK(hipGetLastError());
-  k_adj_zero<<<256, 256, 0, s>>>((float*)(wk + L.part), 6 * adj_n_waves(H, W));
+  k_adj_zero<<<256, 256, 0, s>>>((float*)(wk + L.part), 6 * adj_n_groups(H, W));
   HIP_CHECK(hipGetLastError());
   return FK_OK;
 }
@@ -250,9 +191,8 @@ int32_t fk_adjoint_step(const fk_params* params, const float* D, const float* v,
   const float* lin[3] = {lam_v, lam_w, lam_u};
   float* lout[3] = {lam_v_out, lam_w_out, lam_u_out};
   hipStream_t s = (hipStream_t)stream;
-  HIP_CHECK(launch_pre(L, (char*)work, D, u, H, W, lam_u, nullptr, 0, s));
-  HIP_CHECK(launch_main(L, (char*)work, c, D, v, w, u, H, W, sched.at(t), dt, inv_dx2, lin, lout,
-                        grad_D, 0, nullptr, nullptr, s));
+  HIP_CHECK(launch_rev(L, (char*)work, c, D, v, w, u, H, W, sched.at(t), dt, inv_dx2, lin,
+                       nullptr, lout, grad_D, s));
   return FK_OK;
 }
 
@@ -283,21 +223,13 @@ int32_t fk_adjoint_segment(const fk_params* params, const float* D, int32_t H, i
   StimSchedule sched(stimuli, n_stimuli);
   const Coef c = make_coef(*params);
   const float inv_dx2 = (float)(1.0 / ((double)dx * (double)dx));
-  int cur = 0, set = 0;
-  if (n_steps > 0) {
-    const float* x = states + (size_t)(n_steps - 1) * 3 * n;
-    HIP_CHECK(launch_pre(L, wk, D, x + 2 * n, H, W, lam_u,
-                         inject ? inject[n_steps - 1] : nullptr, set, s));
-  }
+  int cur = 0;
   for (int32_t k = n_steps - 1; k >= 0; --k) {
     const float* x = states + (size_t)k * 3 * n;
-    const float* xp = k > 0 ? states + (size_t)(k - 1) * 3 * n : nullptr;
     const float* lin[3] = {bufs[cur][0], bufs[cur][1], bufs[cur][2]};
-    HIP_CHECK(launch_main(L, wk, c, D, x, x + n, x + 2 * n, H, W, sched.at(t + (double)k), dt,
-                          inv_dx2, lin, bufs[cur ^ 1], grad_D, set, xp ? xp + 2 * n : nullptr,
-                          (xp && inject) ? inject[k - 1] : nullptr, s));
+    HIP_CHECK(launch_rev(L, wk, c, D, x, x + n, x + 2 * n, H, W, sched.at(t + (double)k), dt,
+                         inv_dx2, lin, inject ? inject[k] : nullptr, bufs[cur ^ 1], grad_D, s));
     cur ^= 1;
-    set ^= 1;
   }
   if (cur == 1)
     for (int f = 0; f < 3; ++f)
@@ -310,7 +242,7 @@ int32_t fk_adjoint_tau_grads(void* work, int32_t H, int32_t W, float* g_tau, voi
   ErrorScope es;
   if (!check_grid(H, W) || !check_ptrs({work, g_tau})) return last_code();
   const AdjLayout L = adj_layout(H, W);
-  const size_t n = adj_n_waves(H, W);
+  const size_t n = adj_n_groups(H, W);
   const int blocks = (int)std::min<size_t>((n + 255) / 256, (size_t)kRedBlocks);
   double* part = (double*)((char*)work + L.red);
   k_adj_reduce<<<blocks, 256, 0, (hipStream_t)stream>>>(

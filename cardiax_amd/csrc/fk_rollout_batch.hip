@@ -9,12 +9,10 @@
 // Per problem the schedule is the one the per-grid path runs (adjoint.py
 // with fk_forward_trajectory and fk_adjoint_segment): checkpoints every S
 // steps; for each segment, in reverse, the states are recomputed from its
-// checkpoint, the derived fields of its last step are formed, and the steps
-// are reversed one by one, frame cotangents entering lam_u at the frame
-// steps. Every launch covers all problems through a work list (one wave per
-// forward tile, one block per reverse tile), and the tiles run the same
-// device code as the per-grid kernels: the results are bitwise those of the
-// per-grid path.
+// checkpoint and the steps are reversed one by one, frame cotangents entering
+// lam_u at the frame steps. Every launch covers all problems through a work
+// list (one wave per tile), and the tiles run the same device code as the
+// per-grid kernels: the results are bitwise those of the per-grid path.
 //
 // Reference: there is no counterpart in the reference, whose inverse problem
 // is learnt by a network (deepx); the forward step follows
@@ -37,10 +35,13 @@
 namespace fk {
 
 constexpr int kRollRows = 4;  // band rows of the forward tiles
+// band rows of the reverse tiles: 3.84 M cells 60 us with 4, 68 with 2, 67 with
+// 8; the bits do not depend on it
+constexpr int kRollRev = 4;
 
 struct RollDesc {
   Coef c;
-  int H, W, gx;  // gx: blocks of 64 columns of the reverse grid
+  int H, W;
   float dt, inv_dx2;
   size_t cells;
   const float* D;
@@ -53,19 +54,13 @@ struct RollDesc {
   float* lam;          // cotangent (v, w, u planes) at segment boundaries
   float* lam_alt;      // its ping-pong partner
   const AdjAxisTab* tab;
-  const float *Dx, *Dy;
   double* part;        // tau accumulators
-  AdjPre pre[2];
   int n_stim;
   BatchStim stim[FK_BATCH_MAX_STIMULI];
 };
 
 struct RollTile {
   int sim, cs, rs, flags;  // flags: bit0 band near a row edge, bit1 strip near a column edge
-};
-
-struct RollBlock {
-  int sim, bx, by;
 };
 
 // A pointer field of a descriptor, read as a global-memory pointer. Pointers
@@ -80,9 +75,6 @@ __device__ __forceinline__ T* gfield(T* const& f) {
   GT g;
   __builtin_memcpy(&g, &f, sizeof g);
   return (T*)g;
-}
-__device__ __forceinline__ AdjPre gfield(const AdjPre& a) {
-  return AdjPre{gfield(a.Llap), gfield(a.QPx), gfield(a.QPy), gfield(a.Q2)};
 }
 
 // State x_{c + k} of segment `seg` (c = seg S): the checkpoint at k = 0, else
@@ -185,44 +177,37 @@ __device__ __forceinline__ const float* roll_inject(const RollDesc& S, int j, in
   return (j > 0 && j % fe == 0) ? gfield(S.g_frames) + (size_t)(j / fe - 1) * S.cells : nullptr;
 }
 
-// Derived fields (set 0) of the last step k of segment `seg`, whose output
-// x_j (j = c + k + 1) takes the frame cotangent of j.
-__global__ void __launch_bounds__(kAdjThreads)
-k_roll_pre(const RollDesc* __restrict__ sims, const RollBlock* __restrict__ blocks, int seg,
-           int k, int j, int fe) {
-  __shared__ AdjAxisTab tab[2];
-  const RollBlock b = blocks[blockIdx.x];
-  if (b.sim < 0) return;  // padding of the XCD order (block-uniform)
-  const RollDesc& S = sims[b.sim];
-  adj_pre_tile(roll_state(S, seg, k, 2), gfield(S.D), gfield(S.Dx), gfield(S.Dy),
-               gfield(S.lam) + 2 * S.cells, roll_inject(S, j, fe), S.H, S.W, gfield(S.tab),
-               gfield(S.pre[0]), b.bx, b.by, tab);
-}
-
-// Reverse of step c + k of segment `seg`: cotangent set `cur` (0 lam, 1
-// lam_alt) -> the other, derived fields set `set`; with NEXT (k > 0) also the
-// derived fields of step c + k - 1 into set 1 - set.
-template <bool NEXT>
-__global__ void __launch_bounds__(kAdjThreads)
-k_roll_main(const RollDesc* __restrict__ sims, const RollBlock* __restrict__ blocks,
-            const uint32_t* __restrict__ masks, int seg, int k, int fe, int cur, int set,
-            int c0) {
-  __shared__ AdjAxisTab tab[2];
-  __shared__ float4 xch[kAdjThreads / 2];
-  const RollBlock b = blocks[blockIdx.x];
-  if (b.sim < 0) return;  // padding of the XCD order (block-uniform)
-  const RollDesc& S = sims[b.sim];
+// Reverse of step c + k of segment `seg` (j = c + k + 1): cotangent set `cur`
+// (0 lam, 1 lam_alt) -> the other; x_j's frame cotangent enters first.
+template <int R>
+__global__ void __launch_bounds__(256)
+k_roll_rev(const RollDesc* __restrict__ sims, const RollTile* __restrict__ items, int n_items,
+           const uint32_t* __restrict__ masks, int seg, int k, int j, int fe, int cur) {
+  __shared__ AdjAxisTab tab[4][2];
+  const int it = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x >> 6));
+  if (it >= n_items) return;
+  RollTile item = items[it];
+  if (uni(item.sim) < 0) return;  // padding of the XCD order
+  item.sim = uni(item.sim);
+  const RollDesc& S = sims[item.sim];
   const size_t n = S.cells;
-  float* lin = cur ? gfield(S.lam_alt) : gfield(S.lam);
-  float* lout = cur ? gfield(S.lam) : gfield(S.lam_alt);
-  const AdjNext nx{NEXT ? roll_state(S, seg, k - 1, 2) : nullptr,
-                   NEXT ? roll_inject(S, c0 + k, fe) : nullptr, gfield(S.D), gfield(S.Dx),
-                   gfield(S.Dy), gfield(S.pre[1 - set])};
-  const BatchStimView sv{S.stim, S.n_stim, masks[b.sim]};
-  adj_main_tile<NEXT>(S.c, roll_state(S, seg, k, 0), roll_state(S, seg, k, 1),
-                      roll_state(S, seg, k, 2), S.H, S.W, sv, S.dt, S.inv_dx2, lin, lin + n,
-                      gfield(S.pre[set]), lout, lout + n, lout + 2 * n, gfield(S.gD),
-                      gfield(S.part), gfield(S.tab), nx, b.bx, b.by, S.gx, tab, xch);
+  const float* lin = uni(cur ? S.lam_alt : S.lam);
+  float* lout = uni(cur ? S.lam : S.lam_alt);
+  const AdjArgs a{uni(roll_state(S, seg, k, 0)), uni(roll_state(S, seg, k, 1)),
+                  uni(roll_state(S, seg, k, 2)), uni(S.D), lin, lin + n, lin + 2 * n,
+                  uni(roll_inject(S, j, fe)), lout, lout + n, lout + 2 * n, uni(S.gD),
+                  uni(S.part), uni(S.tab)};
+  const uint32_t mask = uni((int)masks[item.sim]);
+  const BatchStimView sv{S.stim, mask ? uni(S.n_stim) : 0, mask};
+  Coef c = S.c;
+  c.V_c = uni(c.V_c); c.V_v = uni(c.V_v); c.V_csi = uni(c.V_csi); c.kk = uni(c.kk);
+  c.kk_off = uni(c.kk_off);
+  c.inv_tvp = uni(c.inv_tvp); c.inv_tv1m = uni(c.inv_tv1m); c.inv_tv2m = uni(c.inv_tv2m);
+  c.inv_twp = uni(c.inv_twp); c.inv_twm = uni(c.inv_twm); c.inv_td = uni(c.inv_td);
+  c.inv_t0 = uni(c.inv_t0); c.inv_tr = uni(c.inv_tr); c.inv_tsi = uni(c.inv_tsi);
+  c.inv_cm = uni(c.inv_cm);
+  adj_tile_any<R>(c, a, uni(S.H), uni(S.W), sv, uni(S.dt), uni(S.inv_dx2), uni(item.rs),
+                  uni(item.cs), uni(item.flags), tab[threadIdx.x >> 6]);
 }
 
 }  // namespace fk
@@ -238,10 +223,9 @@ struct fk_rollout_batch {
   size_t dev_bytes = 0;
   RollDesc* d_sims = nullptr;
   RollTile* d_tiles = nullptr;
-  RollBlock* d_pre = nullptr;
-  RollBlock* d_main = nullptr;
+  RollTile* d_rev = nullptr;
   uint32_t* d_masks = nullptr;  // n_steps x n
-  int n_tiles = 0, n_pre = 0, n_main = 0;
+  int n_tiles = 0, n_rev = 0;
   size_t max_cells = 0;
   int traj_seg = -1;  // segment whose states the trajectory buffer holds (-1: none)
 };
@@ -298,9 +282,8 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   b->specs.assign(specs, specs + n);
   // work lists: runs of vertically adjacent tiles (which share halo rows),
   // placed whole on one XCD each
-  constexpr int kRunTiles = 16, kRunPre = 8, kRunMain = 16;
-  std::vector<std::vector<RollTile>> tile_runs;
-  std::vector<std::vector<RollBlock>> pre_runs, main_runs;
+  constexpr int kRunTiles = 16;
+  std::vector<std::vector<RollTile>> tile_runs, rev_runs;
   for (int i = 0; i < n; ++i) {
     const fk_rollout_spec& s = specs[i];
     const StreamGeom g = make_stream_geom<kRollRows>(s.H, s.W);
@@ -316,24 +299,22 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
         if (band % kRunTiles == 0) tile_runs.emplace_back();
         tile_runs.back().push_back(t);
       }
-    const int gx = (s.W + 63) / 64;
-    for (int bx = 0; bx < gx; ++bx)
-      for (int by = 0; by < (s.H + 3) / 4; ++by) {
-        if (by % kRunPre == 0) pre_runs.emplace_back();
-        pre_runs.back().push_back(RollBlock{i, bx, by});
-      }
-    for (int bx = 0; bx < gx; ++bx)
-      for (int by = 0; by < (s.H + 1) / 2; ++by) {
-        if (by % kRunMain == 0) main_runs.emplace_back();
-        main_runs.back().push_back(RollBlock{i, bx, by});
+    for (int strip = 0; strip < adj_strips(s.W); ++strip)
+      for (int band = 0; band < (s.H + kRollRev - 1) / kRollRev; ++band) {
+        RollTile t;
+        t.sim = i;
+        t.cs = kRevOut * strip;
+        t.rs = kRollRev * band;
+        t.flags = (adj_edge_band(t.rs, kRollRev, s.H) ? 1 : 0) |
+                  (adj_edge_strip(t.cs, s.W) ? 2 : 0);
+        if (band % kRunTiles == 0) rev_runs.emplace_back();
+        rev_runs.back().push_back(t);
       }
   }
   const std::vector<RollTile> tiles = xcd_order(tile_runs, 4, RollTile{-1, 0, 0, 0});
-  const std::vector<RollBlock> pre = xcd_order(pre_runs, 1, RollBlock{-1, 0, 0});
-  const std::vector<RollBlock> main = xcd_order(main_runs, 1, RollBlock{-1, 0, 0});
+  const std::vector<RollTile> rev = xcd_order(rev_runs, 4, RollTile{-1, 0, 0, 0});
   b->n_tiles = (int)tiles.size();
-  b->n_pre = (int)pre.size();
-  b->n_main = (int)main.size();
+  b->n_rev = (int)rev.size();
   // stimulus activity of every step, as the per-grid path evaluates it
   std::vector<uint32_t> masks((size_t)n_steps * n);
   for (int i = 0; i < n; ++i) {
@@ -351,8 +332,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   };
   const size_t o_sims = take(sizeof(RollDesc) * n);
   const size_t o_tiles = take(sizeof(RollTile) * tiles.size());
-  const size_t o_pre = take(sizeof(RollBlock) * pre.size());
-  const size_t o_main = take(sizeof(RollBlock) * main.size());
+  const size_t o_rev = take(sizeof(RollTile) * rev.size());
   const size_t o_masks = take(sizeof(uint32_t) * masks.size());
   std::vector<size_t> o_ckpt(n), o_traj(n), o_lam(n);
   b->work_off.resize(n);
@@ -374,8 +354,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   }
   b->d_sims = (RollDesc*)(b->dev + o_sims);
   b->d_tiles = (RollTile*)(b->dev + o_tiles);
-  b->d_pre = (RollBlock*)(b->dev + o_pre);
-  b->d_main = (RollBlock*)(b->dev + o_main);
+  b->d_rev = (RollTile*)(b->dev + o_rev);
   b->d_masks = (uint32_t*)(b->dev + o_masks);
   std::vector<RollDesc> desc(n);
   for (int i = 0; i < n; ++i) {
@@ -386,7 +365,6 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
     d.c = make_coef(s.params);
     d.H = s.H;
     d.W = s.W;
-    d.gx = (s.W + 63) / 64;
     d.dt = s.dt;
     d.inv_dx2 = (float)(1.0 / ((double)s.dx * (double)s.dx));
     d.cells = cells;
@@ -404,11 +382,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
     const AdjLayout L = adj_layout(s.H, s.W);
     d.lam_alt = (float*)(wk + L.lam);
     d.tab = (const AdjAxisTab*)(wk + L.tab);
-    d.Dx = (const float*)(wk + L.dx);
-    d.Dy = (const float*)(wk + L.dy);
     d.part = (double*)(wk + L.part);
-    d.pre[0] = pre_fields(L, wk, 0, cells);
-    d.pre[1] = pre_fields(L, wk, 1, cells);
     d.n_stim = s.n_stimuli;
     for (int k = 0; k < s.n_stimuli; ++k)
       d.stim[k] = {s.stimuli[k].start, s.stimuli[k].duration, s.stimuli[k].period,
@@ -419,10 +393,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
     e = hipMemcpy(b->d_tiles, tiles.data(), sizeof(RollTile) * tiles.size(),
                   hipMemcpyHostToDevice);
   if (e == hipSuccess)
-    e = hipMemcpy(b->d_pre, pre.data(), sizeof(RollBlock) * pre.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(b->d_main, main.data(), sizeof(RollBlock) * main.size(),
-                  hipMemcpyHostToDevice);
+    e = hipMemcpy(b->d_rev, rev.data(), sizeof(RollTile) * rev.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(b->d_masks, masks.data(), sizeof(uint32_t) * masks.size(),
                   hipMemcpyHostToDevice);
@@ -459,7 +430,7 @@ int32_t fk_rollout_batch_backward(fk_rollout_batch* b, float* g_tau, void* strea
   ErrorScope es;
   if (b == nullptr) return set_error(FK_ERR_ARG, "null rollout batch");
   hipStream_t s = (hipStream_t)stream;
-  for (int i = 0; i < b->n; ++i) {  // boundary tables, D_x, D_y, tau accumulators
+  for (int i = 0; i < b->n; ++i) {  // boundary tables, tau accumulators
     const fk_rollout_spec& sp = b->specs[i];
     const int32_t rc = fk_adjoint_prepare(sp.D, sp.H, sp.W, b->dev + b->work_off[i],
                                           b->work_bytes[i], stream);
@@ -467,7 +438,7 @@ int32_t fk_rollout_batch_backward(fk_rollout_batch* b, float* g_tau, void* strea
   }
   const dim3 cg = roll_cell_grid(b);
   k_roll_zero<<<cg, 256, 0, s>>>(b->d_sims);
-  const int step_blocks = (b->n_tiles + 3) / 4;
+  const int step_blocks = (b->n_tiles + 3) / 4, rev_blocks = (b->n_rev + 3) / 4;
   for (int seg = b->n_seg - 1; seg >= 0; --seg) {
     const int c = seg * b->S, len = std::min(b->S, b->n_steps - c);
     // recompute x_{c+1} .. x_{c+len-1}, unless the forward's last segment is
@@ -477,19 +448,12 @@ int32_t fk_rollout_batch_backward(fk_rollout_batch* b, float* g_tau, void* strea
         k_roll_step<kRollRows><<<step_blocks, 256, 0, s>>>(
             b->d_sims, b->d_tiles, b->n_tiles, b->d_masks + (size_t)(c + k) * b->n, seg, k);
     b->traj_seg = seg;
-    k_roll_pre<<<b->n_pre, kAdjThreads, 0, s>>>(b->d_sims, b->d_pre, seg, len - 1, c + len,
-                                                b->fe);
-    int cur = 0, set = 0;
+    int cur = 0;
     for (int k = len - 1; k >= 0; --k) {
-      const uint32_t* m = b->d_masks + (size_t)(c + k) * b->n;
-      if (k > 0)
-        k_roll_main<true><<<b->n_main, kAdjThreads, 0, s>>>(b->d_sims, b->d_main, m, seg, k,
-                                                            b->fe, cur, set, c);
-      else
-        k_roll_main<false><<<b->n_main, kAdjThreads, 0, s>>>(b->d_sims, b->d_main, m, seg, k,
-                                                             b->fe, cur, set, c);
+      k_roll_rev<kRollRev><<<rev_blocks, 256, 0, s>>>(b->d_sims, b->d_rev, b->n_rev,
+                                                      b->d_masks + (size_t)(c + k) * b->n, seg, k,
+                                                      c + k + 1, b->fe, cur);
       cur ^= 1;
-      set ^= 1;
     }
     if (cur == 1) k_roll_lam_back<<<cg, 256, 0, s>>>(b->d_sims);
   }

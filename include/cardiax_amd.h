@@ -262,12 +262,11 @@ int32_t fk_stimulate(double t, const float* X, float* out, int64_t n_cells,
  * ------------------------------------------------------------------------- */
 
 /* Scratch bytes of the adjoint for an H x W grid (tables of the boundary
- * operators, D_x, D_y, the per-block tau partial sums, a cotangent
- * ping-pong buffer and the fields derived per reverse step). */
+ * operators, the tau partial sums and a cotangent ping-pong buffer). */
 size_t fk_adjoint_workspace_bytes(int32_t H, int32_t W);
 
-/* Fills the workspace for D and zeroes the tau accumulators; call once per
- * backward pass before the fk_adjoint_step calls. */
+/* Fills the workspace for the grid and zeroes the tau accumulators; call once
+ * per backward pass before the fk_adjoint_step calls. */
 int32_t fk_adjoint_prepare(const float* D, int32_t H, int32_t W, void* work,
                            size_t work_bytes, void* stream);
 
