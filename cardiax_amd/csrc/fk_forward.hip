@@ -22,12 +22,12 @@
 #include <vector>
 
 #include "cardiax_amd.h"
+#include "fk_block.h"
 #include "fk_device.h"
 #include "fk_host.h"
 #include "fk_stream.h"
 #include "fk_stream2.h"
 #include "fk_stream_t.h"
-#include "fk_tb.h"
 
 namespace fk {
 
@@ -309,10 +309,10 @@ enum Variant : int {
   kStream8 = 4,
   kStream16 = 5,
   kStream32 = 6,
-  kTb64x2 = 7,   // temporal blocking: 64 x 64 tiles, 2 steps per launch
-  kTb64x4 = 8,   // 64 x 64 tiles, 4 steps per launch
-  kTb32x2 = 9,   // 32 x 32 tiles, 2 steps per launch
-  kTb32x4 = 10,  // 32 x 32 tiles, 4 steps per launch
+  kBlock48x2 = 7,   // block tiles (fk_block.h) of 48 rows, 2 steps per launch
+  kBlock48x3 = 8,   // 48 rows, 3 steps
+  kBlock56x3 = 9,   // 56 rows, 3 steps
+  kBlock32x4 = 10,  // 32 rows, 4 steps
   kStreamC8 = 11,   // streaming bands of 8 / 16 rows with the static diffusion
   kStreamC16 = 12,  // coefficients precomputed once per solve
   kStream4 = 13,    // streaming bands of 4 rows
@@ -339,7 +339,17 @@ static int pc_base(int v) {
                                                                                  : kStream16;
 }
 
-static bool is_tb(int v) { return v >= kTb64x2 && v <= kTb32x4; }
+// The block variants' tiles: rows per wave, waves, steps.
+// Of the tilings tried (1 and 2 columns per lane, 2 to 6 rows per wave, 6 to 16
+// waves, 2 to 4 steps) these were the fastest somewhere; us per step below.
+typedef BlockCfg<4, 12, 2> Block48x2;
+typedef BlockCfg<4, 12, 3> Block48x3;
+typedef BlockCfg<4, 14, 3> Block56x3;
+typedef BlockCfg<2, 16, 4> Block32x4;
+
+static bool is_block(int v) { return v >= kBlock48x2 && v <= kBlock32x4; }
+
+static int block_steps(int v) { return v == kBlock48x2 ? 2 : v == kBlock32x4 ? 4 : 3; }
 
 static bool is_two_step(int v) { return v >= kStreamT8 && v <= kStreamT24; }
 
@@ -411,7 +421,40 @@ static int default_variant(int H, int W) {
 }
 static int resolve_variant(int v) { return v == kAuto ? (int)kStream2 : v; }
 
-// The variant an automatic launch on an H x W grid uses.
+// The variant an automatic solve of several steps runs when the shape was not
+// tuned: block tiles, which equal the streaming kernels of default_variant bit
+// for bit. The 4-step tile needs the most waves per cell and the fewest
+// launches: while its tiles fit the 256 CUs once (128^2 2.05 us per step
+// against 3.08 of stream2, 256^2 2.2 against 3.1). Else 48 rows and 3 steps
+// (512^2 2.87 against 3.8, 768^2 4.2 against 5.3, 1024^2 6.5 against 7.0, 1200^2
+// 8.8 against 10.0 of streamt8, 1800^2 13.6 against 16.6, 2300 x 2900 25.7
+// against 34.5 of streamt16, 4000^2 71 against 78), unless they just miss one
+// round of the CUs and 56 rows make it (640^2 3.3 against 4.6). Large grids whose
+// rows start on 256-byte boundaries keep streamt16, whose strips lose least to
+// partial lines there (2048^2 16.8 against 17.3, 2560^2 24.1 against 25.2, 4096^2
+// 77 against 79).
+static int auto_variant(int H, int W) {
+  const int d = default_variant(H, W);
+  if (d == kTile16) return d;  // narrow grids above 8 M cells: another rounding
+  if (d == kStreamT16 && W % 64 == 0) return d;
+  auto tiles = [&](auto cfg) {
+    typedef decltype(cfg) Cfg;
+    return (int64_t)Cfg::row_axis(H).n * Cfg::col_axis(W).n;
+  };
+  constexpr int64_t kCUs = 256;
+  if (tiles(Block32x4{}) <= kCUs) return kBlock32x4;
+  if (tiles(Block48x3{}) > kCUs && tiles(Block56x3{}) <= kCUs) return kBlock56x3;
+  return kBlock48x3;
+}
+
+// The variant of a solve of several steps.
+static int resolve_solve(int v, int H, int W) {
+  if (v != kAuto) return v;
+  const int t = tuned_variant(H, W);
+  return t != kAuto ? t : auto_variant(H, W);
+}
+
+// The variant an automatic launch of one step on an H x W grid uses.
 static int resolve_for(int v, int H, int W) {
   if (v != kAuto) return v;
   const int t = tuned_variant(H, W);
@@ -515,32 +558,29 @@ static hipError_t launch_step(int variant, bool euler, const Coef& c, const floa
   return hipGetLastError();
 }
 
-template <int T, int K, int NT>
-static hipError_t launch_tb(const Coef& c, const float* D, const float* v, const float* w,
-                            const float* u, int H, int W, const TbStim& st, int nsteps,
-                            float dt, float inv_dx2, float* ov, float* ow, float* ou,
-                            hipStream_t s) {
-  const int tiles_x = (W + T - 1) / T, tiles_y = (H + T - 1) / T;
-  const int n = tiles_x * tiles_y;
-  k_tb<T, K, NT><<<n, NT, 0, s>>>(c, D, v, w, u, H, W, st, nsteps, dt, inv_dx2, ov, ow, ou,
-                                  tiles_x, n);
-  return hipGetLastError();
-}
-
-static int tb_depth(int variant) {
-  return (variant == kTb64x4 || variant == kTb32x4) ? 4 : 2;
-}
-
-static hipError_t launch_tb_variant(int variant, const Coef& c, const float* D, const float* v,
-                                    const float* w, const float* u, int H, int W,
-                                    const TbStim& st, int nsteps, float dt, float inv_dx2,
-                                    float* ov, float* ow, float* ou, hipStream_t s) {
-  switch (variant) {
-    case kTb64x2: return launch_tb<64, 2, 1024>(c, D, v, w, u, H, W, st, nsteps, dt, inv_dx2, ov, ow, ou, s);
-    case kTb64x4: return launch_tb<64, 4, 1024>(c, D, v, w, u, H, W, st, nsteps, dt, inv_dx2, ov, ow, ou, s);
-    case kTb32x2: return launch_tb<32, 2, 256>(c, D, v, w, u, H, W, st, nsteps, dt, inv_dx2, ov, ow, ou, s);
-    default: return launch_tb<32, 4, 512>(c, D, v, w, u, H, W, st, nsteps, dt, inv_dx2, ov, ow, ou, s);
+// n_lev steps (at most the variant's) of block variant v.
+static hipError_t launch_block(int v, const Coef& c, const BlockIO& io, int H, int W,
+                               const BlockStim& st, int n_lev, float dt, float inv_dx2,
+                               hipStream_t s) {
+  auto go = [&](auto cfg) {
+    typedef decltype(cfg) Cfg;
+    const BlockAxis ra = Cfg::row_axis(H), ca = Cfg::col_axis(W);
+    k_block<Cfg><<<(unsigned)(ra.n * ca.n), Cfg::waves * 64, 0, s>>>(c, io, H, W, st, n_lev, dt,
+                                                                   inv_dx2, ra, ca);
+    return hipGetLastError();
+  };
+  switch (v) {
+    case kBlock48x2: return go(Block48x2{});
+    case kBlock48x3: return go(Block48x3{});
+    case kBlock56x3: return go(Block56x3{});
+    default: return go(Block32x4{});
   }
+}
+
+// The stimuli of the n_lev steps from time t on.
+static void block_stim(const StimSchedule& sched, double t, int n_lev, BlockStim& st) {
+  for (int j = 0; j < kBlockMaxSteps; ++j)
+    st.act[j] = j < n_lev ? sched.mask(t + (double)j) : 0u;
 }
 
 // One stage of a Heun step on the default band height for the shape.
@@ -621,7 +661,7 @@ int32_t forward_loop(int variant, const fk_params* params, const float* D, const
   const float inv_dx2 = (float)(1.0 / ((double)dx * (double)dx));
   float* wk = (float*)work;
   float* bufs[2][3] = {{v_out, w_out, u_out}, {wk, wk + n, wk + 2 * n}};
-  int v = resolve_for(variant, H, W);
+  int v = resolve_solve(variant, H, W);
   // nothing to amortise, or no room for the coefficients
   if (is_pc(v) && (steps < 2 || state_only)) v = pc_base(v);
   if (is_two_step(v) && !two_step_fits(v, H, W)) v = kStream2;
@@ -632,14 +672,13 @@ int32_t forward_loop(int variant, const fk_params* params, const float* D, const
     k_stream_coef<<<grid, 256, 0, s>>>(D, H, W, (float)(inv_dx2 / 144.0), cf);
     HIP_CHECK(hipGetLastError());
   }
-  const int depth = is_tb(v) ? tb_depth(v) : is_two_step(v) ? 2 : 1;
+  const int depth = is_block(v) ? block_steps(v) : is_two_step(v) ? 2 : 1;
   const int64_t launches = (steps + depth - 1) / depth;
   // Ping-pong so that the last launch lands in the output buffers.
   int dst = (launches % 2 == 1) ? 0 : 1;
   const float* src[3] = {v_in, w_in, u_in};
   StimSchedule sched(stimuli, n_stimuli);
-  TbStim st{};
-  st.n = n_stimuli;
+  BlockStim st{};
   for (int i = 0; i < n_stimuli; ++i) st.f[i] = stimuli[i].field;
   for (int64_t k = 0; k < steps; k += depth) {
     float** d = bufs[dst];
@@ -654,11 +693,14 @@ int32_t forward_loop(int variant, const fk_params* params, const float* D, const
         HIP_CHECK(launch_step(kStream2, true, c, D, src[0], src[1], src[2], H, W, s1, dt,
                               inv_dx2, d[0], d[1], d[2], s));
       }
-    } else if (is_tb(v)) {
+    } else if (is_block(v) && steps - k > 1) {
       const int ns = (int)std::min<int64_t>(depth, steps - k);
-      for (int j = 0; j < 8; ++j) st.act[j] = j < ns ? sched.mask(t + (double)(k + j)) : 0u;
-      HIP_CHECK(launch_tb_variant(v, c, D, src[0], src[1], src[2], H, W, st, ns, dt, inv_dx2,
-                                  d[0], d[1], d[2], s));
+      block_stim(sched, t + (double)k, ns, st);
+      const BlockIO io{D, src[0], src[1], src[2], d[0], d[1], d[2], 0, false};
+      HIP_CHECK(launch_block(v, c, io, H, W, st, ns, dt, inv_dx2, s));
+    } else if (is_block(v)) {  // a single last step
+      HIP_CHECK(launch_step(kStream2, true, c, D, src[0], src[1], src[2], H, W,
+                            sched.at(t + (double)k), dt, inv_dx2, d[0], d[1], d[2], s));
     } else if (is_pc(v)) {
       const StimArgs& sa = sched.at(t + (double)k);
       if (v == kStreamC8)
@@ -703,7 +745,7 @@ static int32_t time_candidates(const fk_params* p, const float* D, const float* 
   float best_ms = 0.0f;
   const int cand[] = {kStream8,  kStream4,  kStream2,   kStream16,  kStream32,  kStreamC8,
                       kStreamC4, kStreamC2, kStreamC16, kPair2,     kPair4,     kTile16,
-                      kTile32,   kTb64x2,   kTb64x4,    kTb32x2,    kTb32x4,    kStreamT8,
+                      kTile32,   kBlock48x2, kBlock48x3, kBlock56x3, kBlock32x4, kStreamT8,
                       kStreamT12, kStreamT16, kStreamT24};
   int32_t rc = FK_OK;
   // one warm-up launch of 8 steps, then n_steps timed with events on `s`
@@ -973,15 +1015,31 @@ int32_t fk_forward_trajectory(const fk_params* params, const float* D, const flo
   const Coef c = make_coef(*params);
   const float inv_dx2 = (float)(1.0 / ((double)dx * (double)dx));
   StimSchedule sched(stimuli, n_stimuli);
-  const int v = resolve_for(g_variant.load(), H, W);  // temporal-blocking variants: stream8
+  const int v = resolve_solve(g_variant.load(), H, W);  // two-step variants: stream2
   const float* src[3] = {v0, w0, u0};
-  for (int32_t k = 0; k < n_steps; ++k) {
+  BlockStim st{};
+  for (int i = 0; i < n_stimuli; ++i) st.f[i] = stimuli[i].field;
+  for (int32_t k = 0; k < n_steps;) {
     float* d = states + (size_t)k * 3 * n;
-    HIP_CHECK(launch_step(v, true, c, D, src[0], src[1], src[2], H, W, sched.at(t + (double)k),
-                          dt, inv_dx2, d, d + n, d + 2 * n, (hipStream_t)stream));
+    if (is_block(v) && n_steps - k > 1) {  // every level of a block is a state
+      const int ns = std::min(block_steps(v), n_steps - k);
+      block_stim(sched, t + (double)k, ns, st);
+      const BlockIO io{D, src[0], src[1], src[2], d, d + n, d + 2 * n, 3 * n, true};
+      HIP_CHECK(launch_block(v, c, io, H, W, st, ns, dt, inv_dx2, (hipStream_t)stream));
+      d += (size_t)(ns - 1) * 3 * n;
+      src[0] = d;
+      src[1] = d + n;
+      src[2] = d + 2 * n;
+      k += ns;
+      continue;
+    }
+    HIP_CHECK(launch_step(is_block(v) ? (int)kStream2 : v, true, c, D, src[0], src[1], src[2], H,
+                          W, sched.at(t + (double)k), dt, inv_dx2, d, d + n, d + 2 * n,
+                          (hipStream_t)stream));
     src[0] = d;
     src[1] = d + n;
     src[2] = d + 2 * n;
+    ++k;
   }
   return FK_OK;
 }

@@ -74,14 +74,18 @@ int32_t fk_abi_version(void);
  * fk_forward_euler. No reference counterpart (the reference leaves kernel
  * choice to XLA). Process-wide. Returns the previous setting, or FK_ERR_ARG
  * for an unknown variant.
- *    0      automatic: the autotuned choice for the grid shape, else 15 up to
- *           1.1 M cells, 19 up to 2.5 M cells and 21 above (grids too small
- *           for those: 15, 13 up to 8 M cells, 2 above)
+ *    0      automatic: the autotuned choice for the grid shape. Else single
+ *           steps run 15 up to 1.1 M cells, 19 up to 2.5 M cells and 21 above
+ *           (grids too small for those: 15, 13 up to 8 M cells, 2 above), and
+ *           solves of several steps run 8, 9 or 10 by the number of their
+ *           tiles, with the same bits (narrow grids above 8 M cells: 2; grids
+ *           above 2.5 M cells with W a multiple of 64: 21)
  *    1      plain, one thread per cell
  *    2, 3   LDS tile of 16 / 32 rows
  *    4-6    streaming wavefront bands of 8 / 16 / 32 rows
- *    7-10   temporal blocking: 64x64 tiles with 2 / 4 steps per launch, 32x32
- *           tiles with 2 / 4 steps per launch
+ *    7-10   temporal blocking: tiles of 64 columns by 48 rows with 2 steps per
+ *           launch, 48 rows with 3, 56 rows with 3 and 32 rows with 4,
+ *           bit-identical to as many steps of 15 (a single last step runs 15)
  *    11, 12 streaming bands of 8 / 16 rows with the static diffusion
  *           coefficients precomputed once per fk_forward_euler call
  *    13, 15 streaming bands of 4 / 2 rows
@@ -131,8 +135,9 @@ void fk_autotune_reset(void);
 
 /* The variant fk_forward_euler runs on an H x W grid under the current
  * setting: the fk_set_forward_variant choice when it is not 0, else the tuned
- * one, else the default listed there; 17 / 18 on an odd W report the 15 / 13
- * they run. No reference counterpart. FK_ERR_ARG for H or W below 3. */
+ * one, else the single-step default listed there (whose bits the block tiles of
+ * an automatic solve reproduce); 17 / 18 on an odd W report the 15 / 13 they
+ * run. No reference counterpart. FK_ERR_ARG for H or W below 3. */
 int32_t fk_forward_variant_for(int32_t H, int32_t W);
 
 /* cardiax/solve.py:18-23 -- v = w = 1, u = 0 over n_cells cells. */

@@ -1,0 +1,57 @@
+"""The block-tile kernels (variants tb64x2, tb64x4, tb32x2, tb32x4: tiles of 48,
+48, 56 and 32 rows with 2, 3, 3 and 4 steps per launch) against the one-step
+streaming kernel, bit for bit, at the sizes where their tilings change: grids
+inside one tile, one row or column more, sides that end a tile on each of its
+rows, and the automatic choice on both sides of its rule."""
+import ctypes
+
+import pytest
+import torch
+
+from cardiax_amd import _lib, autotune, solve
+from cardiax_amd import params as P
+
+from test_gpu_two_step import _inputs, _run
+
+pytestmark = pytest.mark.gpu
+
+VARIANTS = ["tb64x2", "tb64x4", "tb32x2", "tb32x4"]
+SHAPES = [(3, 3), (5, 62), (32, 63), (33, 64), (48, 110), (49, 111), (56, 48), (57, 90),
+          (61, 94), (81, 47), (97, 126), (131, 39), (160, 303)]
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("shape", SHAPES)
+def test_blocks_equal_one_step_kernel(gpu, variant, shape):
+    st, D, stims = _inputs(shape, seed=shape[0])
+    prm = P.ALL_PARAMSETS["3" if shape[0] % 2 else "7"]
+    for t0, t1 in ((1, 14), (2, 13), (3, 5), (4, 5)):  # whole blocks and each remainder
+        ref = _run("stream2", st, t0, t1, prm, D, stims)
+        got = _run(variant, st, t0, t1, prm, D, stims)
+        for name, a, b in zip("vwu", got, ref):
+            assert torch.isfinite(b).all()
+            assert torch.equal(a, b), (variant, shape, t0, t1, name)
+
+
+@pytest.mark.parametrize("shape", [(30, 40), (256, 256), (272, 272), (500, 520), (600, 640),
+                                   (1100, 1000), (1201, 1203)])
+def test_automatic_solves(gpu, shape):
+    """The automatic kernel (no variant set, shape not tuned) and the
+    trajectory it writes."""
+    st, D, stims = _inputs(shape, seed=1)
+    autotune.reset()
+    ref = _run("stream2", st, 1, 12, P.PARAMSET_3, D, stims)
+    for a, b in zip(_run("auto", st, 1, 12, P.PARAMSET_3, D, stims), ref):
+        assert torch.equal(a, b)
+    H, W = shape
+    D = torch.from_numpy(D).to(gpu)
+    states = torch.empty((11, 3, H, W), device=gpu)
+    stim = solve._Stimuli(stims, gpu, shape)
+    _lib.check(_lib.lib().fk_forward_trajectory(
+        ctypes.byref(_lib.make_params(P.PARAMSET_3)), D.data_ptr(), *(x.data_ptr() for x in st),
+        H, W, stim.pointer(), stim.n, 1.0, 11, 0.01, 0.01, states.data_ptr(),
+        torch.cuda.current_stream().cuda_stream))
+    for k in (0, 1, 2, 3, 7, 10):
+        ref = _run("stream2", st, 1, 2 + k, P.PARAMSET_3, D, stims)
+        for a, b in zip(states[k], ref):
+            assert torch.equal(a, b), k
