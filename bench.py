@@ -34,8 +34,8 @@ BYTES_PER_CELL_UPDATE = 28  # read v, w, u, D + write v, w, u (fp32)
 # Step-kernel variant -> (kernel the variant launches, Euler steps per launch).
 KERNELS = {"stream8": ("k_stream<8, true>", 1), "stream16": ("k_stream<16, true>", 1),
            "stream32": ("k_stream<32, true>", 1), "tile16": ("k_tile<16, true>", 1),
-           "tile32": ("k_tile<32, true>", 1), "tb64x2": ("k_block<4, 12, 2>", 2),
-           "tb64x4": ("k_block<4, 12, 3>", 3), "tb32x2": ("k_block<4, 14, 3>", 3),
+           "tile32": ("k_tile<32, true>", 1), "tb64x2": ("k_block<4, 8, 2>", 2),
+           "tb64x4": ("k_block<4, 12, 3>", 3), "tb32x2": ("k_block<4, 16, 3>", 3),
            "tb32x4": ("k_block<2, 16, 4>", 4), "streamc8": ("k_stream_c<8>", 1),
            "streamc16": ("k_stream_c<16>", 1), "stream4": ("k_stream<4, true>", 1),
            "streamc4": ("k_stream_c<4>", 1), "stream2": ("k_stream<2, true>", 1),

@@ -3,7 +3,7 @@ fk_autotune_forward_state).
 
 The reference leaves kernel choice to XLA. Here the step kernel has several
 implementations (LDS tiles, streaming wave bands of 8/16/32 rows, blocks
-of 32 to 56 rows advancing 2 to 4 steps per launch); ``tune(shape)`` times each on
+of 32 to 64 rows advancing 2 to 4 steps per launch); ``tune(shape)`` times each on
 the GPU for one grid shape and records the fastest, which every automatic
 launch on that shape uses afterwards (process-wide, guarded in the library).
 """

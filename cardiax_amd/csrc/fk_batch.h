@@ -10,6 +10,8 @@
 #include <algorithm>
 #include <vector>
 
+#include "fk_device.h"
+
 namespace fk {
 
 struct BatchStim {
@@ -52,7 +54,6 @@ struct BatchStimView {
 // halo rows (a column of tiles); each run goes whole to the XCD with the least
 // work so far, and the XCD lists are interleaved, short ones padded with
 // `pad` items that exit at once. `per_wg` items make one workgroup.
-constexpr int kXcds = 8;
 
 template <class T>
 inline std::vector<T> xcd_order(const std::vector<std::vector<T>>& runs, int per_wg, T pad) {

@@ -29,6 +29,10 @@ struct StimArgs {
   const float* f[FK_MAX_STIMULI];
 };
 
+// Accelerator dies, each with its own L2: workgroup b of a launch runs on die
+// b % kXcds.
+constexpr int kXcds = 8;
+
 __device__ __forceinline__ int clampi(int x, int lo, int hi) {
   return x < lo ? lo : (x > hi ? hi : x);
 }

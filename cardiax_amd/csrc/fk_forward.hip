@@ -309,9 +309,9 @@ enum Variant : int {
   kStream8 = 4,
   kStream16 = 5,
   kStream32 = 6,
-  kBlock48x2 = 7,   // block tiles (fk_block.h) of 48 rows, 2 steps per launch
+  kBlock32x2 = 7,   // block tiles (fk_block.h) of 32 rows, 2 steps per launch
   kBlock48x3 = 8,   // 48 rows, 3 steps
-  kBlock56x3 = 9,   // 56 rows, 3 steps
+  kBlock64x3 = 9,   // 64 rows, 3 steps
   kBlock32x4 = 10,  // 32 rows, 4 steps
   kStreamC8 = 11,   // streaming bands of 8 / 16 rows with the static diffusion
   kStreamC16 = 12,  // coefficients precomputed once per solve
@@ -342,14 +342,14 @@ static int pc_base(int v) {
 // The block variants' tiles: rows per wave, waves, steps.
 // Of the tilings tried (1 and 2 columns per lane, 2 to 6 rows per wave, 6 to 16
 // waves, 2 to 4 steps) these were the fastest somewhere; us per step below.
-typedef BlockCfg<4, 12, 2> Block48x2;
+typedef BlockCfg<4, 8, 2> Block32x2;
 typedef BlockCfg<4, 12, 3> Block48x3;
-typedef BlockCfg<4, 14, 3> Block56x3;
+typedef BlockCfg<4, 16, 3> Block64x3;
 typedef BlockCfg<2, 16, 4> Block32x4;
 
-static bool is_block(int v) { return v >= kBlock48x2 && v <= kBlock32x4; }
+static bool is_block(int v) { return v >= kBlock32x2 && v <= kBlock32x4; }
 
-static int block_steps(int v) { return v == kBlock48x2 ? 2 : v == kBlock32x4 ? 4 : 3; }
+static int block_steps(int v) { return v == kBlock32x2 ? 2 : v == kBlock32x4 ? 4 : 3; }
 
 static bool is_two_step(int v) { return v >= kStreamT8 && v <= kStreamT24; }
 
@@ -423,28 +423,31 @@ static int resolve_variant(int v) { return v == kAuto ? (int)kStream2 : v; }
 
 // The variant an automatic solve of several steps runs when the shape was not
 // tuned: block tiles, which equal the streaming kernels of default_variant bit
-// for bit. The 4-step tile needs the most waves per cell and the fewest
-// launches: while its tiles fit the 256 CUs once (128^2 2.05 us per step
-// against 3.08 of stream2, 256^2 2.2 against 3.1). Else 48 rows and 3 steps
-// (512^2 2.87 against 3.8, 768^2 4.2 against 5.3, 1024^2 6.5 against 7.0, 1200^2
-// 8.8 against 10.0 of streamt8, 1800^2 13.6 against 16.6, 2300 x 2900 25.7
-// against 34.5 of streamt16, 4000^2 71 against 78), unless they just miss one
-// round of the CUs and 56 rows make it (640^2 3.3 against 4.6). Large grids whose
-// rows start on 256-byte boundaries keep streamt16, whose strips lose least to
-// partial lines there (2048^2 16.8 against 17.3, 2560^2 24.1 against 25.2, 4096^2
-// 77 against 79).
+// for bit. A launch takes the GPU's 256 CUs in rounds of tiles, and each tiling's
+// time per step is close to a + b ceil(tiles / 256), measured from 64^2 to
+// 2500^2: few steps per launch cost the launch (a), many cost the columns and
+// rows that only feed the stencil (b). The least of the four is taken. Against
+// the best streaming kernel, us per step: 128^2 2.05 and 3.07 (32 rows, 4
+// steps), 500^2 3.0 and 3.9 (48 rows, 3), 700 x 600 3.5 and 5.4 (64 rows, 3),
+// 1024^2 6.2 and 7.2, 1200^2 7.3 and 10.0, 2048^2 15.9 and 17.2, 4096^2 70 and
+// 78 (32 rows, 2).
 static int auto_variant(int H, int W) {
   const int d = default_variant(H, W);
   if (d == kTile16) return d;  // narrow grids above 8 M cells: another rounding
-  if (d == kStreamT16 && W % 64 == 0) return d;
-  auto tiles = [&](auto cfg) {
-    typedef decltype(cfg) Cfg;
-    return (int64_t)Cfg::row_axis(H).n * Cfg::col_axis(W).n;
-  };
   constexpr int64_t kCUs = 256;
-  if (tiles(Block32x4{}) <= kCUs) return kBlock32x4;
-  if (tiles(Block48x3{}) > kCUs && tiles(Block56x3{}) <= kCUs) return kBlock56x3;
-  return kBlock48x3;
+  int best = kAuto;
+  double least = 0.0;
+  auto offer = [&](int v, auto cfg, double a, double b) {
+    typedef decltype(cfg) Cfg;
+    const int64_t tiles = (int64_t)Cfg::row_axis(H).n * Cfg::col_axis(W).n;
+    const double us = a + b * (double)((tiles + kCUs - 1) / kCUs);
+    if (best == kAuto || us < least) best = v, least = us;
+  };
+  offer(kBlock32x4, Block32x4{}, 1.0, 1.05);
+  offer(kBlock48x3, Block48x3{}, 1.7, 1.25);
+  offer(kBlock64x3, Block64x3{}, 1.4, 2.05);
+  offer(kBlock32x2, Block32x2{}, 2.2, 1.0);
+  return best;
 }
 
 // The variant of a solve of several steps.
@@ -565,14 +568,14 @@ static hipError_t launch_block(int v, const Coef& c, const BlockIO& io, int H, i
   auto go = [&](auto cfg) {
     typedef decltype(cfg) Cfg;
     const BlockAxis ra = Cfg::row_axis(H), ca = Cfg::col_axis(W);
-    k_block<Cfg><<<(unsigned)(ra.n * ca.n), Cfg::waves * 64, 0, s>>>(c, io, H, W, st, n_lev, dt,
-                                                                   inv_dx2, ra, ca);
+    k_block<Cfg><<<(unsigned)(ra.n * ca.n), Cfg::waves * 64, 0, s>>>(
+        c, io, H, W, st, n_lev, dt, inv_dx2, ra, ca, make_block_order(ra, ca));
     return hipGetLastError();
   };
   switch (v) {
-    case kBlock48x2: return go(Block48x2{});
+    case kBlock32x2: return go(Block32x2{});
     case kBlock48x3: return go(Block48x3{});
-    case kBlock56x3: return go(Block56x3{});
+    case kBlock64x3: return go(Block64x3{});
     default: return go(Block32x4{});
   }
 }
@@ -745,7 +748,7 @@ static int32_t time_candidates(const fk_params* p, const float* D, const float* 
   float best_ms = 0.0f;
   const int cand[] = {kStream8,  kStream4,  kStream2,   kStream16,  kStream32,  kStreamC8,
                       kStreamC4, kStreamC2, kStreamC16, kPair2,     kPair4,     kTile16,
-                      kTile32,   kBlock48x2, kBlock48x3, kBlock56x3, kBlock32x4, kStreamT8,
+                      kTile32,   kBlock32x2, kBlock48x3, kBlock64x3, kBlock32x4, kStreamT8,
                       kStreamT12, kStreamT16, kStreamT24};
   int32_t rc = FK_OK;
   // one warm-up launch of 8 steps, then n_steps timed with events on `s`

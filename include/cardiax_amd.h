@@ -77,14 +77,13 @@ int32_t fk_abi_version(void);
  *    0      automatic: the autotuned choice for the grid shape. Else single
  *           steps run 15 up to 1.1 M cells, 19 up to 2.5 M cells and 21 above
  *           (grids too small for those: 15, 13 up to 8 M cells, 2 above), and
- *           solves of several steps run 8, 9 or 10 by the number of their
- *           tiles, with the same bits (narrow grids above 8 M cells: 2; grids
- *           above 2.5 M cells with W a multiple of 64: 21)
+ *           solves of several steps run 7 to 10 by the number of their
+ *           tiles, with the same bits (narrow grids above 8 M cells: 2)
  *    1      plain, one thread per cell
  *    2, 3   LDS tile of 16 / 32 rows
  *    4-6    streaming wavefront bands of 8 / 16 / 32 rows
- *    7-10   temporal blocking: tiles of 64 columns by 48 rows with 2 steps per
- *           launch, 48 rows with 3, 56 rows with 3 and 32 rows with 4,
+ *    7-10   temporal blocking: tiles of 64 columns by 32 rows with 2 steps per
+ *           launch, 48 rows with 3, 64 rows with 3 and 32 rows with 4,
  *           bit-identical to as many steps of 15 (a single last step runs 15)
  *    11, 12 streaming bands of 8 / 16 rows with the static diffusion
  *           coefficients precomputed once per fk_forward_euler call

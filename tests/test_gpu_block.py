@@ -1,5 +1,5 @@
-"""The block-tile kernels (variants tb64x2, tb64x4, tb32x2, tb32x4: tiles of 48,
-48, 56 and 32 rows with 2, 3, 3 and 4 steps per launch) against the one-step
+"""The block-tile kernels (variants tb64x2, tb64x4, tb32x2, tb32x4: tiles of 32,
+48, 64 and 32 rows with 2, 3, 3 and 4 steps per launch) against the one-step
 streaming kernel, bit for bit, at the sizes where their tilings change: grids
 inside one tile, one row or column more, sides that end a tile on each of its
 rows, and the automatic choice on both sides of its rule."""
