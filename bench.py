@@ -414,10 +414,8 @@ def bench_inverse(seed, n=32, iters=100, n_steps=1000, frame_every=50, per_insta
 
 def bench_heun(seed, size=1024, n_steps=2000):
     """TimeIntegrator.HEUN (cardiax/solve.py:103-111) on the single-tissue
-    workload: two streaming launches per step. Algorithmic bytes per Heun
-    cell-step: stage 1 reads v, w, u, D and writes k1 (28 B); stage 2 reads
-    x0, k1 and D, rebuilds x1 = x0 + dt k1 in registers and writes the state
-    (40 B): 68 B."""
+    workload: one launch per step, both stages on chip. Algorithmic bytes per
+    Heun cell-step: reads v, w, u, D and writes v, w, u: 28 B."""
     import torch
 
     from cardiax_amd import solve, workloads
@@ -437,14 +435,11 @@ def bench_heun(seed, size=1024, n_steps=2000):
     torch.cuda.synchronize()
     sec = e0.elapsed_time(e1) / 1e3
     gcups = size * size * n_steps / sec / 1e9
-    # HBM bytes per Heun step from the committed PMC summary of both stages (None if absent)
-    R = 2 if size * size <= 1536 * 1024 else 4
-    t1 = measured_traffic("k_stream_heun<%d, 1>" % R, size, size)
-    t2 = measured_traffic("k_stream_heun<%d, 2>" % R, size, size)
-    traffic = t1 + t2 if t1 is not None and t2 is not None else None
-    return {"workload": "%dx%d grid, %d Heun steps (two launches each)" % (size, size, n_steps),
+    # HBM bytes per Heun step from the committed PMC summary (None if absent)
+    traffic = measured_traffic("k_block<5, 8, 2, heun>", size, size)
+    return {"workload": "%dx%d grid, %d Heun steps (one launch each)" % (size, size, n_steps),
             "gcups": round(gcups, 3), "us_per_step": round(sec / n_steps * 1e6, 3),
-            "hbm_frac": round(gcups * 68 / HBM_PEAK_GBS, 4),
+            "hbm_frac": round(gcups * 28 / HBM_PEAK_GBS, 4),
             "traffic_bytes_per_step": traffic,
             "u_finite": bool(torch.isfinite(out.u).all().item())}
 

@@ -113,7 +113,7 @@ k_batch_step(const SimDesc* __restrict__ sims, const TileItem* __restrict__ item
   const float dt = uni(S.dt), inv_dx2 = uni(S.inv_dx2);
   const int sel = item.flags | (mask ? 4 : 0);
 #define FK_BT(X, Y, ST)                                                                    \
-  stream_tile<R, true, X, Y, ST, BatchStimView, false, 0, true>(c, Dp, nullptr, i0, i1, i2, H, W,  \
+  stream_tile<R, true, X, Y, ST, BatchStimView, false, true>(c, Dp, nullptr, i0, i1, i2, H, W,  \
                                                                 sv, dt, inv_dx2, o0, o1, o2,      \
                                                                 item.rs, item.cs)
   switch (sel) {

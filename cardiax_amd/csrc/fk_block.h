@@ -174,8 +174,11 @@ __device__ __forceinline__ int row_edge(int i0, int R, int H) {
 }
 
 // The tile at (rsp, csp) over n_lev <= K levels. lds: Cfg::lds_floats floats.
-// Every wave of the block calls it (a barrier between levels).
-template <class Cfg, int YG, class SV>
+// Every wave of the block calls it (a barrier between levels). HEUN: levels
+// come in pairs, the two stages of a Heun step (cardiax/solve.py:73-85): an odd
+// level forms x1 = x0 + dt k1 and keeps x0 and k1, the even one x0 + (k1 + k2)
+// dt / 2, by the operations of stream_tile's stages; n_lev is even.
+template <class Cfg, int YG, bool HEUN, class SV>
 __device__ __forceinline__ void block_tile(const Coef& c, const BlockIO& io, int H, int W,
                                            const SV& sv, int n_lev, float dt, float inv_dx2,
                                            const BlockSpan& rsp, const BlockSpan& csp,
@@ -200,6 +203,7 @@ __device__ __forceinline__ void block_tile(const Coef& c, const BlockIO& io, int
   const float k2 = inv_dx2 * (1.0f / 144.0f);
 
   float u[R], v[R], w[R], Dc[R], Dx[R], Dy[R];
+  float x0[HEUN ? 3 * R : 1], k1[HEUN ? 3 * R : 1];  // v, w, u of the rows
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     u[k] = ldr(io.u, i0 + k);
@@ -362,6 +366,17 @@ __device__ __forceinline__ void block_tile(const Coef& c, const BlockIO& io, int
             jion = (sval != 0.0f) ? sval : jion;
           }
           const float du = del[k] + jion;
+          if (HEUN && (l & 1) == 0) {
+            const float half = dt * 0.5f;
+            v[k] = fmaf(k1[3 * k] + dv, half, x0[3 * k]);
+            w[k] = fmaf(k1[3 * k + 1] + dw, half, x0[3 * k + 1]);
+            u[k] = fmaf(k1[3 * k + 2] + du, half, x0[3 * k + 2]);
+            continue;
+          }
+          if constexpr (HEUN) {
+            x0[3 * k] = v[k], x0[3 * k + 1] = w[k], x0[3 * k + 2] = u[k];
+            k1[3 * k] = dv, k1[3 * k + 1] = dw, k1[3 * k + 2] = du;
+          }
           v[k] = fmaf(dt, dv, v[k]);
           w[k] = fmaf(dt, dw, w[k]);
           u[k] = fmaf(dt, du, u[k]);
@@ -414,17 +429,17 @@ __device__ __forceinline__ int block_sides(const BlockSpan& c, int C, int W) {
 }
 
 // block_tile of the tile in band `band` and strip `strip`.
-template <class Cfg, class SV>
+template <class Cfg, bool HEUN, class SV>
 __device__ __forceinline__ void block_tile_at(const Coef& c, const BlockIO& io, int H, int W,
                                               const SV& sv, int n_lev, float dt, float inv_dx2,
                                               const BlockAxis& ra, const BlockAxis& ca, int band,
                                               int strip, float* lds) {
   const BlockSpan r = block_span(ra, band), s = block_span(ca, strip);
   switch (block_sides(s, Cfg::C, W)) {
-    case 0: block_tile<Cfg, 0>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
-    case 1: block_tile<Cfg, 1>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
-    case 2: block_tile<Cfg, 2>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
-    default: block_tile<Cfg, 3>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
+    case 0: block_tile<Cfg, 0, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
+    case 1: block_tile<Cfg, 1, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
+    case 2: block_tile<Cfg, 2, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
+    default: block_tile<Cfg, 3, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
   }
 }
 
@@ -468,14 +483,14 @@ __device__ __forceinline__ BlockPlace block_place(int b, const BlockOrder& o, co
   return {g * kBlockGroup + rem - strip * bands, strip};
 }
 
-template <class Cfg>
+template <class Cfg, bool HEUN>
 __global__ void __launch_bounds__(Cfg::waves * 64)
 k_block(Coef c, BlockIO io, int H, int W, BlockStim st, int n_lev, float dt, float inv_dx2,
         BlockAxis ra, BlockAxis ca, BlockOrder ord) {
   __shared__ float lds[Cfg::lds_floats];
   const BlockPlace at = block_place(blockIdx.x, ord, ra, ca);
   const BlockStimArgs sv{st};
-  block_tile_at<Cfg>(c, io, H, W, sv, n_lev, dt, inv_dx2, ra, ca, at.band, at.strip, lds);
+  block_tile_at<Cfg, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, ra, ca, at.band, at.strip, lds);
 }
 
 }  // namespace fk

@@ -421,6 +421,19 @@ static int default_variant(int H, int W) {
 }
 static int resolve_variant(int v) { return v == kAuto ? (int)kStream2 : v; }
 
+// The tiling with the least a + b ceil(tiles / 256) of those offered.
+struct LeastRounds {
+  int best = -1;
+  double least = 0.0;
+  template <class Cfg>
+  void offer(int id, Cfg, int H, int W, double a, double b) {
+    constexpr int64_t kCUs = 256;
+    const int64_t tiles = (int64_t)Cfg::row_axis(H).n * Cfg::col_axis(W).n;
+    const double us = a + b * (double)((tiles + kCUs - 1) / kCUs);
+    if (best < 0 || us < least) best = id, least = us;
+  }
+};
+
 // The variant an automatic solve of several steps runs when the shape was not
 // tuned: block tiles, which equal the streaming kernels of default_variant bit
 // for bit. A launch takes the GPU's 256 CUs in rounds of tiles, and each tiling's
@@ -434,20 +447,12 @@ static int resolve_variant(int v) { return v == kAuto ? (int)kStream2 : v; }
 static int auto_variant(int H, int W) {
   const int d = default_variant(H, W);
   if (d == kTile16) return d;  // narrow grids above 8 M cells: another rounding
-  constexpr int64_t kCUs = 256;
-  int best = kAuto;
-  double least = 0.0;
-  auto offer = [&](int v, auto cfg, double a, double b) {
-    typedef decltype(cfg) Cfg;
-    const int64_t tiles = (int64_t)Cfg::row_axis(H).n * Cfg::col_axis(W).n;
-    const double us = a + b * (double)((tiles + kCUs - 1) / kCUs);
-    if (best == kAuto || us < least) best = v, least = us;
-  };
-  offer(kBlock32x4, Block32x4{}, 1.0, 1.05);
-  offer(kBlock48x3, Block48x3{}, 1.7, 1.25);
-  offer(kBlock64x3, Block64x3{}, 1.4, 2.05);
-  offer(kBlock32x2, Block32x2{}, 2.2, 1.0);
-  return best;
+  LeastRounds r;
+  r.offer(kBlock32x4, Block32x4{}, H, W, 1.0, 1.05);
+  r.offer(kBlock48x3, Block48x3{}, H, W, 1.7, 1.25);
+  r.offer(kBlock64x3, Block64x3{}, H, W, 1.4, 2.05);
+  r.offer(kBlock32x2, Block32x2{}, H, W, 2.2, 1.0);
+  return r.best;
 }
 
 // The variant of a solve of several steps.
@@ -561,22 +566,29 @@ static hipError_t launch_step(int variant, bool euler, const Coef& c, const floa
   return hipGetLastError();
 }
 
+// n_lev (at most Cfg::steps) levels on every tile.
+template <class Cfg, bool HEUN>
+static hipError_t launch_tiles(const Coef& c, const BlockIO& io, int H, int W,
+                               const BlockStim& st, int n_lev, float dt, float inv_dx2,
+                               hipStream_t s) {
+  const BlockAxis ra = Cfg::row_axis(H), ca = Cfg::col_axis(W);
+  k_block<Cfg, HEUN><<<(unsigned)(ra.n * ca.n), Cfg::waves * 64, 0, s>>>(
+      c, io, H, W, st, n_lev, dt, inv_dx2, ra, ca, make_block_order(ra, ca));
+  return hipGetLastError();
+}
+
 // n_lev steps (at most the variant's) of block variant v.
 static hipError_t launch_block(int v, const Coef& c, const BlockIO& io, int H, int W,
                                const BlockStim& st, int n_lev, float dt, float inv_dx2,
                                hipStream_t s) {
-  auto go = [&](auto cfg) {
-    typedef decltype(cfg) Cfg;
-    const BlockAxis ra = Cfg::row_axis(H), ca = Cfg::col_axis(W);
-    k_block<Cfg><<<(unsigned)(ra.n * ca.n), Cfg::waves * 64, 0, s>>>(
-        c, io, H, W, st, n_lev, dt, inv_dx2, ra, ca, make_block_order(ra, ca));
-    return hipGetLastError();
-  };
   switch (v) {
-    case kBlock32x2: return go(Block32x2{});
-    case kBlock48x3: return go(Block48x3{});
-    case kBlock64x3: return go(Block64x3{});
-    default: return go(Block32x4{});
+    case kBlock32x2:
+      return launch_tiles<Block32x2, false>(c, io, H, W, st, n_lev, dt, inv_dx2, s);
+    case kBlock48x3:
+      return launch_tiles<Block48x3, false>(c, io, H, W, st, n_lev, dt, inv_dx2, s);
+    case kBlock64x3:
+      return launch_tiles<Block64x3, false>(c, io, H, W, st, n_lev, dt, inv_dx2, s);
+    default: return launch_tiles<Block32x4, false>(c, io, H, W, st, n_lev, dt, inv_dx2, s);
   }
 }
 
@@ -586,26 +598,43 @@ static void block_stim(const StimSchedule& sched, double t, int n_lev, BlockStim
     st.act[j] = j < n_lev ? sched.mask(t + (double)j) : 0u;
 }
 
-// One stage of a Heun step on the default band height for the shape.
-static hipError_t launch_heun(int stage, const Coef& c, const float* D, const float* const x[3],
-                              int H, int W, const StimArgs& sa, float dt, float inv_dx2,
-                              float* const o[3], const HeunIO& io, hipStream_t s) {
-  const bool two = (size_t)H * W <= 1536 * 1024;  // 2-row bands up to 1.5 M cells
-  const StreamGeom g = two ? make_stream_geom<2>(H, W) : make_stream_geom<4>(H, W);
-#define FK_HEUN(R, ST)                                                                     \
-  k_stream_heun<R, ST><<<g.blocks, 256, 0, s>>>(c, D, x[0], x[1], x[2], H, W, sa, dt, inv_dx2, \
-                                                o[0], o[1], o[2], g, io)
-  if (two) {
-    if (stage == 1) FK_HEUN(2, 1); else FK_HEUN(2, 2);
-  } else {
-    if (stage == 1) FK_HEUN(4, 1); else FK_HEUN(4, 2);
+// Heun steps per launch (n <= 2) on block tiles, each two levels. The tiling is
+// chosen as in auto_variant. Two launches per step of a streaming kernel, the
+// slope k1 in memory between them, and this, us per step: 150 x 170 7.3 and 4.7
+// (32 rows, 2 steps), 517 x 389 9.1 and 6.1 (48 rows, 2 steps), 760^2 14.1 and 9.8
+// (64 rows, 1 step), 1000 x 760 18.1 and 11.6, 1200^2 30.1 and 18.9, 3000 x 2000 101
+// and 57 (40 rows, 1 step).
+typedef BlockCfg<2, 16, 4> Heun32x2;
+typedef BlockCfg<3, 16, 4> Heun48x2;
+typedef BlockCfg<4, 16, 2> Heun64x1;
+typedef BlockCfg<5, 8, 2> Heun40x1;
+
+enum HeunTiling { kHeun32x2, kHeun48x2, kHeun64x1, kHeun40x1 };
+
+static int heun_tiling(int H, int W) {
+  LeastRounds r;
+  r.offer(kHeun32x2, Heun32x2{}, H, W, 2.0, 2.9);
+  r.offer(kHeun48x2, Heun48x2{}, H, W, 1.8, 4.2);
+  r.offer(kHeun64x1, Heun64x1{}, H, W, 2.2, 7.45);
+  r.offer(kHeun40x1, Heun40x1{}, H, W, 4.3, 3.55);
+  return r.best;
+}
+
+static int heun_steps(int tiling) { return tiling == kHeun32x2 || tiling == kHeun48x2 ? 2 : 1; }
+
+static hipError_t launch_heun(int tiling, const Coef& c, const BlockIO& io, int H, int W,
+                              const BlockStim& st, int n, float dt, float inv_dx2,
+                              hipStream_t s) {
+  switch (tiling) {
+    case kHeun32x2: return launch_tiles<Heun32x2, true>(c, io, H, W, st, 2 * n, dt, inv_dx2, s);
+    case kHeun48x2: return launch_tiles<Heun48x2, true>(c, io, H, W, st, 2 * n, dt, inv_dx2, s);
+    case kHeun64x1: return launch_tiles<Heun64x1, true>(c, io, H, W, st, 2 * n, dt, inv_dx2, s);
+    default: return launch_tiles<Heun40x1, true>(c, io, H, W, st, 2 * n, dt, inv_dx2, s);
   }
-#undef FK_HEUN
-  return hipGetLastError();
 }
 
 // Heun steps at times t .. t_end-1 (cardiax/solve.py:103-111) from `in` to
-// `out`; the workspace holds k1 (3 fields) and a ping-pong state.
+// `out`; the workspace holds a ping-pong state.
 static int32_t heun_loop(const fk_params* params, const float* D, const float* const in[3],
                          int32_t H, int32_t W, const fk_stimulus* stimuli, int32_t n_stimuli,
                          double t, int64_t steps, float dt, float dx, float* const out[3],
@@ -614,20 +643,22 @@ static int32_t heun_loop(const fk_params* params, const float* D, const float* c
   const Coef c = make_coef(*params);
   const float inv_dx2 = (float)(1.0 / ((double)dx * (double)dx));
   float* wk = (float*)work;
-  float* k1[3] = {wk, wk + n, wk + 2 * n};
-  float* ping[3] = {wk + 3 * n, wk + 4 * n, wk + 5 * n};
+  float* ping[3] = {wk, wk + n, wk + 2 * n};
   float* const* bufs[2] = {out, ping};
-  int dst = (steps % 2 == 1) ? 0 : 1;  // the last step lands in `out`
+  const int tiling = heun_tiling(H, W), per = heun_steps(tiling);
+  const int64_t launches = (steps + per - 1) / per;
+  int dst = (launches % 2 == 1) ? 0 : 1;  // the last launch lands in `out`
   const float* src[3] = {in[0], in[1], in[2]};
-  StimSchedule sched(stimuli, n_stimuli);
-  for (int64_t k = 0; k < steps; ++k) {
-    const StimArgs& sa = sched.at(t + (double)k);  // both stages at time t + k
-    // stage 1 writes only k1 (its state outputs are not written)
-    HeunIO io1{k1[0], k1[1], k1[2], nullptr, nullptr, nullptr};
-    HIP_CHECK(launch_heun(1, c, D, src, H, W, sa, dt, inv_dx2, k1, io1, s));
-    HeunIO io2{nullptr, nullptr, nullptr, k1[0], k1[1], k1[2]};
+  const StimSchedule sched(stimuli, n_stimuli);
+  BlockStim st{};
+  for (int i = 0; i < n_stimuli; ++i) st.f[i] = stimuli[i].field;
+  for (int64_t k = 0; k < steps; k += per) {
+    const int m = (int)std::min<int64_t>(per, steps - k);
+    for (int l = 0; l < 2 * m; ++l)  // both stages of step k + j at time t + k + j
+      st.act[l] = sched.mask(t + (double)(k + l / 2));
     float* const* d = bufs[dst];
-    HIP_CHECK(launch_heun(2, c, D, src, H, W, sa, dt, inv_dx2, d, io2, s));
+    const BlockIO io{D, src[0], src[1], src[2], d[0], d[1], d[2], 0, false};
+    HIP_CHECK(launch_heun(tiling, c, io, H, W, st, m, dt, inv_dx2, s));
     src[0] = d[0];
     src[1] = d[1];
     src[2] = d[2];

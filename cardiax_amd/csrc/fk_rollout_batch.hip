@@ -121,7 +121,7 @@ k_roll_step(const RollDesc* __restrict__ sims, const RollTile* __restrict__ item
   const float dt = uni(S.dt), inv_dx2 = uni(S.inv_dx2);
   const int sel = item.flags | (mask ? 4 : 0);
 #define FK_RS(X, Y, ST)                                                                   \
-  stream_tile<R, true, X, Y, ST, BatchStimView, false, 0, true>(c, Dp, nullptr, i0, i1, i2, H, \
+  stream_tile<R, true, X, Y, ST, BatchStimView, false, true>(c, Dp, nullptr, i0, i1, i2, H, \
                                                                 W, sv, dt, inv_dx2, o0, o1,   \
                                                                 o2, item.rs, item.cs)
   switch (sel) {

@@ -116,25 +116,13 @@ struct StimListView {
   __device__ const float* field(int m) const { return sa.f[m]; }
 };
 
-// The extra inputs and outputs of the two stages of a Heun step
-// (cardiax/solve.py:73-85). Stage 1 reads x0 and writes only the slope
-// k1 = step(x0). Stage 2 reads x0 (as the state) and k1, rebuilds
-// x1 = x0 + dt k1 in registers with the one fmaf stage 1 would have used,
-// evaluates k2 = step(x1) and writes x0 + (k1 + k2) dt / 2. x1 never goes to
-// memory: 68 bytes per cell-step instead of 92.
-struct HeunIO {
-  float *kv, *kw, *ku;              // stage 1: k1 out
-  const float *k1v, *k1w, *k1u;     // stage 2: k1 in
-};
-
 // PC: the static diffusion coefficients come precomputed from `cf`
-// (k_stream_coef) instead of being derived from D each step. HEUN: 0 = an
-// Euler step (EULER) or the derivatives, 1 / 2 = stage 1 / 2 of a Heun step.
-// FIELD_MAJOR: loads field by field with scalar row bases, measured faster
+// (k_stream_coef) instead of being derived from D each step. EULER: an Euler
+// step, else the derivatives. FIELD_MAJOR: loads field by field with scalar row bases, measured faster
 // when the fields stream from DRAM (the batch); otherwise in the order the
 // output rows need them, measured faster for grids held in the 256 MB cache.
 template <int R, bool EULER, bool XG, bool YG, bool STIM, class SV, bool PC = false,
-          int HEUN = 0, bool FIELD_MAJOR = false>
+          bool FIELD_MAJOR = false>
 __device__ __forceinline__ void stream_tile(const Coef& c, const float* __restrict__ D,
                                             const float4* __restrict__ cf,
                                             const float* __restrict__ v,
@@ -142,8 +130,7 @@ __device__ __forceinline__ void stream_tile(const Coef& c, const float* __restri
                                             const float* __restrict__ u, int H, int W,
                                             const SV& sv, float dt, float inv_dx2,
                                             float* __restrict__ o_v, float* __restrict__ o_w,
-                                            float* __restrict__ o_u, int rs, int cs,
-                                            const HeunIO& io = HeunIO{}) {
+                                            float* __restrict__ o_u, int rs, int cs) {
 #pragma clang fp contract(off)  // explicit fmaf only: identical rounding in every kernel
   const int lane = threadIdx.x & 63;
   const int col = cs - 4 + lane;                           // this lane's column
@@ -186,36 +173,18 @@ __device__ __forceinline__ void stream_tile(const Coef& c, const float* __restri
   float dd[PC ? 1 : R + 4];  // D rows rs-2 .. rs+R+1
   float4 cc[PC ? R : 1];     // precomputed coefficients of rows rs .. rs+R-1
   float vv[R], ww[R];
-  float h0[HEUN == 2 ? 3 * R : 1], hk[HEUN == 2 ? 3 * R : 1];  // stage 2: x0, k1 of the band
-  // Row k of state field f (0 v, 1 w, 2 u) from `a`. In stage 2 of a Heun step
-  // that is x1 = fmaf(dt, k1, x0) from x0 (`a`) and k1 (`ka`); the band's own
-  // rows also keep x0 and k1 for the final combination.
-  auto ldx = [&](const float* a, const float* ka, int k, int f) {
-    if constexpr (HEUN == 2) {
-      const float x0 = ldk(a, k), k1 = ldk(ka, k);
-      if (k >= 4 && k < R + 4) {
-        h0[3 * (k - 4) + f] = x0;
-        hk[3 * (k - 4) + f] = k1;
-      }
-      return fmaf(dt, k1, x0);
-    } else {
-      (void)ka;
-      (void)f;
-      return ldk(a, k);
-    }
-  };
   if constexpr (FIELD_MAJOR) {
     // Field by field: every u row of the window, then D, then v and w.
 #pragma unroll
-    for (int k = 0; k < R + 8; ++k) uu[k] = ldx(u, io.k1u, k, 2);
+    for (int k = 0; k < R + 8; ++k) uu[k] = ldk(u, k);
     if constexpr (!PC) {
 #pragma unroll
       for (int k = 0; k < R + 4; ++k) dd[k] = ldk(D, k + 2);
     }
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      vv[k] = ldx(v, io.k1v, k + 4, 0);
-      ww[k] = ldx(w, io.k1w, k + 4, 1);
+      vv[k] = ldk(v, k + 4);
+      ww[k] = ldk(w, k + 4);
     }
     if constexpr (PC) {
 #pragma unroll
@@ -230,20 +199,20 @@ __device__ __forceinline__ void stream_tile(const Coef& c, const float* __restri
     // flight.
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-      uu[k] = ldx(u, io.k1u, k, 2);
+      uu[k] = ldk(u, k);
       if constexpr (!PC)
         if (k >= 2 && k < 7) dd[k - 2] = ldk(D, k);
     }
     if constexpr (PC) cc[0] = ldc(0);
-    vv[0] = ldx(v, io.k1v, 4, 0);
-    ww[0] = ldx(w, io.k1w, 4, 1);
+    vv[0] = ldk(v, 4);
+    ww[0] = ldk(w, 4);
 #pragma unroll
     for (int j = 1; j < R; ++j) {
-      uu[j + 8] = ldx(u, io.k1u, j + 8, 2);
+      uu[j + 8] = ldk(u, j + 8);
       if constexpr (!PC) dd[j + 4] = ldk(D, j + 6);
       if constexpr (PC) cc[j] = ldc(j);
-      vv[j] = ldx(v, io.k1v, j + 4, 0);
-      ww[j] = ldx(w, io.k1w, j + 4, 1);
+      vv[j] = ldk(v, j + 4);
+      ww[j] = ldk(w, j + 4);
     }
   }
 
@@ -303,16 +272,7 @@ __device__ __forceinline__ void stream_tile(const Coef& c, const float* __restri
     }
     const float du = del_u + jion;
     if (out_col && (!XG || i < H)) {  // rows past the grid only when H < R
-      if constexpr (HEUN == 1) {  // k1 only
-        stk(io.kv, k + 4, dv);
-        stk(io.kw, k + 4, dw);
-        stk(io.ku, k + 4, du);
-      } else if constexpr (HEUN == 2) {  // x0 + (k1 + k2) dt / 2
-        const float half = dt * 0.5f;
-        stk(o_v, k + 4, fmaf(hk[3 * k] + dv, half, h0[3 * k]));
-        stk(o_w, k + 4, fmaf(hk[3 * k + 1] + dw, half, h0[3 * k + 1]));
-        stk(o_u, k + 4, fmaf(hk[3 * k + 2] + du, half, h0[3 * k + 2]));
-      } else if (EULER) {
+      if (EULER) {
         stk(o_v, k + 4, fmaf(dt, dv, vv[k]));
         stk(o_w, k + 4, fmaf(dt, dw, ww[k]));
         stk(o_u, k + 4, fmaf(dt, du, uc));
@@ -336,13 +296,12 @@ __host__ __device__ inline bool edge_band(int rs, int R, int H, int W) {
 // One wave per (strip, band) tile, band-major within a strip so that
 // consecutive tiles share row halos; four waves per block. PC: Euler steps
 // from precomputed coefficients (k_stream_c), else derived from D.
-template <int R, bool EULER, bool PC, int HEUN = 0>
+template <int R, bool EULER, bool PC>
 __device__ __forceinline__ void stream_kernel_body(
     const Coef& c, const float* __restrict__ D, const float4* __restrict__ cf,
     const float* __restrict__ v, const float* __restrict__ w, const float* __restrict__ u,
     int H, int W, const StimArgs& sa, float dt, float inv_dx2, float* __restrict__ o_v,
-    float* __restrict__ o_w, float* __restrict__ o_u, const StreamGeom& g,
-    const HeunIO& io = HeunIO{}) {
+    float* __restrict__ o_w, float* __restrict__ o_u, const StreamGeom& g) {
   const int tile = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x >> 6));
   if (tile >= g.n_tiles) return;  // whole wave leaves; the kernel has no barrier
   const int strip = tile / g.n_bands, band = tile - strip * g.n_bands;
@@ -353,8 +312,8 @@ __device__ __forceinline__ void stream_kernel_body(
   const int sel = (xg ? 1 : 0) | (yg ? 2 : 0) | (sa.n ? 4 : 0);
   const StimListView sv{sa};
 #define FK_TILE(X, Y, S)                                                                 \
-  stream_tile<R, EULER, X, Y, S, StimListView, PC, HEUN>(c, D, cf, v, w, u, H, W, sv, dt,  \
-                                                         inv_dx2, o_v, o_w, o_u, rs, cs, io)
+  stream_tile<R, EULER, X, Y, S, StimListView, PC>(c, D, cf, v, w, u, H, W, sv, dt, inv_dx2, \
+                                                   o_v, o_w, o_u, rs, cs)
   switch (sel) {
     case 0: FK_TILE(false, false, false); break;
     case 1: FK_TILE(true, false, false); break;
@@ -376,17 +335,6 @@ k_stream(Coef c, const float* __restrict__ D, const float* __restrict__ v,
          float* __restrict__ o_u, StreamGeom g) {
   stream_kernel_body<R, EULER, false>(c, D, nullptr, v, w, u, H, W, sa, dt, inv_dx2, o_v, o_w,
                                       o_u, g);
-}
-
-// Stage STAGE (1 or 2) of a Heun step on streaming bands of R rows.
-template <int R, int STAGE>
-__global__ void __launch_bounds__(256)
-k_stream_heun(Coef c, const float* __restrict__ D, const float* __restrict__ v,
-              const float* __restrict__ w, const float* __restrict__ u, int H, int W,
-              StimArgs sa, float dt, float inv_dx2, float* __restrict__ o_v,
-              float* __restrict__ o_w, float* __restrict__ o_u, StreamGeom g, HeunIO io) {
-  stream_kernel_body<R, true, false, STAGE>(c, D, nullptr, v, w, u, H, W, sa, dt, inv_dx2, o_v,
-                                            o_w, o_u, g, io);
 }
 
 template <int R>

@@ -141,7 +141,7 @@ def step_euler(state, t, params, diffusivity, stimuli, dt, dx) -> State:
 
 def step_heun(state, t, params, diffusivity, stimuli, dt, dx) -> State:
     """cardiax/solve.py:73-85: k1 = step(x, t), k2 = step(x + dt k1, t),
-    x + (k1 + k2) dt / 2, as two fused launches (fk_step_heun)."""
+    x + (k1 + k2) dt / 2, in one launch (fk_step_heun)."""
     dev = require_gpu("step_heun")
     st = _dev_state(state, dev)
     H, W = _shape_of(st)

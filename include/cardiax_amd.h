@@ -212,14 +212,13 @@ int32_t fk_forward_euler_plain(const fk_params* params, const float* D, const fl
                                float* w_out, float* u_out, void* work, size_t work_bytes,
                                void* stream);
 
-/* Scratch bytes fk_step_heun and fk_forward_heun need for an H x W grid
- * (the stage-1 slope and a ping-pong state: 6 fields). */
+/* Scratch bytes fk_step_heun and fk_forward_heun ask for on an H x W grid (6
+ * fields; they use 3, a ping-pong state). */
 size_t fk_heun_workspace_bytes(int32_t H, int32_t W);
 
 /* cardiax/solve.py:73-85 -- one Heun step at time t: k1 = step(x, t),
- * x1 = x + dt k1, k2 = step(x1, t), out = x + (k1 + k2) dt / 2. Two fused
- * launches: the first writes k1 to the workspace, the second rebuilds x1
- * from x and k1 in registers. Outputs must not alias inputs or the
+ * x1 = x + dt k1, k2 = step(x1, t), out = x + (k1 + k2) dt / 2. One
+ * launch, k1 and x1 stay on chip. Outputs must not alias inputs or the
  * workspace. */
 int32_t fk_step_heun(const fk_params* params, const float* D, const float* v, const float* w,
                      const float* u, int32_t H, int32_t W, const fk_stimulus* stimuli,
