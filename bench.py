@@ -179,9 +179,13 @@ def bench_batched(n_sims, n_steps, seed, per_sim_steps=64):
         n_bad = sum(int(not bool(torch.isfinite(x.u).all().item())) for x in b.states)
         umax = max(float(x.u.abs().max().item()) for x in b.states)
     batched = cells * n_steps / el / 1e9
-    # the tuned work list: one or two Euler steps per launch
-    per_launch = 2 if tuned["two_step"] else 1
-    kernel = ("k_batch_step_t<%d>" if tuned["two_step"] else "k_batch_step<%d>") % tuned["rows"]
+    # the tuned work list: one Euler step per launch, or block tiles of 32 rows (2 steps, for
+    # a batch this size) or 48 rows (3)
+    per_launch = 1
+    kernel = "k_batch_step<%d>" % tuned["rows"]
+    if tuned["two_step"]:
+        per_launch, kernel = {8: (2, "k_batch_block<4, 8, 2>"),
+                              16: (3, "k_batch_block<4, 12, 3>")}[tuned["rows"]]
     # per-simulation launches: the same simulations, one call each
     for x in bs[:4]:
         solve._forward_euler(x.state, 0, 4, x.params, x.diffusivity, x.stimuli, x.dt, x.dx)

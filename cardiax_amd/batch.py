@@ -2,10 +2,9 @@
 
 Each simulation is what one ``cardiax.solve._forward_euler`` call advances
 (cardiax/solve.py:92-100): its own state, parameter set, D-map, stimuli and
-time. ``Batch`` builds one work list over all of them; every Euler step of
-the whole batch is one kernel launch, and the launches are replayed from a
-recorded hipGraph (one graph launch per 32 steps); with a two-step option
-each launch advances the batch two steps. The reference has no
+time. ``Batch`` builds one work list over all of them; one kernel launch
+advances the whole batch up to four Euler steps, and the launches are replayed
+from a recorded hipGraph (one graph launch per 32 steps). The reference has no
 batched path: its experiments loop over simulations one call at a time
 (experiments/generate_fd_data_128.py:25-56).
 """
@@ -99,8 +98,9 @@ class Batch:
 
     def autotune(self, n_steps: int = 64) -> dict:
         """Time every available work-list option (bands of 2, 4, 8 or 16 rows
-        advanced one step per launch; bands of 8 or 16 rows advanced two steps
-        per launch when every simulation fits) and keep the fastest for later
+        advanced one step per launch; block tiles of 32 or 48 rows, "t8" and
+        "t16", advanced 2 to 4 steps per launch when every simulation fits) and
+        keep the fastest for later
         runs (fk_batch_autotune); the simulations' states are not touched.
         Returns ``{"rows": R, "two_step": bool, "times_ms": {option: ms}}``
         with options "2", "4", "8", "16", "t8", "t16" (unavailable ones left

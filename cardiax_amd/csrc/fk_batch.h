@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "fk_block.h"
 #include "fk_device.h"
 
 namespace fk {
@@ -76,6 +77,52 @@ inline std::vector<T> xcd_order(const std::vector<std::vector<T>>& runs, int per
       for (int k = 0; k < per_wg; ++k)
         out.push_back(j * per_wg + k < lists[x].size() ? lists[x][j * per_wg + k] : pad);
   return out;
+}
+
+// One block tile (fk_block.h) of problem `sim`; sim < 0: padding.
+struct BlockItem {
+  int sim;
+  BlockSpan r, c;
+  int pad;
+};
+
+// The simulation's stimuli at the levels of a launch: bits 4 l .. 4 l + 3 of
+// `packed` are the activity mask of level l.
+static_assert(FK_BATCH_MAX_STIMULI <= 4 && kBlockMaxSteps <= 8, "masks of a launch in one word");
+struct BatchBlockStim {
+  const BatchStim* s;
+  uint32_t packed;
+  __device__ uint32_t active(int l) const { return (packed >> (4 * l)) & 15u; }
+  __device__ const float* field(int m) const { return s[m].field; }
+};
+
+// masks: the activity words of one simulation, `stride` apart per step.
+__device__ __forceinline__ uint32_t pack_masks(const uint32_t* masks, int stride, int n_lev) {
+  uint32_t p = 0;
+  for (int l = 0; l < n_lev; ++l) p |= (masks[(size_t)l * stride] & 15u) << (4 * l);
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
+}
+
+// The tiles of an H x W problem, in the patches of block_place.
+template <class Cfg>
+inline void append_block_items(int sim, int H, int W, std::vector<BlockItem>& out) {
+  const BlockAxis ra = Cfg::row_axis(H), ca = Cfg::col_axis(W);
+  for (int g = 0; g < ra.n; g += kBlockGroup)
+    for (int strip = 0; strip < ca.n; ++strip)
+      for (int band = g; band < std::min(g + kBlockGroup, ra.n); ++band)
+        out.push_back({sim, block_span(ra, band), block_span(ca, strip), 0});
+}
+
+// The work list of block tiles over the XCDs: runs of neighbouring tiles, at
+// least eight runs per XCD so that the lists come out even.
+inline std::vector<BlockItem> block_work_list(const std::vector<BlockItem>& items) {
+  const size_t run = std::max<size_t>(1, items.size() / (8 * kXcds));
+  std::vector<std::vector<BlockItem>> runs;
+  for (size_t k = 0; k < items.size(); k += run)
+    runs.emplace_back(items.begin() + k, items.begin() + std::min(k + run, items.size()));
+  BlockItem pad{};
+  pad.sim = -1;
+  return xcd_order(runs, 1, pad);
 }
 
 }  // namespace fk

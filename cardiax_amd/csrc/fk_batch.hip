@@ -1,17 +1,16 @@
 // Batched forward Euler: many independent simulations of uneven sizes and
 // parameter sets advanced together.
 //
-// One launch over a work list that holds every (column strip, row band) tile
-// of every simulation advances the whole batch by one Euler step (the
-// streaming step, stream_tile) or by two (the two-step streaming tile,
-// stream_t_tile, which reads and writes the state once for both); each tile
-// takes its simulation's constants, D-map and stimuli from a device-resident
-// descriptor. Stimulus activity follows the law of cardiax/solve.py:262-267
+// One launch over a work list that holds every tile of every simulation
+// advances the whole batch by one Euler step (streaming tiles, stream_tile) or
+// by two to four (block tiles, block_tile, which read and write the state once
+// for all of them); each tile takes its simulation's constants, D-map and
+// stimuli from a device-resident descriptor. Stimulus activity follows the law of cardiax/solve.py:262-267
 // (floor modulo in double precision, as on the host path), evaluated on the
 // device by one small kernel for up to kGraphSteps steps at a time. Steps are
 // recorded once into a hipGraph (that kernel, the step launches and a
 // one-thread kernel that advances the device-side step counter) and the graph
-// is replayed: the host issues one graph launch per kGraphSteps steps for the
+// is replayed: the host issues one graph launch per graph_steps steps for the
 // whole batch.
 //
 // Reference: the batch has no counterpart in the reference, which runs one
@@ -33,17 +32,22 @@
 namespace fk {
 
 // Work-list options, chosen by fk_batch_autotune: one step per launch on bands
-// of 2, 4, 8 or 16 rows, or two steps per launch on bands of 8 or 16 rows
-// (those only when every simulation fits stream_t_fits).
+// of 2, 4, 8 or 16 rows, or several steps per launch on block tiles: of 32 rows
+// (option 8 | FK_BATCH_TWO_STEP) or of 48 rows (16 | FK_BATCH_TWO_STEP). Block
+// tiles cover every grid, but these two options are offered and accepted only
+// for simulations of at least 2 R + 16 rows (R the option's number) and 56..96
+// or >= 104 columns, the sizes they were first defined for. An untuned batch
+// runs the block tiling that LeastRounds finds.
 constexpr int kNumRowOpts = FK_BATCH_N_OPTIONS;
 constexpr int kBatchRows[kNumRowOpts] = {2, 4, 8, 16, 8, 16};
 constexpr bool kBatchTwo[kNumRowOpts] = {false, false, false, false, true, true};
-constexpr int kDefaultRowOpt = 2;  // 8 rows, one step
-constexpr int kGraphSteps = 32;   // Euler steps recorded in one graph (even)
+constexpr int kGraphSteps = 32;  // Euler steps of one mask window; at most as many in a graph
 
-// The one-step option with the band height of option o (the odd last step of
-// a two-step option).
-constexpr int one_step_opt(int o) { return o == 4 ? 2 : o == 5 ? 3 : o; }
+// Block tiling of a batch option.
+enum BatchBlock { kNone, kBatch32x4, kBatch32x2, kBatch48x3 };
+constexpr int batch_steps(int blk) {
+  return blk == kBatch32x4 ? 4 : blk == kBatch48x3 ? 3 : blk == kBatch32x2 ? 2 : 1;
+}
 
 struct SimDesc {
   Coef c;
@@ -129,26 +133,18 @@ k_batch_step(const SimDesc* __restrict__ sims, const TileItem* __restrict__ item
 #undef FK_BT
 }
 
-// Two Euler steps of every tile (two-step bands of R rows). Reads
-// state[parity], writes state[parity ^ 1]; masks1 / masks2 hold the activity
-// of the two steps.
-template <int R>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-k_batch_step_t(const SimDesc* __restrict__ sims, const TileItem* __restrict__ items,
-               int n_items, const uint32_t* __restrict__ masks1,
-               const uint32_t* __restrict__ masks2, int parity) {
-  const int it = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x >> 6));
-  if (it >= n_items) return;
-  TileItem item = items[it];
-  item.sim = __builtin_amdgcn_readfirstlane(item.sim);
-  item.cs = __builtin_amdgcn_readfirstlane(item.cs);
-  item.rs = __builtin_amdgcn_readfirstlane(item.rs);
-  item.flags = __builtin_amdgcn_readfirstlane(item.flags);
-  const SimDesc& S = sims[item.sim];
-  const uint32_t m1 = __builtin_amdgcn_readfirstlane(masks1[item.sim]);
-  const uint32_t m2 = __builtin_amdgcn_readfirstlane(masks2[item.sim]);
-  const int n_stim = uni(S.n_stim);
-  const BatchStimView sv1{S.stim, n_stim, m1}, sv2{S.stim, n_stim, m2};
+// n_lev Euler steps of every block tile. Reads state[parity], writes
+// state[parity ^ 1]; masks holds the activity of the steps, n_sims words each.
+template <class Cfg>
+__global__ void __launch_bounds__(Cfg::waves * 64)
+k_batch_block(const SimDesc* __restrict__ sims, const BlockItem* __restrict__ items, int n_sims,
+              const uint32_t* __restrict__ masks, int n_lev, int parity) {
+  __shared__ float lds[Cfg::lds_floats];
+  const BlockItem& it = items[blockIdx.x];
+  const int sim = uni(it.sim);
+  if (sim < 0) return;  // padding of the XCD order: the whole block leaves
+  const SimDesc& S = sims[sim];
+  const BatchBlockStim sv{S.stim, pack_masks(masks + sim, n_sims, n_lev)};
   Coef c = S.c;
   c.V_c = uni(c.V_c); c.V_v = uni(c.V_v); c.V_csi = uni(c.V_csi); c.kk = uni(c.kk);
   c.kk_off = uni(c.kk_off);
@@ -156,36 +152,13 @@ k_batch_step_t(const SimDesc* __restrict__ sims, const TileItem* __restrict__ it
   c.inv_twp = uni(c.inv_twp); c.inv_twm = uni(c.inv_twm); c.inv_td = uni(c.inv_td);
   c.inv_t0 = uni(c.inv_t0); c.inv_tr = uni(c.inv_tr); c.inv_tsi = uni(c.inv_tsi);
   c.inv_cm = uni(c.inv_cm);
-  const float* Dp = uni(S.D);
-  const float* i0 = uni(S.buf[parity][0]);
-  const float* i1 = uni(S.buf[parity][1]);
-  const float* i2 = uni(S.buf[parity][2]);
-  float* o0 = uni(S.buf[parity ^ 1][0]);
-  float* o1 = uni(S.buf[parity ^ 1][1]);
-  float* o2 = uni(S.buf[parity ^ 1][2]);
-  const int H = uni(S.H), W = uni(S.W);
-  const float dt = uni(S.dt), inv_dx2 = uni(S.inv_dx2);
-  // flags: bits 0-1 the band's kind (0 interior, 1 first, 2 last), bit 2 a
-  // strip at a side
-  const int sel = (item.flags & 3) * 4 + ((item.flags & 4) ? 2 : 0) + ((m1 | m2) ? 1 : 0);
-#define FK_BT2(X, Y, ST)                                                                  \
-  stream_t_tile<R, X, Y, ST, BatchStimView>(c, Dp, i0, i1, i2, H, W, sv1, sv2, dt, inv_dx2, \
-                                            o0, o1, o2, item.rs, item.cs)
-  switch (sel) {
-    case 0: FK_BT2(0, false, false); break;
-    case 1: FK_BT2(0, false, true); break;
-    case 2: FK_BT2(0, true, false); break;
-    case 3: FK_BT2(0, true, true); break;
-    case 4: FK_BT2(1, false, false); break;
-    case 5: FK_BT2(1, false, true); break;
-    case 6: FK_BT2(1, true, false); break;
-    case 7: FK_BT2(1, true, true); break;
-    case 8: FK_BT2(2, false, false); break;
-    case 9: FK_BT2(2, false, true); break;
-    case 10: FK_BT2(2, true, false); break;
-    default: FK_BT2(2, true, true); break;
-  }
-#undef FK_BT2
+  const BlockIO io{uni(S.D), uni(S.buf[parity][0]), uni(S.buf[parity][1]),
+                   uni(S.buf[parity][2]), uni(S.buf[parity ^ 1][0]), uni(S.buf[parity ^ 1][1]),
+                   uni(S.buf[parity ^ 1][2]), 0, false};
+  const BlockSpan r{uni(it.r.o), uni(it.r.a), uni(it.r.b)};
+  const BlockSpan q{uni(it.c.o), uni(it.c.a), uni(it.c.b)};
+  block_tile_any<Cfg, false>(c, io, uni(S.H), uni(S.W), sv, n_lev, uni(S.dt), uni(S.inv_dx2), r,
+                             q, lds);
 }
 
 // n floats from src to dst, blocks [blk, blk + stride, ...) of 1024: 16-byte
@@ -238,14 +211,16 @@ using namespace fk;
 // Opaque batch handle.
 struct fk_batch {
   int n_sims = 0;
-  int opt = kDefaultRowOpt;  // index into kBatchRows
+  int opt = 0, untuned = 0;        // index into kBatchRows: in use, until tuned
+  int block[kNumRowOpts] = {};     // BatchBlock of the option
+  bool offered[kNumRowOpts] = {};  // accepted by fk_batch_set_rows
   int n_items_opt[kNumRowOpts] = {};
   std::vector<fk_sim> host_sims;   // caller's descriptors (state pointers)
   std::vector<size_t> offset;      // per-sim cell offset in the pools
   size_t total_cells = 0;
   char* dev = nullptr;             // one allocation: descriptors, items, counter, pools
   SimDesc* d_sims = nullptr;
-  TileItem* d_items[kNumRowOpts] = {};
+  char* d_items[kNumRowOpts] = {};  // TileItem (one step) or BlockItem
   int64_t* d_step = nullptr;
   uint32_t* d_mask = nullptr;  // stimulus activity: kGraphSteps x n_sims
   float* pool[2] = {nullptr, nullptr};  // ping-pong pools of 3 * total_cells floats
@@ -290,29 +265,22 @@ int32_t fk_batch_create(const fk_sim* sims, int32_t n, fk_batch** out) {
   b->n_sims = n;
   b->host_sims.assign(sims, sims + n);
   std::vector<TileItem> items[kNumRowOpts];
+  std::vector<BlockItem> tiles[kNumRowOpts];
   b->offset.resize(n);
+  int64_t n32x4 = 0, n32x2 = 0, n48x3 = 0;
+  bool fit[2] = {true, true};
   for (int i = 0; i < n; ++i) {
     const fk_sim& s = sims[i];
     b->offset[i] = b->total_cells;
     b->total_cells += (size_t)s.H * s.W;
+    n32x4 += block_tiles<Block32x4>(s.H, s.W);
+    n32x2 += block_tiles<Block32x2>(s.H, s.W);
+    n48x3 += block_tiles<Block48x3>(s.H, s.W);
+    fit[0] = fit[0] && stream_t_fits<8>(s.H, s.W);
+    fit[1] = fit[1] && stream_t_fits<16>(s.H, s.W);
     for (int o = 0; o < kNumRowOpts; ++o) {
+      if (kBatchTwo[o]) continue;
       const int R = kBatchRows[o];
-      if (kBatchTwo[o]) {  // two-step bands, placed from both ends of each axis
-        const StreamTGeom g = o == 4 ? make_stream_t_geom<8>(s.H, s.W)
-                                     : make_stream_t_geom<16>(s.H, s.W);
-        for (int strip = 0; strip < g.n_strips; ++strip)
-          for (int band = 0; band < g.n_bands; ++band) {
-            TileItem t;
-            t.sim = i;
-            t.cs = stream_t_origin(strip, g.n_strips, kTOut, s.W);
-            t.rs = stream_t_origin(band, g.n_bands, R, s.H);
-            const int xe = t.rs == 0 ? 1 : (t.rs == s.H - R ? 2 : 0);
-            const bool yg = t.cs == 0 || t.cs == s.W - kTOut;
-            t.flags = xe | (yg ? 4 : 0);
-            items[o].push_back(t);
-          }
-        continue;
-      }
       const StreamGeom g = o == 0   ? make_stream_geom<kBatchRows[0]>(s.H, s.W)
                            : o == 1 ? make_stream_geom<kBatchRows[1]>(s.H, s.W)
                            : o == 2 ? make_stream_geom<kBatchRows[2]>(s.H, s.W)
@@ -330,19 +298,35 @@ int32_t fk_batch_create(const fk_sim* sims, int32_t n, fk_batch** out) {
         }
     }
   }
-  // the two-step options exist only when every simulation fits them
+  // 32 rows: 4 steps per launch for batches of few tiles, else 2
+  LeastRounds by32, least;
+  by32.offer(kBatch32x4, Block32x4{}, n32x4);
+  by32.offer(kBatch32x2, Block32x2{}, n32x2);
+  b->block[4] = by32.best;
+  b->block[5] = kBatch48x3;
+  least.offer(4, Block32x4{}, n32x4);
+  least.offer(4, Block32x2{}, n32x2);
+  least.offer(5, Block48x3{}, n48x3);
+  b->untuned = b->opt = least.best;
   for (int o = 0; o < kNumRowOpts; ++o) {
+    b->offered[o] = !kBatchTwo[o] || fit[o - 4];
     if (!kBatchTwo[o]) continue;
-    bool all_fit = true;
-    for (int i = 0; i < n; ++i)
-      all_fit = all_fit && (kBatchRows[o] == 8 ? stream_t_fits<8>(sims[i].H, sims[i].W)
-                                               : stream_t_fits<16>(sims[i].H, sims[i].W));
-    if (!all_fit) items[o].clear();
+    for (int i = 0; i < n; ++i) {
+      const int H = sims[i].H, W = sims[i].W;
+      switch (b->block[o]) {
+        case kBatch32x4: append_block_items<Block32x4>(i, H, W, tiles[o]); break;
+        case kBatch32x2: append_block_items<Block32x2>(i, H, W, tiles[o]); break;
+        default: append_block_items<Block48x3>(i, H, W, tiles[o]); break;
+      }
+    }
+    tiles[o] = block_work_list(tiles[o]);
   }
   size_t sz_it[kNumRowOpts], sz_items = 0;
   for (int o = 0; o < kNumRowOpts; ++o) {
-    b->n_items_opt[o] = (int)items[o].size();
-    sz_it[o] = ((sizeof(TileItem) * items[o].size() + 255) / 256) * 256;
+    b->n_items_opt[o] = (int)(kBatchTwo[o] ? tiles[o].size() : items[o].size());
+    const size_t bytes =
+        kBatchTwo[o] ? sizeof(BlockItem) * tiles[o].size() : sizeof(TileItem) * items[o].size();
+    sz_it[o] = ((bytes + 255) / 256) * 256;
     sz_items += sz_it[o];
   }
   const size_t sz_sims = ((sizeof(SimDesc) * n + 255) / 256) * 256;
@@ -358,7 +342,7 @@ int32_t fk_batch_create(const fk_sim* sims, int32_t n, fk_batch** out) {
   {
     size_t at = sz_sims;
     for (int o = 0; o < kNumRowOpts; ++o) {
-      b->d_items[o] = (TileItem*)(b->dev + at);
+      b->d_items[o] = b->dev + at;
       at += sz_it[o];
     }
   }
@@ -391,9 +375,10 @@ int32_t fk_batch_create(const fk_sim* sims, int32_t n, fk_batch** out) {
   }
   e = hipMemcpy(b->d_sims, desc.data(), sizeof(SimDesc) * n, hipMemcpyHostToDevice);
   for (int o = 0; o < kNumRowOpts && e == hipSuccess; ++o)
-    if (!items[o].empty())
-      e = hipMemcpy(b->d_items[o], items[o].data(), sizeof(TileItem) * items[o].size(),
-                    hipMemcpyHostToDevice);
+    e = kBatchTwo[o] ? hipMemcpy(b->d_items[o], tiles[o].data(),
+                                 sizeof(BlockItem) * tiles[o].size(), hipMemcpyHostToDevice)
+                     : hipMemcpy(b->d_items[o], items[o].data(),
+                                 sizeof(TileItem) * items[o].size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking);
   if (e != hipSuccess) {
     batch_free(b);
@@ -421,37 +406,43 @@ static hipError_t batch_masks(fk_batch* b, int n_rel, hipStream_t s) {
   return hipGetLastError();
 }
 
-// One launch of option o at step rel of the current mask window (its masks
-// computed): two steps when o is a two-step option and `two` is set, else
-// one. Reads pool[parity], writes pool[parity ^ 1].
-static hipError_t batch_launch(fk_batch* b, int o, bool two, int rel, int parity,
+// One launch of option o, n_lev steps from step rel of the current mask window
+// on (its masks computed). Reads pool[parity], writes pool[parity ^ 1].
+static hipError_t batch_launch(fk_batch* b, int o, int n_lev, int rel, int parity,
                                hipStream_t s) {
-  if (!two) o = one_step_opt(o);
-  const int n_items = b->n_items_opt[o];
+  const int n_items = b->n_items_opt[o], n = b->n_sims;
   const int blocks = (n_items + 3) / 4;
-  const TileItem* it = b->d_items[o];
-  const uint32_t* m1 = b->d_mask + (size_t)rel * b->n_sims;
+  const TileItem* it = (const TileItem*)b->d_items[o];
+  const BlockItem* bi = (const BlockItem*)b->d_items[o];
+  const uint32_t* m = b->d_mask + (size_t)rel * n;
+  auto block = [&](auto cfg) {
+    typedef decltype(cfg) Cfg;
+    k_batch_block<Cfg><<<n_items, Cfg::waves * 64, 0, s>>>(b->d_sims, bi, n, m, n_lev, parity);
+  };
+  switch (b->block[o]) {
+    case kBatch32x4: block(Block32x4{}); return hipGetLastError();
+    case kBatch32x2: block(Block32x2{}); return hipGetLastError();
+    case kBatch48x3: block(Block48x3{}); return hipGetLastError();
+    default: break;
+  }
   switch (o) {
-    case 0: k_batch_step<kBatchRows[0]><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m1, parity); break;
-    case 1: k_batch_step<kBatchRows[1]><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m1, parity); break;
-    case 2: k_batch_step<kBatchRows[2]><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m1, parity); break;
-    case 3: k_batch_step<kBatchRows[3]><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m1, parity); break;
-    case 4: k_batch_step_t<8><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m1, m1 + b->n_sims, parity); break;
-    default: k_batch_step_t<16><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m1, m1 + b->n_sims, parity); break;
+    case 0: k_batch_step<kBatchRows[0]><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m, parity); break;
+    case 1: k_batch_step<kBatchRows[1]><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m, parity); break;
+    case 2: k_batch_step<kBatchRows[2]><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m, parity); break;
+    default: k_batch_step<kBatchRows[3]><<<blocks, 256, 0, s>>>(b->d_sims, it, n_items, m, parity); break;
   }
   return hipGetLastError();
 }
 
 // n (<= kGraphSteps) steps of option o from the counter on: their masks, the
-// step launches (two steps each where possible) and the counter bump. Starts
-// at pool[*parity] and leaves the pool of the result in *parity.
+// step launches and the counter bump. Starts at pool[*parity] and leaves the
+// pool of the result in *parity.
 static hipError_t batch_chunk(fk_batch* b, int o, int n, int* parity, hipStream_t s) {
   hipError_t e = batch_masks(b, n, s);
-  for (int r = 0; r < n && e == hipSuccess;) {
-    const bool two = kBatchTwo[o] && n - r >= 2;
-    e = batch_launch(b, o, two, r, *parity, s);
+  const int per = batch_steps(b->block[o]);
+  for (int r = 0; r < n && e == hipSuccess; r += per) {
+    e = batch_launch(b, o, std::min(per, n - r), r, *parity, s);
     *parity ^= 1;
-    r += two ? 2 : 1;
   }
   if (e == hipSuccess) {
     k_batch_bump<<<1, 64, 0, s>>>(b->d_step, n);
@@ -460,17 +451,19 @@ static hipError_t batch_chunk(fk_batch* b, int o, int n, int* parity, hipStream_
   return e;
 }
 
-// Launches of one chunk of kGraphSteps steps of option o, and so the parity
-// change a recorded graph makes.
-static int chunk_launches(int o) { return kBatchTwo[o] ? kGraphSteps / 2 : kGraphSteps; }
+// Steps of a recorded graph of option o: whole launches.
+static int graph_steps(const fk_batch* b, int o) {
+  const int per = batch_steps(b->block[o]);
+  return kGraphSteps / per * per;
+}
 
-// Records a chunk of kGraphSteps steps starting at `parity`.
+// Records a chunk of graph_steps steps starting at `parity`.
 static hipError_t batch_build_graph(fk_batch* b, int parity) {
   hipGraph_t g = nullptr;
   hipError_t e = hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return e;
   int p = parity;
-  e = batch_chunk(b, b->opt, kGraphSteps, &p, b->cap);
+  e = batch_chunk(b, b->opt, graph_steps(b, b->opt), &p, b->cap);
   const hipError_t e2 = hipStreamEndCapture(b->cap, &g);
   if (e == hipSuccess) e = e2;
   if (e == hipSuccess) e = hipGraphInstantiate(&b->exec[parity], g, nullptr, nullptr, 0);
@@ -494,24 +487,29 @@ int32_t fk_batch_autotune(fk_batch* b, int32_t n_steps, void* stream, float* tim
   if (e == hipSuccess) e = hipEventCreate(&e1);
   float ms[kNumRowOpts];
   for (int o = 0; o < kNumRowOpts; ++o) ms[o] = -1.0f;
+  const int untuned = b->untuned;
   for (int o = 0; o < kNumRowOpts && e == hipSuccess; ++o) {
-    if (b->n_items_opt[o] == 0) continue;  // a two-step option some simulation does not fit
+    if (!b->offered[o] && o != untuned) continue;
     int parity = 0;
     k_batch_set<<<1, 64, 0, s>>>(b->d_step, 0);
-    e = batch_chunk(b, o, 2, &parity, s);  // warm-up
+    e = batch_chunk(b, o, 4, &parity, s);  // warm-up
     if (e == hipSuccess) e = hipEventRecord(e0, s);
-    for (int k = 0; k < n_steps && e == hipSuccess; k += kGraphSteps)
-      e = batch_chunk(b, o, std::min(kGraphSteps, n_steps - k), &parity, s);
+    const int chunk = graph_steps(b, o);
+    for (int k = 0; k < n_steps && e == hipSuccess; k += chunk)
+      e = batch_chunk(b, o, std::min(chunk, n_steps - k), &parity, s);
     if (e == hipSuccess) e = hipEventRecord(e1, s);
     if (e == hipSuccess) e = hipEventSynchronize(e1);
     if (e == hipSuccess) e = hipEventElapsedTime(&ms[o], e0, e1);
   }
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
-  int best = kDefaultRowOpt;
+  int best = untuned, best_offered = 0;
   if (e == hipSuccess)
-    for (int o = 0; o < kNumRowOpts; ++o)
-      if (ms[o] >= 0.0f && ms[o] < ms[best]) best = o;
+    for (int o = 0; o < kNumRowOpts; ++o) {
+      if (ms[o] < 0.0f) continue;
+      if (ms[o] < ms[best]) best = o;
+      if (b->offered[o] && ms[o] < ms[best_offered]) best_offered = o;
+    }
   b->opt = best;
   // graphs recorded for another work list are stale
   for (auto& x : b->exec)
@@ -522,8 +520,9 @@ int32_t fk_batch_autotune(fk_batch* b, int32_t n_steps, void* stream, float* tim
   if (e != hipSuccess) return set_error(FK_ERR_HIP, "batch autotune failed: %s",
                                         hipGetErrorString(e));
   if (times_ms)
-    for (int o = 0; o < kNumRowOpts; ++o) times_ms[o] = ms[o];
-  if (best_rows) *best_rows = kBatchRows[b->opt] | (kBatchTwo[b->opt] ? FK_BATCH_TWO_STEP : 0);
+    for (int o = 0; o < kNumRowOpts; ++o) times_ms[o] = b->offered[o] ? ms[o] : -1.0f;
+  if (best_rows)
+    *best_rows = kBatchRows[best_offered] | (kBatchTwo[best_offered] ? FK_BATCH_TWO_STEP : 0);
   return FK_OK;
 }
 
@@ -538,7 +537,7 @@ int32_t fk_batch_set_rows(fk_batch* b, int32_t rows) {
     return set_error(FK_ERR_ARG,
                      "band height must be 2, 4, 8 or 16, or 8 or 16 with FK_BATCH_TWO_STEP, "
                      "got %d", rows);
-  if (b->n_items_opt[o] == 0)
+  if (!b->offered[o])
     return set_error(FK_ERR_UNSUPPORTED,
                      "two steps per launch need every simulation of at least 2R + 16 rows "
                      "and 56..96 or >= 104 columns");
@@ -567,11 +566,13 @@ int32_t fk_batch_run(fk_batch* b, int64_t n_steps, int32_t use_graph, void* stre
   int64_t k = 0;
   int parity = 0;
   if (use_graph) {
-    while (n_steps - k >= kGraphSteps) {
+    const int chunk = graph_steps(b, b->opt);
+    const int flips = chunk / batch_steps(b->block[b->opt]) & 1;
+    while (n_steps - k >= chunk) {
       if (!b->exec[parity]) HIP_CHECK(batch_build_graph(b, parity));
       HIP_CHECK(hipGraphLaunch(b->exec[parity], s));
-      k += kGraphSteps;
-      parity ^= chunk_launches(b->opt) & 1;
+      k += chunk;
+      parity ^= flips;
     }
   }
   // the remainder (or everything without graphs): direct launches

@@ -428,13 +428,12 @@ __device__ __forceinline__ int block_sides(const BlockSpan& c, int C, int W) {
   return (c.o < 0 ? 1 : 0) | (c.o + C > W ? 2 : 0);
 }
 
-// block_tile of the tile in band `band` and strip `strip`.
+// block_tile over the spans of one tile, by the sides it reaches over.
 template <class Cfg, bool HEUN, class SV>
-__device__ __forceinline__ void block_tile_at(const Coef& c, const BlockIO& io, int H, int W,
-                                              const SV& sv, int n_lev, float dt, float inv_dx2,
-                                              const BlockAxis& ra, const BlockAxis& ca, int band,
-                                              int strip, float* lds) {
-  const BlockSpan r = block_span(ra, band), s = block_span(ca, strip);
+__device__ __forceinline__ void block_tile_any(const Coef& c, const BlockIO& io, int H, int W,
+                                               const SV& sv, int n_lev, float dt, float inv_dx2,
+                                               const BlockSpan& r, const BlockSpan& s,
+                                               float* lds) {
   switch (block_sides(s, Cfg::C, W)) {
     case 0: block_tile<Cfg, 0, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
     case 1: block_tile<Cfg, 1, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, r, s, lds); break;
@@ -490,7 +489,38 @@ k_block(Coef c, BlockIO io, int H, int W, BlockStim st, int n_lev, float dt, flo
   __shared__ float lds[Cfg::lds_floats];
   const BlockPlace at = block_place(blockIdx.x, ord, ra, ca);
   const BlockStimArgs sv{st};
-  block_tile_at<Cfg, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, ra, ca, at.band, at.strip, lds);
+  block_tile_any<Cfg, HEUN>(c, io, H, W, sv, n_lev, dt, inv_dx2, block_span(ra, at.band),
+                            block_span(ca, at.strip), lds);
+}
+
+// The tilings of Euler steps, and the choice among those offered. A launch takes
+// the GPU's 256 CUs in rounds of tiles, and each tiling's time per step is close
+// to a + b ceil(tiles / 256) us, measured from 64^2 to 2500^2: few steps per
+// launch cost the launch (a), many cost the columns and rows that only feed the
+// stencil (b). The least is taken. Of the tilings tried (1 and 2 columns per lane,
+// 2 to 6 rows per wave, 4 to 16 waves, 2 to 4 steps) these four were the fastest
+// somewhere.
+typedef BlockCfg<2, 16, 4> Block32x4;
+typedef BlockCfg<4, 8, 2> Block32x2;
+typedef BlockCfg<4, 12, 3> Block48x3;
+typedef BlockCfg<4, 16, 3> Block64x3;
+
+struct LeastRounds {
+  int best = -1;
+  double least = 0.0;
+  void offer(int id, int64_t tiles, double a, double b) {
+    const double us = a + b * (double)((tiles + 255) / 256);
+    if (best < 0 || us < least) best = id, least = us;
+  }
+  void offer(int id, Block32x4, int64_t tiles) { offer(id, tiles, 1.0, 1.05); }
+  void offer(int id, Block48x3, int64_t tiles) { offer(id, tiles, 1.7, 1.25); }
+  void offer(int id, Block64x3, int64_t tiles) { offer(id, tiles, 1.4, 2.05); }
+  void offer(int id, Block32x2, int64_t tiles) { offer(id, tiles, 2.2, 1.0); }
+};
+
+template <class Cfg>
+inline int64_t block_tiles(int H, int W) {
+  return (int64_t)Cfg::row_axis(H).n * Cfg::col_axis(W).n;
 }
 
 }  // namespace fk

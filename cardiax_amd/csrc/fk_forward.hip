@@ -339,14 +339,6 @@ static int pc_base(int v) {
                                                                                  : kStream16;
 }
 
-// The block variants' tiles: rows per wave, waves, steps.
-// Of the tilings tried (1 and 2 columns per lane, 2 to 6 rows per wave, 6 to 16
-// waves, 2 to 4 steps) these were the fastest somewhere; us per step below.
-typedef BlockCfg<4, 8, 2> Block32x2;
-typedef BlockCfg<4, 12, 3> Block48x3;
-typedef BlockCfg<4, 16, 3> Block64x3;
-typedef BlockCfg<2, 16, 4> Block32x4;
-
 static bool is_block(int v) { return v >= kBlock32x2 && v <= kBlock32x4; }
 
 static int block_steps(int v) { return v == kBlock32x2 ? 2 : v == kBlock32x4 ? 4 : 3; }
@@ -421,26 +413,10 @@ static int default_variant(int H, int W) {
 }
 static int resolve_variant(int v) { return v == kAuto ? (int)kStream2 : v; }
 
-// The tiling with the least a + b ceil(tiles / 256) of those offered.
-struct LeastRounds {
-  int best = -1;
-  double least = 0.0;
-  template <class Cfg>
-  void offer(int id, Cfg, int H, int W, double a, double b) {
-    constexpr int64_t kCUs = 256;
-    const int64_t tiles = (int64_t)Cfg::row_axis(H).n * Cfg::col_axis(W).n;
-    const double us = a + b * (double)((tiles + kCUs - 1) / kCUs);
-    if (best < 0 || us < least) best = id, least = us;
-  }
-};
-
 // The variant an automatic solve of several steps runs when the shape was not
 // tuned: block tiles, which equal the streaming kernels of default_variant bit
-// for bit. A launch takes the GPU's 256 CUs in rounds of tiles, and each tiling's
-// time per step is close to a + b ceil(tiles / 256), measured from 64^2 to
-// 2500^2: few steps per launch cost the launch (a), many cost the columns and
-// rows that only feed the stencil (b). The least of the four is taken. Against
-// the best streaming kernel, us per step: 128^2 2.05 and 3.07 (32 rows, 4
+// for bit, in the tiling that LeastRounds finds. Against the best streaming
+// kernel, us per step: 128^2 2.05 and 3.07 (32 rows, 4
 // steps), 500^2 3.0 and 3.9 (48 rows, 3), 700 x 600 3.5 and 5.4 (64 rows, 3),
 // 1024^2 6.2 and 7.2, 1200^2 7.3 and 10.0, 2048^2 15.9 and 17.2, 4096^2 70 and
 // 78 (32 rows, 2).
@@ -448,10 +424,10 @@ static int auto_variant(int H, int W) {
   const int d = default_variant(H, W);
   if (d == kTile16) return d;  // narrow grids above 8 M cells: another rounding
   LeastRounds r;
-  r.offer(kBlock32x4, Block32x4{}, H, W, 1.0, 1.05);
-  r.offer(kBlock48x3, Block48x3{}, H, W, 1.7, 1.25);
-  r.offer(kBlock64x3, Block64x3{}, H, W, 1.4, 2.05);
-  r.offer(kBlock32x2, Block32x2{}, H, W, 2.2, 1.0);
+  r.offer(kBlock32x4, Block32x4{}, block_tiles<Block32x4>(H, W));
+  r.offer(kBlock48x3, Block48x3{}, block_tiles<Block48x3>(H, W));
+  r.offer(kBlock64x3, Block64x3{}, block_tiles<Block64x3>(H, W));
+  r.offer(kBlock32x2, Block32x2{}, block_tiles<Block32x2>(H, W));
   return r.best;
 }
 
@@ -613,10 +589,10 @@ enum HeunTiling { kHeun32x2, kHeun48x2, kHeun64x1, kHeun40x1 };
 
 static int heun_tiling(int H, int W) {
   LeastRounds r;
-  r.offer(kHeun32x2, Heun32x2{}, H, W, 2.0, 2.9);
-  r.offer(kHeun48x2, Heun48x2{}, H, W, 1.8, 4.2);
-  r.offer(kHeun64x1, Heun64x1{}, H, W, 2.2, 7.45);
-  r.offer(kHeun40x1, Heun40x1{}, H, W, 4.3, 3.55);
+  r.offer(kHeun32x2, block_tiles<Heun32x2>(H, W), 2.0, 2.9);
+  r.offer(kHeun48x2, block_tiles<Heun48x2>(H, W), 1.8, 4.2);
+  r.offer(kHeun64x1, block_tiles<Heun64x1>(H, W), 2.2, 7.45);
+  r.offer(kHeun40x1, block_tiles<Heun40x1>(H, W), 4.3, 3.55);
   return r.best;
 }
 

@@ -315,10 +315,10 @@ int32_t fk_adjoint_tau_grads(void* work, int32_t H, int32_t W, float* g_tau, voi
 #define FK_BATCH_MAX_STIMULI 4
 
 /* Work-list options of a batch: bands of 2, 4, 8 or 16 rows advanced one step
- * per launch, and bands of 8 or 16 rows advanced two steps per launch (those
- * two only when every simulation has >= 2R + 16 rows and 56..96 or >= 104
- * columns). A band height or'ed with FK_BATCH_TWO_STEP names a two-step
- * option. */
+ * per launch, and, named by 8 and 16 or'ed with FK_BATCH_TWO_STEP, block tiles
+ * of 32 rows advanced 4 steps per launch (2 for batches of many tiles) and of
+ * 48 rows advanced 3. Those two are offered only when every simulation has >=
+ * 2R + 16 rows, R = 8 or 16, and 56..96 or >= 104 columns. */
 #define FK_BATCH_N_OPTIONS 6
 #define FK_BATCH_TWO_STEP 256
 
@@ -347,20 +347,22 @@ int32_t fk_batch_create(const fk_sim* sims, int32_t n, fk_batch** out);
 
 /* Advances every simulation by n_steps Euler steps; results land in each
  * fk_sim's v, w, u and each simulation's time advances by n_steps. Each
- * launch advances the whole batch one step (or two, with a two-step option);
+ * launch advances the whole batch one step (or up to four, with block tiles);
  * the stimulus activity of up to 32 steps comes from one small kernel.
- * use_graph != 0 replays a recorded hipGraph of 32 steps (one graph launch
- * per 32 steps for the whole batch), otherwise direct launches. */
+ * use_graph != 0 replays a recorded hipGraph of 32 steps (30 with 3 steps per
+ * launch; one graph launch for the whole batch), otherwise direct launches. */
 int32_t fk_batch_run(fk_batch* b, int64_t n_steps, int32_t use_graph, void* stream);
 
 /* Autotuner of the batch: times n_steps (1..10000) batched steps with each
  * available work-list option on `stream` (synchronising it) and keeps the
- * fastest for later runs (8 rows, one step per launch, until tuned).
+ * fastest for later runs. Until tuned, a batch of any sizes runs block tiles of
+ * 32 or 48 rows, by their number; the tuner times those too, and keeps them if
+ * they are the fastest, where the size rule does not offer them.
  * Overwrites only the batch's internal ping-pong pools, never a simulation's
  * state. times_ms (FK_BATCH_N_OPTIONS floats in the order 2, 4, 8, 16 rows,
- * then 8, 16 rows with two steps; -1 for an unavailable option; may be NULL)
- * and best_rows (may be NULL) receive the timings and the chosen band height
- * (or'ed with FK_BATCH_TWO_STEP for a two-step option). */
+ * then the two of FK_BATCH_TWO_STEP; -1 for one that is not offered; may be
+ * NULL) and best_rows (may be NULL) receive the timings and the fastest option
+ * offered. */
 int32_t fk_batch_autotune(fk_batch* b, int32_t n_steps, void* stream, float* times_ms,
                           int32_t* best_rows);
 
