@@ -11,8 +11,9 @@
 // steps; for each segment, in reverse, the states are recomputed from its
 // checkpoint and the steps are reversed one by one, frame cotangents entering
 // lam_u at the frame steps. Every launch covers all problems through a work
-// list (one wave per tile), and the tiles run the same device code as the
-// per-grid kernels: the results are bitwise those of the per-grid path.
+// list (forward steps a block per block tile, two to four steps; reverse steps a
+// wave per tile), and the tiles run the same device code as the per-grid
+// kernels: the results are bitwise those of the per-grid path.
 //
 // Reference: there is no counterpart in the reference, whose inverse problem
 // is learnt by a network (deepx); the forward step follows
@@ -34,10 +35,9 @@
 
 namespace fk {
 
-constexpr int kRollRows = 4;  // band rows of the forward tiles
-// band rows of the reverse tiles: 3.84 M cells 60 us with 4, 68 with 2, 67 with
-// 8; the bits do not depend on it
-constexpr int kRollRev = 4;
+// Block tiling of the forward steps.
+enum RollBlock { kRoll32x4, kRoll48x3, kRoll32x2 };
+constexpr int roll_steps(int blk) { return blk == kRoll32x4 ? 4 : blk == kRoll48x3 ? 3 : 2; }
 
 struct RollDesc {
   Coef c;
@@ -85,23 +85,18 @@ __device__ __forceinline__ const float* roll_state(const RollDesc& S, int seg, i
   return gfield(S.traj) + ((size_t)(k - 1) * 3 + f) * S.cells;
 }
 
-// One Euler step of every tile: x_{c+k} -> trajectory slot k. masks: this
-// step's stimulus activity, one word per problem.
-template <int R>
-__global__ void __launch_bounds__(256)
-k_roll_step(const RollDesc* __restrict__ sims, const RollTile* __restrict__ items, int n_items,
-            const uint32_t* __restrict__ masks, int seg, int k) {
-  const int it = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x >> 6));
-  if (it >= n_items) return;
-  RollTile item = items[it];
-  if (uni(item.sim) < 0) return;  // padding of the XCD order
-  item.sim = uni(item.sim);
-  item.cs = uni(item.cs);
-  item.rs = uni(item.rs);
-  item.flags = uni(item.flags);
-  const RollDesc& S = sims[item.sim];
-  const uint32_t mask = __builtin_amdgcn_readfirstlane(masks[item.sim]);
-  const BatchStimView sv{S.stim, uni(S.n_stim), mask};
+// n_lev Euler steps of every block tile: x_{c+k} -> trajectory slots k ..
+// k + n_lev - 1. masks: the steps' stimulus activity, n words each.
+template <class Cfg>
+__global__ void __launch_bounds__(Cfg::waves * 64)
+k_roll_block(const RollDesc* __restrict__ sims, const BlockItem* __restrict__ items, int n,
+             const uint32_t* __restrict__ masks, int seg, int k, int n_lev) {
+  __shared__ float lds[Cfg::lds_floats];
+  const BlockItem& it = items[blockIdx.x];
+  const int sim = uni(it.sim);
+  if (sim < 0) return;  // padding of the XCD order: the whole block leaves
+  const RollDesc& S = sims[sim];
+  const BatchBlockStim sv{S.stim, pack_masks(masks + sim, n, n_lev)};
   Coef c = S.c;
   c.V_c = uni(c.V_c); c.V_v = uni(c.V_v); c.V_csi = uni(c.V_csi); c.kk = uni(c.kk);
   c.kk_off = uni(c.kk_off);
@@ -109,32 +104,15 @@ k_roll_step(const RollDesc* __restrict__ sims, const RollTile* __restrict__ item
   c.inv_twp = uni(c.inv_twp); c.inv_twm = uni(c.inv_twm); c.inv_td = uni(c.inv_td);
   c.inv_t0 = uni(c.inv_t0); c.inv_tr = uni(c.inv_tr); c.inv_tsi = uni(c.inv_tsi);
   c.inv_cm = uni(c.inv_cm);
-  const float* Dp = uni(S.D);
-  const float* i0 = uni(roll_state(S, seg, k, 0));
-  const float* i1 = uni(roll_state(S, seg, k, 1));
-  const float* i2 = uni(roll_state(S, seg, k, 2));
   const size_t cells = S.cells;
-  float* o0 = uni(S.traj + ((size_t)k * 3 + 0) * cells);
-  float* o1 = uni(S.traj + ((size_t)k * 3 + 1) * cells);
-  float* o2 = uni(S.traj + ((size_t)k * 3 + 2) * cells);
-  const int H = uni(S.H), W = uni(S.W);
-  const float dt = uni(S.dt), inv_dx2 = uni(S.inv_dx2);
-  const int sel = item.flags | (mask ? 4 : 0);
-#define FK_RS(X, Y, ST)                                                                   \
-  stream_tile<R, true, X, Y, ST, BatchStimView, false, true>(c, Dp, nullptr, i0, i1, i2, H, \
-                                                                W, sv, dt, inv_dx2, o0, o1,   \
-                                                                o2, item.rs, item.cs)
-  switch (sel) {
-    case 0: FK_RS(false, false, false); break;
-    case 1: FK_RS(true, false, false); break;
-    case 2: FK_RS(false, true, false); break;
-    case 3: FK_RS(true, true, false); break;
-    case 4: FK_RS(false, false, true); break;
-    case 5: FK_RS(true, false, true); break;
-    case 6: FK_RS(false, true, true); break;
-    default: FK_RS(true, true, true); break;
-  }
-#undef FK_RS
+  float* out = uni(S.traj + (size_t)k * 3 * cells);
+  const BlockIO io{uni(S.D), uni(roll_state(S, seg, k, 0)), uni(roll_state(S, seg, k, 1)),
+                   uni(roll_state(S, seg, k, 2)), out, out + cells, out + 2 * cells, 3 * cells,
+                   true};
+  const BlockSpan r{uni(it.r.o), uni(it.r.a), uni(it.r.b)};
+  const BlockSpan q{uni(it.c.o), uni(it.c.a), uni(it.c.b)};
+  block_tile_any<Cfg, false>(c, io, uni(S.H), uni(S.W), sv, n_lev, uni(S.dt), uni(S.inv_dx2), r,
+                             q, lds);
 }
 
 // After forward segment `seg` (steps c .. c + len - 1): the frames it holds
@@ -222,10 +200,12 @@ struct fk_rollout_batch {
   char* dev = nullptr;
   size_t dev_bytes = 0;
   RollDesc* d_sims = nullptr;
-  RollTile* d_tiles = nullptr;
-  RollTile* d_rev = nullptr;
+  BlockItem* d_tiles = nullptr;  // forward
+  RollTile* d_rev = nullptr;     // reverse
   uint32_t* d_masks = nullptr;  // n_steps x n
   int n_tiles = 0, n_rev = 0;
+  int block = kRoll32x4;  // RollBlock of the forward steps
+  int rev_rows = 4;       // band rows of the reverse tiles
   size_t max_cells = 0;
   int traj_seg = -1;  // segment whose states the trajectory buffer holds (-1: none)
 };
@@ -280,38 +260,51 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   b->S = std::min(checkpoint_every, n_steps);
   b->n_seg = (n_steps + b->S - 1) / b->S;
   b->specs.assign(specs, specs + n);
-  // work lists: runs of vertically adjacent tiles (which share halo rows),
-  // placed whole on one XCD each
+  int64_t n32x4 = 0, n48x3 = 0, n32x2 = 0, n_rev4 = 0;
+  for (int i = 0; i < n; ++i) {
+    const int H = specs[i].H, W = specs[i].W;
+    n32x4 += block_tiles<Block32x4>(H, W);
+    n48x3 += block_tiles<Block48x3>(H, W);
+    n32x2 += block_tiles<Block32x2>(H, W);
+    n_rev4 += (int64_t)adj_strips(W) * ((H + 3) / 4);
+  }
+  LeastRounds least;
+  least.offer(kRoll32x4, Block32x4{}, n32x4);
+  least.offer(kRoll48x3, Block48x3{}, n48x3);
+  least.offer(kRoll32x2, Block32x2{}, n32x2);
+  b->block = least.best;
+  // Reverse bands of 2 rows while the waves are few and a wave's rows, one after
+  // the other, set the time (2 problems 64 to 200 wide, 100 steps: 1.07 ms, 1.33 with
+  // 4; 10 of 128 to 480: 3.33 and 3.40); 4 rows for more (12 of 128 to 512: 4.63 and
+  // 4.69; one reverse step of 3.84 M cells 60 and 68 us, 67 with 8). The bits do not
+  // depend on it.
+  b->rev_rows = n_rev4 <= 5000 ? 2 : 4;
+  const int rows = b->rev_rows;
+  // work lists over the dies: neighbouring forward tiles, and runs of vertically
+  // adjacent reverse tiles (which share halo rows), whole on one die each
   constexpr int kRunTiles = 16;
-  std::vector<std::vector<RollTile>> tile_runs, rev_runs;
+  std::vector<BlockItem> blocks;
+  std::vector<std::vector<RollTile>> rev_runs;
   for (int i = 0; i < n; ++i) {
     const fk_rollout_spec& s = specs[i];
-    const StreamGeom g = make_stream_geom<kRollRows>(s.H, s.W);
-    for (int strip = 0; strip < g.n_strips; ++strip)
-      for (int band = 0; band < g.n_bands; ++band) {
-        RollTile t;
-        t.sim = i;
-        t.cs = std::min(kStripOut * strip, g.cs_last);
-        t.rs = std::min(kRollRows * band, g.rs_last);
-        const bool xg = edge_band(t.rs, kRollRows, s.H, s.W);
-        const bool yg = t.cs < 3 || t.cs + kStripOut + 3 > s.W;
-        t.flags = (xg ? 1 : 0) | (yg ? 2 : 0);
-        if (band % kRunTiles == 0) tile_runs.emplace_back();
-        tile_runs.back().push_back(t);
-      }
+    switch (b->block) {
+      case kRoll32x4: append_block_items<Block32x4>(i, s.H, s.W, blocks); break;
+      case kRoll48x3: append_block_items<Block48x3>(i, s.H, s.W, blocks); break;
+      default: append_block_items<Block32x2>(i, s.H, s.W, blocks); break;
+    }
     for (int strip = 0; strip < adj_strips(s.W); ++strip)
-      for (int band = 0; band < (s.H + kRollRev - 1) / kRollRev; ++band) {
+      for (int band = 0; band < (s.H + rows - 1) / rows; ++band) {
         RollTile t;
         t.sim = i;
         t.cs = kRevOut * strip;
-        t.rs = kRollRev * band;
-        t.flags = (adj_edge_band(t.rs, kRollRev, s.H) ? 1 : 0) |
+        t.rs = rows * band;
+        t.flags = (adj_edge_band(t.rs, rows, s.H) ? 1 : 0) |
                   (adj_edge_strip(t.cs, s.W) ? 2 : 0);
         if (band % kRunTiles == 0) rev_runs.emplace_back();
         rev_runs.back().push_back(t);
       }
   }
-  const std::vector<RollTile> tiles = xcd_order(tile_runs, 4, RollTile{-1, 0, 0, 0});
+  const std::vector<BlockItem> tiles = block_work_list(blocks);
   const std::vector<RollTile> rev = xcd_order(rev_runs, 4, RollTile{-1, 0, 0, 0});
   b->n_tiles = (int)tiles.size();
   b->n_rev = (int)rev.size();
@@ -331,7 +324,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
     return at;
   };
   const size_t o_sims = take(sizeof(RollDesc) * n);
-  const size_t o_tiles = take(sizeof(RollTile) * tiles.size());
+  const size_t o_tiles = take(sizeof(BlockItem) * tiles.size());
   const size_t o_rev = take(sizeof(RollTile) * rev.size());
   const size_t o_masks = take(sizeof(uint32_t) * masks.size());
   std::vector<size_t> o_ckpt(n), o_traj(n), o_lam(n);
@@ -353,7 +346,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
     return set_error(FK_ERR_HIP, "hipMalloc(%zu) failed: %s", o, hipGetErrorString(e));
   }
   b->d_sims = (RollDesc*)(b->dev + o_sims);
-  b->d_tiles = (RollTile*)(b->dev + o_tiles);
+  b->d_tiles = (BlockItem*)(b->dev + o_tiles);
   b->d_rev = (RollTile*)(b->dev + o_rev);
   b->d_masks = (uint32_t*)(b->dev + o_masks);
   std::vector<RollDesc> desc(n);
@@ -390,7 +383,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   }
   e = hipMemcpy(b->d_sims, desc.data(), sizeof(RollDesc) * n, hipMemcpyHostToDevice);
   if (e == hipSuccess)
-    e = hipMemcpy(b->d_tiles, tiles.data(), sizeof(RollTile) * tiles.size(),
+    e = hipMemcpy(b->d_tiles, tiles.data(), sizeof(BlockItem) * tiles.size(),
                   hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(b->d_rev, rev.data(), sizeof(RollTile) * rev.size(), hipMemcpyHostToDevice);
@@ -407,17 +400,32 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
 
 size_t fk_rollout_batch_device_bytes(const fk_rollout_batch* b) { return b ? b->dev_bytes : 0; }
 
+// Steps c .. c + n_steps - 1 of segment `seg` (c = seg S) into the trajectory.
+static void roll_steps_of(fk_rollout_batch* b, int seg, int n_steps, hipStream_t s) {
+  const int per = roll_steps(b->block);
+  auto go = [&](auto cfg, int k, int n_lev) {
+    typedef decltype(cfg) Cfg;
+    k_roll_block<Cfg><<<b->n_tiles, Cfg::waves * 64, 0, s>>>(
+        b->d_sims, b->d_tiles, b->n, b->d_masks + (size_t)(seg * b->S + k) * b->n, seg, k, n_lev);
+  };
+  for (int k = 0; k < n_steps; k += per) {
+    const int n_lev = std::min(per, n_steps - k);
+    switch (b->block) {
+      case kRoll32x4: go(Block32x4{}, k, n_lev); break;
+      case kRoll48x3: go(Block48x3{}, k, n_lev); break;
+      default: go(Block32x2{}, k, n_lev); break;
+    }
+  }
+}
+
 int32_t fk_rollout_batch_forward(fk_rollout_batch* b, void* stream) {
   ErrorScope es;
   if (b == nullptr) return set_error(FK_ERR_ARG, "null rollout batch");
   hipStream_t s = (hipStream_t)stream;
-  const int step_blocks = (b->n_tiles + 3) / 4;
   const dim3 cg = roll_cell_grid(b);
   for (int seg = 0; seg < b->n_seg; ++seg) {
     const int c = seg * b->S, len = std::min(b->S, b->n_steps - c);
-    for (int k = 0; k < len; ++k)
-      k_roll_step<kRollRows><<<step_blocks, 256, 0, s>>>(
-          b->d_sims, b->d_tiles, b->n_tiles, b->d_masks + (size_t)(c + k) * b->n, seg, k);
+    roll_steps_of(b, seg, len, s);
     k_roll_gather<<<cg, 256, 0, s>>>(b->d_sims, seg, c, len, b->fe,
                                      seg + 1 < b->n_seg ? 1 : 0);
   }
@@ -438,21 +446,22 @@ int32_t fk_rollout_batch_backward(fk_rollout_batch* b, float* g_tau, void* strea
   }
   const dim3 cg = roll_cell_grid(b);
   k_roll_zero<<<cg, 256, 0, s>>>(b->d_sims);
-  const int step_blocks = (b->n_tiles + 3) / 4, rev_blocks = (b->n_rev + 3) / 4;
+  const int rev_blocks = (b->n_rev + 3) / 4;
   for (int seg = b->n_seg - 1; seg >= 0; --seg) {
     const int c = seg * b->S, len = std::min(b->S, b->n_steps - c);
     // recompute x_{c+1} .. x_{c+len-1}, unless the forward's last segment is
     // still in place (the same states: same kernels from the same checkpoint)
-    if (seg != b->traj_seg)
-      for (int k = 0; k + 1 < len; ++k)
-        k_roll_step<kRollRows><<<step_blocks, 256, 0, s>>>(
-            b->d_sims, b->d_tiles, b->n_tiles, b->d_masks + (size_t)(c + k) * b->n, seg, k);
+    if (seg != b->traj_seg) roll_steps_of(b, seg, len - 1, s);
     b->traj_seg = seg;
     int cur = 0;
     for (int k = len - 1; k >= 0; --k) {
-      k_roll_rev<kRollRev><<<rev_blocks, 256, 0, s>>>(b->d_sims, b->d_rev, b->n_rev,
-                                                      b->d_masks + (size_t)(c + k) * b->n, seg, k,
-                                                      c + k + 1, b->fe, cur);
+      const uint32_t* m = b->d_masks + (size_t)(c + k) * b->n;
+      if (b->rev_rows == 2)
+        k_roll_rev<2><<<rev_blocks, 256, 0, s>>>(b->d_sims, b->d_rev, b->n_rev, m, seg, k,
+                                                 c + k + 1, b->fe, cur);
+      else
+        k_roll_rev<4><<<rev_blocks, 256, 0, s>>>(b->d_sims, b->d_rev, b->n_rev, m, seg, k,
+                                                 c + k + 1, b->fe, cur);
       cur ^= 1;
     }
     if (cur == 1) k_roll_lam_back<<<cg, 256, 0, s>>>(b->d_sims);
