@@ -3,10 +3,13 @@ frames with respect to the diffusivity map D and tau_d, tau_r, tau_si.
 
 ``rollout(...)`` runs cardiax/solve.py:92-100 on the GPU and returns the u
 fields after every ``frame_every`` steps. Its backward pass is the
-hand-written adjoint of the Euler step: the states are recomputed segment by
-segment from checkpoints kept every ~sqrt(N) steps (fk_forward_trajectory),
-so memory is O(sqrt(N)) states instead of N, and each segment is reversed by
-one fk_adjoint_segment call. Gates are fixed masks and the
+hand-written adjoint of the Euler step over the states of the forward pass.
+Those are kept when they take at most KEEP_BYTES, a small part of the GPU's
+memory (256 x 256 over 2000 steps: 1.6 GB, and 4.7 of 23.6 ms less than
+recomputing them). Longer or larger rollouts, and those that set
+``checkpoint_every``, recompute them segment by segment from checkpoints every
+~sqrt(N) steps (fk_forward_trajectory): O(sqrt(N)) states instead of N. Each
+segment is reversed by one fk_adjoint_segment call. Gates are fixed masks and the
 stimulus replacement routes no cotangent to j_ion -- what jax.grad computes
 through the reference's greater_equal and where.
 """
@@ -22,6 +25,9 @@ from . import _lib
 from ._device import on_device, require_gpu, stream_handle
 from .params import Params
 from .solve import State, _Stimuli, _scalar
+
+# Bytes of states that rollout keeps for its backward pass instead of recomputing them.
+KEEP_BYTES = 4 << 30
 
 # Params fields that carry gradients, in the order of the returned gradients.
 GRAD_FIELDS = ("tau_d", "tau_r", "tau_si")
@@ -48,6 +54,26 @@ class _Rollout(torch.autograd.Function):
         stim = _Stimuli(cfg["stimuli"], dev, (H, W))
         p = _lib.make_params(prm)
         s = stream_handle()
+        ctx.cfg = cfg
+        ctx.prm = prm
+        ctx.S = S
+        ctx.states = None
+        ctx.save_for_backward(D)
+        if cfg["grad"] and cfg["checkpoint_every"] is None and 12 * (n + 1) * H * W <= KEEP_BYTES:
+            try:
+                states = torch.empty((n + 1, 3, H, W), dtype=torch.float32, device=dev)
+            except torch.cuda.OutOfMemoryError:
+                states = None  # checkpoints take a fraction
+            if states is not None:
+                for f in range(3):
+                    states[0, f].copy_(st[f])
+                if n > 0:
+                    _lib.check(L.fk_forward_trajectory(
+                        ctypes.byref(p), D.data_ptr(), *(x.data_ptr() for x in states[0]), H, W,
+                        stim.pointer(), stim.n, float(t0), n, float(cfg["dt"]),
+                        float(cfg["dx"]), states[1:].data_ptr(), s))
+                ctx.S, ctx.states, ctx.ckpts = n, states, {0: st} if n else {}
+                return states[fe::fe, 2].clone(memory_format=torch.contiguous_format)
         frames = torch.empty((n // fe, H, W), dtype=torch.float32, device=dev)
         # Each checkpoint interval runs through fk_forward_trajectory, the call
         # the backward pass uses to recompute it, so the backward linearises
@@ -69,11 +95,7 @@ class _Rollout(torch.autograd.Function):
             cur, k = State(last[0].clone(), last[1].clone(), last[2].clone()), e
             if k < n:
                 ckpts[k] = cur
-        ctx.cfg = cfg
-        ctx.prm = prm
-        ctx.S = S
         ctx.ckpts = ckpts
-        ctx.save_for_backward(D)
         return frames
 
     @staticmethod
@@ -94,14 +116,17 @@ class _Rollout(torch.autograd.Function):
         lam = [torch.zeros((H, W), dtype=torch.float32, device=dev) for _ in range(3)]
         gD = torch.zeros((H, W), dtype=torch.float32, device=dev)
         # states x_c .. x_{e-1} of one segment, (v, w, u) planes per state
-        states = torch.empty((S, 3, H, W), dtype=torch.float32, device=dev)
+        states = ctx.states
+        if states is None:
+            states = torch.empty((S, 3, H, W), dtype=torch.float32, device=dev)
         for c in sorted(ctx.ckpts, reverse=True):
             e = min(n, c + S)
             x = ctx.ckpts[c]
-            states[0, 0].copy_(x.v)
-            states[0, 1].copy_(x.w)
-            states[0, 2].copy_(x.u)
-            if e - c > 1:  # recompute x_{c+1} .. x_{e-1}
+            if ctx.states is None:
+                states[0, 0].copy_(x.v)
+                states[0, 1].copy_(x.w)
+                states[0, 2].copy_(x.u)
+            if ctx.states is None and e - c > 1:  # recompute x_{c+1} .. x_{e-1}
                 _lib.check(L.fk_forward_trajectory(
                     ctypes.byref(p), D.data_ptr(), x.v.data_ptr(), x.w.data_ptr(),
                     x.u.data_ptr(), H, W, stim.pointer(), stim.n, float(t0 + c), e - c - 1,
@@ -152,7 +177,8 @@ def rollout(D: torch.Tensor, tau_d, tau_r, tau_si, state0, params, stimuli: Sequ
     cfg = {"params": params, "state0": state0, "stimuli": list(stimuli or []),
            "t0": _scalar(t0), "n_steps": int(n_steps), "frame_every": int(frame_every),
            "dt": float(dt), "dx": float(dx), "checkpoint_every": checkpoint_every,
-           "tau_host": host}
+           "tau_host": host,
+           "grad": torch.is_grad_enabled() and any(x.requires_grad for x in [D] + taus)}
     return _Rollout.apply(D, taus[0], taus[1], taus[2], cfg)
 
 
