@@ -250,6 +250,18 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
 #pragma unroll
     for (int k = 0; k < NW; ++k) LL[k] = LL[k] + at(a.inj, rs - E + k);
   }
+  // The tau sums of the band's row pairs (lane 63 adds to them at the end; every
+  // lane loads the same words, so that they arrive with the rest: read where they
+  // are added to, they ended the wave with a trip to memory).
+  double* gt = a.g_tau + 3 * ((size_t)(cs / kRevOut) * ((H + 1) / 2) + rs / 2);
+  double g0[3 * (R / 2)];
+#pragma unroll
+  for (int p = 0; p < R / 2; ++p)
+#pragma unroll
+    for (int f = 0; f < 3; ++f)
+      g0[3 * p + f] = !XG || rs + 2 * p < H
+                          ? ((const double __attribute__((address_space(1)))*)gt)[3 * p + f]
+                          : 0.0;
   float vv[R], ww[R], lvv[R], lww[R], gd[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) {
@@ -414,10 +426,11 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
       const float r0 = wave_sum63(ts[0] + t_d), r1 = wave_sum63(ts[1] + t_r),
                   r2 = wave_sum63(ts[2] + t_si);
       if (lane == 63 && (!XG || i - 1 < H)) {
-        double* g = a.g_tau + 3 * ((size_t)(cs / kRevOut) * ((H + 1) / 2) + (i - 1) / 2);
-        g[0] += (double)r0;
-        g[1] += (double)r1;
-        g[2] += (double)r2;
+        double __attribute__((address_space(1)))* g =
+            (double __attribute__((address_space(1)))*)gt + 3 * (k / 2);
+        g[0] = g0[3 * (k / 2)] + (double)r0;
+        g[1] = g0[3 * (k / 2) + 1] + (double)r1;
+        g[2] = g0[3 * (k / 2) + 2] + (double)r2;
       }
     }
   }
