@@ -140,7 +140,9 @@ __global__ void __launch_bounds__(Cfg::waves * 64)
 k_batch_block(const SimDesc* __restrict__ sims, const BlockItem* __restrict__ items, int n_sims,
               const uint32_t* __restrict__ masks, int n_lev, int parity) {
   __shared__ float lds[Cfg::lds_floats];
-  const BlockItem& it = items[blockIdx.x];
+  // each XCD's run forward and backward in turn, as in BlockOrder
+  const int x = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+  const BlockItem& it = items[kXcds * (parity ? (int)gridDim.x / kXcds - 1 - j : j) + x];
   const int sim = uni(it.sim);
   if (sim < 0) return;  // padding of the XCD order: the whole block leaves
   const SimDesc& S = sims[sim];
@@ -299,7 +301,7 @@ int32_t fk_batch_create(const fk_sim* sims, int32_t n, fk_batch** out) {
     }
   }
   // 32 rows: 4 steps per launch for batches of few tiles, else 2
-  LeastRounds by32, least;
+  LeastRounds by32((int64_t)b->total_cells), least((int64_t)b->total_cells);
   by32.offer(kBatch32x4, Block32x4{}, n32x4);
   by32.offer(kBatch32x2, Block32x2{}, n32x2);
   b->block[4] = by32.best;

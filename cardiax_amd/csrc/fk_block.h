@@ -450,27 +450,32 @@ __device__ __forceinline__ void block_tile_any(const Coef& c, const BlockIO& io,
 // order (bands of a strip, workgroup b tile b) every neighbour sits on another
 // XCD; times per step of the 32-row 2-step tiling, plain and so: 760^2 5.2 and
 // 4.2 us, 1200^2 9.4 and 7.3, 2048^2 22.4 and 15.9, 4096^2 90 and 69. Groups of
-// 4 or 16 bands are within 3% of 8, of 32 up to 15% slower.
+// 4 or 16 bands are within 3% of 8, of 32 up to 15% slower. A solve's launches
+// go through each run forward and backward in turn (`back`): where the fields
+// exceed the 256 MB cache, what a launch wrote last is still there for the next
+// (4096^2 69.9 and 66.5 us per step, 5000^2 104 and 100; no change below).
 constexpr int kBlockGroup = 8;
 
 struct BlockOrder {
   int per_xcd, extra;  // the first `extra` XCDs take one tile more
   float inv_group;     // 1 / tiles of a group of bands
+  int back;            // each XCD's run from its end
 };
 
 struct BlockPlace {
   int band, strip;
 };
 
-inline BlockOrder make_block_order(const BlockAxis& ra, const BlockAxis& ca) {
+inline BlockOrder make_block_order(const BlockAxis& ra, const BlockAxis& ca, bool back) {
   const int n = ra.n * ca.n;
-  return {n / kXcds, n % kXcds, 1.0f / (float)(kBlockGroup * ca.n)};
+  return {n / kXcds, n % kXcds, 1.0f / (float)(kBlockGroup * ca.n), back ? 1 : 0};
 }
 
 __device__ __forceinline__ BlockPlace block_place(int b, const BlockOrder& o, const BlockAxis& ra,
                                                   const BlockAxis& ca) {
-  const int x = b % kXcds;
-  const int t = x * o.per_xcd + min(x, o.extra) + b / kXcds;
+  const int x = b % kXcds, k = b / kXcds;
+  const int last = o.per_xcd - (x < o.extra ? 0 : 1);
+  const int t = x * o.per_xcd + min(x, o.extra) + (o.back ? last - k : k);
   const int per = kBlockGroup * ca.n;
   // t / per: the float quotient is within one of it (t < 2^24)
   int g = __builtin_amdgcn_readfirstlane((int)((float)t * o.inv_group));
@@ -499,15 +504,19 @@ k_block(Coef c, BlockIO io, int H, int W, BlockStim st, int n_lev, float dt, flo
 // launch cost the launch (a), many cost the columns and rows that only feed the
 // stencil (b). The least is taken. Of the tilings tried (1 and 2 columns per lane,
 // 2 to 6 rows per wave, 4 to 16 waves, 2 to 4 steps) these four were the fastest
-// somewhere.
+// somewhere. Where a step's 28 bytes per cell exceed the 256 MB cache, two steps
+// per launch wait for memory (32 rows 66.5 us at 4096^2 and 100 at 5000^2, 48 rows
+// and three steps 65.1 and 95.3; at 3000^2 30.8 and 34.7): a larger b there.
 typedef BlockCfg<2, 16, 4> Block32x4;
 typedef BlockCfg<4, 8, 2> Block32x2;
 typedef BlockCfg<4, 12, 3> Block48x3;
 typedef BlockCfg<4, 16, 3> Block64x3;
 
 struct LeastRounds {
+  const bool streams;
   int best = -1;
   double least = 0.0;
+  explicit LeastRounds(int64_t cells) : streams(28 * cells > (256 << 20)) {}
   void offer(int id, int64_t tiles, double a, double b) {
     const double us = a + b * (double)((tiles + 255) / 256);
     if (best < 0 || us < least) best = id, least = us;
@@ -515,7 +524,7 @@ struct LeastRounds {
   void offer(int id, Block32x4, int64_t tiles) { offer(id, tiles, 1.0, 1.05); }
   void offer(int id, Block48x3, int64_t tiles) { offer(id, tiles, 1.7, 1.25); }
   void offer(int id, Block64x3, int64_t tiles) { offer(id, tiles, 1.4, 2.05); }
-  void offer(int id, Block32x2, int64_t tiles) { offer(id, tiles, 2.2, 1.0); }
+  void offer(int id, Block32x2, int64_t tiles) { offer(id, tiles, 2.2, streams ? 1.15 : 1.0); }
 };
 
 template <class Cfg>

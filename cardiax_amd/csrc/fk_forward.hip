@@ -416,14 +416,13 @@ static int resolve_variant(int v) { return v == kAuto ? (int)kStream2 : v; }
 // The variant an automatic solve of several steps runs when the shape was not
 // tuned: block tiles, which equal the streaming kernels of default_variant bit
 // for bit, in the tiling that LeastRounds finds. Against the best streaming
-// kernel, us per step: 128^2 2.05 and 3.07 (32 rows, 4
-// steps), 500^2 3.0 and 3.9 (48 rows, 3), 700 x 600 3.5 and 5.4 (64 rows, 3),
-// 1024^2 6.2 and 7.2, 1200^2 7.3 and 10.0, 2048^2 15.9 and 17.2, 4096^2 70 and
-// 78 (32 rows, 2).
+// kernel, us per step: 128^2 2.05 and 3.07 (32 rows, 4 steps), 500^2 3.0 and 3.9
+// (48 rows, 3), 700 x 600 3.5 and 5.4 (64 rows, 3), 1024^2 6.1 and 7.2, 1200^2 7.2
+// and 10.0, 2048^2 15.6 and 17.2 (32 rows, 2), 4096^2 65 and 78 (48 rows, 3).
 static int auto_variant(int H, int W) {
   const int d = default_variant(H, W);
   if (d == kTile16) return d;  // narrow grids above 8 M cells: another rounding
-  LeastRounds r;
+  LeastRounds r((int64_t)H * W);
   r.offer(kBlock32x4, Block32x4{}, block_tiles<Block32x4>(H, W));
   r.offer(kBlock48x3, Block48x3{}, block_tiles<Block48x3>(H, W));
   r.offer(kBlock64x3, Block64x3{}, block_tiles<Block64x3>(H, W));
@@ -542,29 +541,29 @@ static hipError_t launch_step(int variant, bool euler, const Coef& c, const floa
   return hipGetLastError();
 }
 
-// n_lev (at most Cfg::steps) levels on every tile.
+// n_lev (at most Cfg::steps) levels on every tile. back: see BlockOrder.
 template <class Cfg, bool HEUN>
 static hipError_t launch_tiles(const Coef& c, const BlockIO& io, int H, int W,
-                               const BlockStim& st, int n_lev, float dt, float inv_dx2,
+                               const BlockStim& st, int n_lev, float dt, float inv_dx2, bool back,
                                hipStream_t s) {
   const BlockAxis ra = Cfg::row_axis(H), ca = Cfg::col_axis(W);
   k_block<Cfg, HEUN><<<(unsigned)(ra.n * ca.n), Cfg::waves * 64, 0, s>>>(
-      c, io, H, W, st, n_lev, dt, inv_dx2, ra, ca, make_block_order(ra, ca));
+      c, io, H, W, st, n_lev, dt, inv_dx2, ra, ca, make_block_order(ra, ca, back));
   return hipGetLastError();
 }
 
 // n_lev steps (at most the variant's) of block variant v.
 static hipError_t launch_block(int v, const Coef& c, const BlockIO& io, int H, int W,
-                               const BlockStim& st, int n_lev, float dt, float inv_dx2,
+                               const BlockStim& st, int n_lev, float dt, float inv_dx2, bool back,
                                hipStream_t s) {
   switch (v) {
     case kBlock32x2:
-      return launch_tiles<Block32x2, false>(c, io, H, W, st, n_lev, dt, inv_dx2, s);
+      return launch_tiles<Block32x2, false>(c, io, H, W, st, n_lev, dt, inv_dx2, back, s);
     case kBlock48x3:
-      return launch_tiles<Block48x3, false>(c, io, H, W, st, n_lev, dt, inv_dx2, s);
+      return launch_tiles<Block48x3, false>(c, io, H, W, st, n_lev, dt, inv_dx2, back, s);
     case kBlock64x3:
-      return launch_tiles<Block64x3, false>(c, io, H, W, st, n_lev, dt, inv_dx2, s);
-    default: return launch_tiles<Block32x4, false>(c, io, H, W, st, n_lev, dt, inv_dx2, s);
+      return launch_tiles<Block64x3, false>(c, io, H, W, st, n_lev, dt, inv_dx2, back, s);
+    default: return launch_tiles<Block32x4, false>(c, io, H, W, st, n_lev, dt, inv_dx2, back, s);
   }
 }
 
@@ -588,7 +587,7 @@ typedef BlockCfg<5, 8, 2> Heun40x1;
 enum HeunTiling { kHeun32x2, kHeun48x2, kHeun64x1, kHeun40x1 };
 
 static int heun_tiling(int H, int W) {
-  LeastRounds r;
+  LeastRounds r((int64_t)H * W);
   r.offer(kHeun32x2, block_tiles<Heun32x2>(H, W), 2.0, 2.9);
   r.offer(kHeun48x2, block_tiles<Heun48x2>(H, W), 1.8, 4.2);
   r.offer(kHeun64x1, block_tiles<Heun64x1>(H, W), 2.2, 7.45);
@@ -599,13 +598,14 @@ static int heun_tiling(int H, int W) {
 static int heun_steps(int tiling) { return tiling == kHeun32x2 || tiling == kHeun48x2 ? 2 : 1; }
 
 static hipError_t launch_heun(int tiling, const Coef& c, const BlockIO& io, int H, int W,
-                              const BlockStim& st, int n, float dt, float inv_dx2,
+                              const BlockStim& st, int n, float dt, float inv_dx2, bool back,
                               hipStream_t s) {
+  const int l = 2 * n;
   switch (tiling) {
-    case kHeun32x2: return launch_tiles<Heun32x2, true>(c, io, H, W, st, 2 * n, dt, inv_dx2, s);
-    case kHeun48x2: return launch_tiles<Heun48x2, true>(c, io, H, W, st, 2 * n, dt, inv_dx2, s);
-    case kHeun64x1: return launch_tiles<Heun64x1, true>(c, io, H, W, st, 2 * n, dt, inv_dx2, s);
-    default: return launch_tiles<Heun40x1, true>(c, io, H, W, st, 2 * n, dt, inv_dx2, s);
+    case kHeun32x2: return launch_tiles<Heun32x2, true>(c, io, H, W, st, l, dt, inv_dx2, back, s);
+    case kHeun48x2: return launch_tiles<Heun48x2, true>(c, io, H, W, st, l, dt, inv_dx2, back, s);
+    case kHeun64x1: return launch_tiles<Heun64x1, true>(c, io, H, W, st, l, dt, inv_dx2, back, s);
+    default: return launch_tiles<Heun40x1, true>(c, io, H, W, st, l, dt, inv_dx2, back, s);
   }
 }
 
@@ -634,7 +634,7 @@ static int32_t heun_loop(const fk_params* params, const float* D, const float* c
       st.act[l] = sched.mask(t + (double)(k + l / 2));
     float* const* d = bufs[dst];
     const BlockIO io{D, src[0], src[1], src[2], d[0], d[1], d[2], 0, false};
-    HIP_CHECK(launch_heun(tiling, c, io, H, W, st, m, dt, inv_dx2, s));
+    HIP_CHECK(launch_heun(tiling, c, io, H, W, st, m, dt, inv_dx2, dst == 1, s));
     src[0] = d[0];
     src[1] = d[1];
     src[2] = d[2];
@@ -707,7 +707,7 @@ int32_t forward_loop(int variant, const fk_params* params, const float* D, const
       const int ns = (int)std::min<int64_t>(depth, steps - k);
       block_stim(sched, t + (double)k, ns, st);
       const BlockIO io{D, src[0], src[1], src[2], d[0], d[1], d[2], 0, false};
-      HIP_CHECK(launch_block(v, c, io, H, W, st, ns, dt, inv_dx2, s));
+      HIP_CHECK(launch_block(v, c, io, H, W, st, ns, dt, inv_dx2, dst == 1, s));
     } else if (is_block(v)) {  // a single last step
       HIP_CHECK(launch_step(kStream2, true, c, D, src[0], src[1], src[2], H, W,
                             sched.at(t + (double)k), dt, inv_dx2, d[0], d[1], d[2], s));
@@ -1035,7 +1035,7 @@ int32_t fk_forward_trajectory(const fk_params* params, const float* D, const flo
       const int ns = std::min(block_steps(v), n_steps - k);
       block_stim(sched, t + (double)k, ns, st);
       const BlockIO io{D, src[0], src[1], src[2], d, d + n, d + 2 * n, 3 * n, true};
-      HIP_CHECK(launch_block(v, c, io, H, W, st, ns, dt, inv_dx2, (hipStream_t)stream));
+      HIP_CHECK(launch_block(v, c, io, H, W, st, ns, dt, inv_dx2, false, (hipStream_t)stream));
       d += (size_t)(ns - 1) * 3 * n;
       src[0] = d;
       src[1] = d + n;

@@ -268,7 +268,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
     n32x2 += block_tiles<Block32x2>(H, W);
     n_rev4 += (int64_t)adj_strips(W) * ((H + 3) / 4);
   }
-  LeastRounds least;
+  LeastRounds least(0);  // every step writes its state, whatever the cache holds
   least.offer(kRoll32x4, Block32x4{}, n32x4);
   least.offer(kRoll48x3, Block48x3{}, n48x3);
   least.offer(kRoll32x2, Block32x2{}, n32x2);
