@@ -210,12 +210,16 @@ struct AdjArgs {
 // tab: the wave's LDS copy of the tables, filled here where they are used (read
 // from memory one row after another they were most of an edge wave's time: a
 // dozen dependent scalar loads, 33 us in place of 29 for the 12 problems).
+// R = 1: a wave per row, the even row of a pair and the odd one next to each
+// other in a block; every wave of the block calls it (a barrier). The even row
+// passes its tau terms on through `pair` (3 x 64 floats), the odd one adds.
 template <int R, bool XG, bool YG, class SV>
 __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H, int W,
                                          const SV& sv, float dt, float inv_dx2, int rs, int cs,
-                                         AdjAxisTab* tab) {
+                                         AdjAxisTab* tab, float* pair = nullptr) {
 #pragma clang fp contract(off)
-  static_assert(R % 2 == 0, "tau groups are pairs of rows");
+  static_assert(R == 1 || R % 2 == 0, "tau groups are pairs of rows");
+  constexpr int P = R == 1 ? 1 : R / 2;  // pairs of rows
   constexpr int E = XG ? kRevHalo : 4;  // window rows above and below the band
   constexpr int NW = R + 2 * E, NG = NW - 4;  // window; its first differences
   const int lane = threadIdx.x & 63;
@@ -254,12 +258,12 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
   // lane loads the same words, so that they arrive with the rest: read where they
   // are added to, they ended the wave with a trip to memory).
   double* gt = a.g_tau + 3 * ((size_t)(cs / kRevOut) * ((H + 1) / 2) + rs / 2);
-  double g0[3 * (R / 2)];
+  double g0[3 * P];
 #pragma unroll
-  for (int p = 0; p < R / 2; ++p)
+  for (int p = 0; p < P; ++p)
 #pragma unroll
     for (int f = 0; f < 3; ++f)
-      g0[3 * p + f] = !XG || rs + 2 * p < H
+      g0[3 * p + f] = !XG || (rs & ~1) + 2 * p < H
                           ? ((const double __attribute__((address_space(1)))*)gt)[3 * p + f]
                           : 0.0;
   float vv[R], ww[R], lvv[R], lww[R], gd[R];
@@ -418,7 +422,18 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
     const float t_d = (q ? -vv[k] * a1 * c.inv_td : 0.0f) * lt;
     const float t_r = (q ? c.inv_tr * c.inv_tr * c.inv_cm : 0.0f) * lt;
     const float t_si = (-ww[k] * S * c.inv_tsi * c.inv_tsi * c.inv_cm) * lt;
-    if (k % 2 == 0) {
+    if (R == 1) {
+      if ((rs & 1) == 0) {
+        pair[lane] = t_d;
+        pair[64 + lane] = t_r;
+        pair[128 + lane] = t_si;
+      }
+      lds_barrier();
+      if ((rs & 1) == 0) return;
+#pragma unroll
+      for (int f = 0; f < 3; ++f) ts[f] = pair[64 * f + lane];
+    }
+    if (R > 1 && k % 2 == 0) {
       ts[0] = t_d;
       ts[1] = t_r;
       ts[2] = t_si;
@@ -436,6 +451,12 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
   }
 }
 
+// Up to this many bands of 2 rows a reverse step runs a wave per row: the waves
+// all run at once and an edge wave's rows, 1.2 us each, set the time. Forward and
+// backward over 200 steps, 2 rows per wave and one: 128^2 2.00 and 1.70 ms, 256^2
+// (640 bands) 2.05 and 1.88, 400^2 (1600) 2.47 and 2.32, 600^2 (3600) 3.39 and 3.56.
+constexpr int kRevRowTiles = 2048;
+
 // Whether the band of R rows at rs, the strip at cs take the edge rules.
 __host__ __device__ inline bool adj_edge_band(int rs, int R, int H) {
   return rs < kAdjT || rs + R + kAdjT > H;
@@ -448,12 +469,12 @@ __host__ __device__ inline bool adj_edge_strip(int cs, int W) {
 template <int R, class SV>
 __device__ __forceinline__ void adj_tile_any(const Coef& c, const AdjArgs& a, int H, int W,
                                              const SV& sv, float dt, float inv_dx2, int rs, int cs,
-                                             int flags, AdjAxisTab* tab) {
+                                             int flags, AdjAxisTab* tab, float* pair = nullptr) {
   switch (flags) {
-    case 0: adj_tile<R, false, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
-    case 1: adj_tile<R, true, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
-    case 2: adj_tile<R, false, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
-    default: adj_tile<R, true, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
+    case 0: adj_tile<R, false, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab, pair); break;
+    case 1: adj_tile<R, true, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab, pair); break;
+    case 2: adj_tile<R, false, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab, pair); break;
+    default: adj_tile<R, true, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab, pair); break;
   }
 }
 

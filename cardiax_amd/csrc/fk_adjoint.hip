@@ -72,6 +72,21 @@ k_adj_rev(Coef c, AdjArgs a, int H, int W, StimArgs sa, float dt, float inv_dx2,
                   tab[threadIdx.x >> 6]);
 }
 
+// The same with a wave per row, a pair of rows per block.
+__global__ void __launch_bounds__(128)
+k_adj_rev_row(Coef c, AdjArgs a, int H, int W, StimArgs sa, float dt, float inv_dx2,
+              int n_pairs) {
+  __shared__ AdjAxisTab tab[2][2];
+  __shared__ float pair[3 * 64];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int strip = blockIdx.x / n_pairs;
+  const int rs = 2 * (blockIdx.x - strip * n_pairs) + wave, cs = kRevOut * strip;
+  const AdjStimList sv{sa};
+  adj_tile_any<1>(c, a, H, W, sv, dt, inv_dx2, rs, cs,
+                  (adj_edge_band(rs, 1, H) ? 1 : 0) | (adj_edge_strip(cs, W) ? 2 : 0), tab[wave],
+                  pair);
+}
+
 __global__ void k_adj_zero(float* a, size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
@@ -135,6 +150,11 @@ static hipError_t launch_rev(const AdjLayout& L, char* wk, const Coef& c, const 
                   lam_out[2], gD, (double*)(wk + L.part), (const AdjAxisTab*)(wk + L.tab)};
   const int strips = adj_strips(W), bands = (H + kRevRows - 1) / kRevRows;
   const int tiles = strips * bands;
+  if (tiles <= kRevRowTiles) {
+    const int pairs = (H + 1) / 2;
+    k_adj_rev_row<<<strips * pairs, 128, 0, s>>>(c, a, H, W, sa, dt, inv_dx2, pairs);
+    return hipGetLastError();
+  }
   k_adj_rev<kRevRows><<<(tiles + 3) / 4, 256, 0, s>>>(c, a, H, W, sa, dt, inv_dx2, bands, tiles);
   return hipGetLastError();
 }

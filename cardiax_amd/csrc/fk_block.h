@@ -145,13 +145,6 @@ __device__ __forceinline__ void reaction_side(const Coef& c, float v, float w, f
   }
 }
 
-// Barrier that orders LDS only: global stores of a level stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Inputs and outputs of a tile. Level l (from 1) writes to o_* + (l - 1)
 // o_stride when `all` is set (a trajectory), else the last one to o_*.
 struct BlockIO {

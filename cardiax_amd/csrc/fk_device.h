@@ -12,6 +12,13 @@
 
 namespace fk {
 
+// Barrier that orders LDS only: global stores of a level stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Per-launch constants derived from fk_params on the host (double math, then
 // rounded once to float). Reciprocals replace the reference's divisions.
 struct Coef {

@@ -156,16 +156,19 @@ __device__ __forceinline__ const float* roll_inject(const RollDesc& S, int j, in
 }
 
 // Reverse of step c + k of segment `seg` (j = c + k + 1): cotangent set `cur`
-// (0 lam, 1 lam_alt) -> the other; x_j's frame cotangent enters first.
+// (0 lam, 1 lam_alt) -> the other; x_j's frame cotangent enters first. R = 1: a
+// pair of rows per block of two waves.
 template <int R>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(R == 1 ? 128 : 256)
 k_roll_rev(const RollDesc* __restrict__ sims, const RollTile* __restrict__ items, int n_items,
            const uint32_t* __restrict__ masks, int seg, int k, int j, int fe, int cur) {
-  __shared__ AdjAxisTab tab[4][2];
-  const int it = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x >> 6));
+  constexpr int kWaves = R == 1 ? 2 : 4;
+  __shared__ AdjAxisTab tab[kWaves][2];
+  __shared__ float pair[R == 1 ? 3 * 64 : 1];
+  const int it = __builtin_amdgcn_readfirstlane(blockIdx.x * kWaves + (int)(threadIdx.x >> 6));
   if (it >= n_items) return;
   RollTile item = items[it];
-  if (uni(item.sim) < 0) return;  // padding of the XCD order
+  if (uni(item.sim) < 0) return;  // padding of the XCD order (of whole pairs)
   item.sim = uni(item.sim);
   const RollDesc& S = sims[item.sim];
   const size_t n = S.cells;
@@ -185,7 +188,7 @@ k_roll_rev(const RollDesc* __restrict__ sims, const RollTile* __restrict__ items
   c.inv_t0 = uni(c.inv_t0); c.inv_tr = uni(c.inv_tr); c.inv_tsi = uni(c.inv_tsi);
   c.inv_cm = uni(c.inv_cm);
   adj_tile_any<R>(c, a, uni(S.H), uni(S.W), sv, uni(S.dt), uni(S.inv_dx2), uni(item.rs),
-                  uni(item.cs), uni(item.flags), tab[threadIdx.x >> 6]);
+                  uni(item.cs), uni(item.flags), tab[threadIdx.x >> 6], pair);
 }
 
 }  // namespace fk
@@ -260,25 +263,26 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   b->S = std::min(checkpoint_every, n_steps);
   b->n_seg = (n_steps + b->S - 1) / b->S;
   b->specs.assign(specs, specs + n);
-  int64_t n32x4 = 0, n48x3 = 0, n32x2 = 0, n_rev4 = 0;
+  int64_t n32x4 = 0, n48x3 = 0, n32x2 = 0, n_rev4 = 0, n_rev2 = 0;
   for (int i = 0; i < n; ++i) {
     const int H = specs[i].H, W = specs[i].W;
     n32x4 += block_tiles<Block32x4>(H, W);
     n48x3 += block_tiles<Block48x3>(H, W);
     n32x2 += block_tiles<Block32x2>(H, W);
     n_rev4 += (int64_t)adj_strips(W) * ((H + 3) / 4);
+    n_rev2 += (int64_t)adj_strips(W) * ((H + 1) / 2);
   }
   LeastRounds least(0);  // every step writes its state, whatever the cache holds
   least.offer(kRoll32x4, Block32x4{}, n32x4);
   least.offer(kRoll48x3, Block48x3{}, n48x3);
   least.offer(kRoll32x2, Block32x2{}, n32x2);
   b->block = least.best;
-  // Reverse bands of 2 rows while the waves are few and a wave's rows, one after
+  // A row per wave as in the per-grid step; bands of 2 rows while the waves are few and a wave's rows, one after
   // the other, set the time (2 problems 64 to 200 wide, 100 steps: 1.07 ms, 1.33 with
   // 4; 10 of 128 to 480: 3.33 and 3.40); 4 rows for more (12 of 128 to 512: 4.63 and
   // 4.69; one reverse step of 3.84 M cells 60 and 68 us, 67 with 8). The bits do not
   // depend on it.
-  b->rev_rows = n_rev4 <= 5000 ? 2 : 4;
+  b->rev_rows = n_rev2 <= kRevRowTiles ? 1 : n_rev4 <= 5000 ? 2 : 4;
   const int rows = b->rev_rows;
   // work lists over the dies: neighbouring forward tiles, and runs of vertically
   // adjacent reverse tiles (which share halo rows), whole on one die each
@@ -293,7 +297,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
       default: append_block_items<Block32x2>(i, s.H, s.W, blocks); break;
     }
     for (int strip = 0; strip < adj_strips(s.W); ++strip)
-      for (int band = 0; band < (s.H + rows - 1) / rows; ++band) {
+      for (int band = 0; band < (rows == 1 ? (s.H + 1) / 2 * 2 : (s.H + rows - 1) / rows); ++band) {
         RollTile t;
         t.sim = i;
         t.cs = kRevOut * strip;
@@ -305,7 +309,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
       }
   }
   const std::vector<BlockItem> tiles = block_work_list(blocks);
-  const std::vector<RollTile> rev = xcd_order(rev_runs, 4, RollTile{-1, 0, 0, 0});
+  const std::vector<RollTile> rev = xcd_order(rev_runs, rows == 1 ? 2 : 4, RollTile{-1, 0, 0, 0});
   b->n_tiles = (int)tiles.size();
   b->n_rev = (int)rev.size();
   // stimulus activity of every step, as the per-grid path evaluates it
@@ -446,7 +450,7 @@ int32_t fk_rollout_batch_backward(fk_rollout_batch* b, float* g_tau, void* strea
   }
   const dim3 cg = roll_cell_grid(b);
   k_roll_zero<<<cg, 256, 0, s>>>(b->d_sims);
-  const int rev_blocks = (b->n_rev + 3) / 4;
+  const int rev_blocks = b->n_rev / (b->rev_rows == 1 ? 2 : 4);  // whole blocks, padded
   for (int seg = b->n_seg - 1; seg >= 0; --seg) {
     const int c = seg * b->S, len = std::min(b->S, b->n_steps - c);
     // recompute x_{c+1} .. x_{c+len-1}, unless the forward's last segment is
@@ -456,7 +460,10 @@ int32_t fk_rollout_batch_backward(fk_rollout_batch* b, float* g_tau, void* strea
     int cur = 0;
     for (int k = len - 1; k >= 0; --k) {
       const uint32_t* m = b->d_masks + (size_t)(c + k) * b->n;
-      if (b->rev_rows == 2)
+      if (b->rev_rows == 1)
+        k_roll_rev<1><<<rev_blocks, 128, 0, s>>>(b->d_sims, b->d_rev, b->n_rev, m, seg, k,
+                                                 c + k + 1, b->fe, cur);
+      else if (b->rev_rows == 2)
         k_roll_rev<2><<<rev_blocks, 256, 0, s>>>(b->d_sims, b->d_rev, b->n_rev, m, seg, k,
                                                  c + k + 1, b->fe, cur);
       else
