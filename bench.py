@@ -28,7 +28,7 @@ TRAFFIC_NOTE = "FETCH_SIZE + WRITE_SIZE (L2-to-fabric; includes MALL hits)"
 # What `achieved` counts: the algorithmic bytes of the Euler steps a launch
 # performs, so for a two-step launch it is an effective bandwidth (the launch
 # moves the state once for both steps; `traffic` is what it moved).
-ACHIEVED_BASIS = "28 B per cell-update x the launch's cell-updates (effective for two-step launches)"
+ACHIEVED_BASIS = "28 B per cell-update x the launch's cell-updates (effective for launches of several steps)"
 BYTES_PER_CELL_UPDATE = 28  # read v, w, u, D + write v, w, u (fp32)
 
 # Step-kernel variant -> (kernel the variant launches, Euler steps per launch).
@@ -234,7 +234,7 @@ def leg_roofline(bytes_per_launch, seconds_per_launch, kernel, key):
 
 def bench_adjoint(seed, size=256, n_steps=2000, frame_every=50, reps=2):
     """Gradient of the frame MSE with respect to D (size^2) and tau_d, tau_r,
-    tau_si by the hand-written adjoint with sqrt(N) checkpoints, against the
+    tau_si by the hand-written adjoint over the forward's kept states, against the
     plain forward of the same rollout."""
     import numpy as np
     import torch
@@ -280,7 +280,7 @@ def bench_adjoint(seed, size=256, n_steps=2000, frame_every=50, reps=2):
     per_step = adjoint_step_seconds(st, prm, Dstar, stims, shape, t_mid=n_steps // 2)
     fwd_adj = ADJ_FWD_BWD_BYTES * cells / tb / 1e9
     return {"workload": "%dx%d, %d Euler steps, u frames every %d, MSE vs a hidden scar D-map, "
-                        "grad wrt D and tau_d/tau_r/tau_si, sqrt(N) checkpoints"
+                        "grad wrt D and tau_d/tau_r/tau_si, states kept"
                         % (size, size, n_steps, frame_every),
             "forward_s": round(tf, 4), "fwd_adjoint_s": round(tb, 4),
             "cost_ratio": round(tb / tf, 2),
@@ -290,24 +290,23 @@ def bench_adjoint(seed, size=256, n_steps=2000, frame_every=50, reps=2):
                                 "achieved": round(fwd_adj, 1),
                                 "frac": round(fwd_adj / HBM_PEAK_GBS, 4)},
             "roofline": dict(leg_roofline(ADJ_BWD_BYTES * size * size, per_step,
-                                          "k_adj_rev<2>", "%dx%d" % shape),
+                                          "k_adj_rev_row", "%dx%d" % shape),
                              design_bytes_per_launch=ADJ_BWD_DESIGN_BYTES * size * size),
             "grad_finite": bool(torch.isfinite(D.grad).all().item())}
 
 
 # Algorithmic bytes of the adjoint per cell-step: the reverse step reads the
 # cotangent (12), the state (12) and D (4), writes the cotangent (12) and
-# read-modify-writes dL/dD (8); forward + backward adds the forward step (28)
-# and its recompute from the checkpoints (28).
+# read-modify-writes dL/dD (8); forward + backward adds the forward step (28).
 ADJ_BWD_BYTES = 48
-ADJ_FWD_BWD_BYTES = 104
+ADJ_FWD_BWD_BYTES = 76
 # What the reverse kernel moves by construction per cell: nothing more, beside
 # the halo rows and columns of its windows of u, D and lam_u.
 ADJ_BWD_DESIGN_BYTES = 48
 
 
 def adjoint_step_seconds(st, prm, D, stims, shape, t_mid, n_short=10, n_long=40):
-    """Time of one reverse step (k_adj_rev<2>) on the stream it runs on:
+    """Time of one reverse step (k_adj_rev_row) on the stream it runs on:
     fk_adjoint_segment over n_long and n_short steps of a trajectory from the
     middle of the rollout, HIP events around each; the difference cancels the
     segment's fixed launches."""
@@ -553,7 +552,7 @@ def bench_scar(seed, size=1200, reps=5):
     deepx/utils_scars.py:246-426) at the reference's default 1200^2 image:
     the whole call (host contours + device rasterisation, blur and rescale)
     and each device kernel on its own, timed with HIP events on the current
-    stream. The blur dominates: 2 kh kw FP64 flops per pixel (kh = kw =
+    stream. The blur dominates: 2 (kh + kw) FP64 flops per pixel (kh = kw =
     int(0.1 size)), against the FP64 peak. The CPU leg is the oracle
     pipeline (brute-force crossing numbers, scipy's FFT convolution, FP64
     rescale) on one core."""
@@ -594,7 +593,7 @@ def bench_scar(seed, size=1200, reps=5):
     for _ in range(n):
         scars.rasterize(cs, shape, out=mask)  # synchronises per call
     raster_s = (time.perf_counter() - t0) / n
-    flops = 2.0 * ksize * ksize * size * size
+    flops = 2.0 * (ksize + ksize) * size * size
     achieved = flops / blur_s / 1e12
     # CPU: the oracle pipeline on the same contours
     from oracle import scar_oracle as so
@@ -614,7 +613,7 @@ def bench_scar(seed, size=1200, reps=5):
             "roofline": {"bound": "fp64", "achieved": round(achieved, 2),
                          "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
-                         "kernel": "k_convolve_same", "flops_per_launch": int(flops)},
+                         "kernel": "k_conv_cols + k_conv_rows", "flops_per_launch": int(flops)},
             "D_range": [float(D.min()), float(D.max())],
             "cpu_oracle_ms": {"raster": round(t_mask * 1e3, 1),
                               "fft_blur_and_rescale": round(t_fft * 1e3, 1), "cores": 1}}

@@ -201,9 +201,10 @@ struct AdjArgs {
 // cotangent 12 in and 12 out, D 4, dL/dD 8: 48 per cell, and the windows' halo
 // rows). It replaced a kernel that kept seven derived fields in memory (104
 // bytes by design, 121-142 measured), two threads per cell:
-// 59.1 us before, 28.9 now per step of 12 problems of 128^2 to 512^2 (1.26 M
-// cells); 61 us for 3.84 M cells (3.0 TB/s of the 48 bytes); 7.05 and 7.0 at
-// 256^2, where a launch and an edge wave's own instructions bound both.
+// 59.1 us before, 27.6 now per step of 12 problems of 128^2 to 512^2 (1.26 M
+// cells; 167 registers, three waves per SIMD); 61 us for 3.84 M cells (3.0 TB/s of
+// the 48 bytes); 7.05 and, a wave per row, 6.2 at 256^2, where a launch and an edge
+// wave's own instructions bound both.
 // XG, YG: a row within 13 of an edge, a column within 13 of a side. In such a
 // band each row, and in such a strip each lane, takes the table or the central
 // taps by itself, so neither the band height nor the strip changes a bit.

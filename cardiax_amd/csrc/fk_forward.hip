@@ -396,14 +396,13 @@ static int tuned_variant(int H, int W) {
   return it == g_tuned.end() ? (int)kAuto : it->second;
 }
 
-// Default when no variant is set and the shape was not tuned, from the
-// variants measured on MI355X. Up to 1.1 M cells, streaming bands of 2 rows:
-// small bands give enough waves to hide latency, and a grid this small is
-// limited by issue rate more than by memory. Above, two steps per launch
-// (bands of 8 rows up to 2.5 M cells, of 16 above): half the memory traffic
-// and half the launches per step, 20-30% faster at 1200^2, 2048^2 and
-// 4096^2. Grids too small for those run 2-row bands up to 8 M cells and the
-// LDS tile above.
+// Streaming default when no variant is set and the shape was not tuned: the
+// kernel of single steps, and what auto_variant's solves replace. Up to 1.1 M
+// cells, streaming bands of 2 rows: small bands give enough waves to hide
+// latency, and a grid this small is limited by issue rate more than by memory.
+// Above, two steps per launch (bands of 8 rows up to 2.5 M cells, of 16 above),
+// which single steps run as 2-row bands. Grids too small for those run 4-row
+// bands up to 8 M cells and the LDS tile above.
 static int default_variant(int H, int W) {
   const size_t n = (size_t)H * W;
   if (n <= 1100 * 1024) return kStream2;
