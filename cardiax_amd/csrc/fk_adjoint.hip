@@ -72,15 +72,21 @@ k_adj_rev(Coef c, AdjArgs a, int H, int W, StimArgs sa, float dt, float inv_dx2,
                   tab[threadIdx.x >> 6]);
 }
 
-// The same with a wave per row, a pair of rows per block.
+// The same with a wave per row, a pair of rows per block. A die takes a run of
+// whole bands across the strips, so that neighbours' windows come from its L2 and
+// the edge strips spread over all dies; forward and backward over 200 steps,
+// strips first in plain order and so: 256^2 1.88 and 1.76 ms, 350^2 2.33 and 2.16,
+// 400^2 2.32 and 2.30 (runs along a strip: 1.82, 2.19 and 2.46).
 __global__ void __launch_bounds__(128)
 k_adj_rev_row(Coef c, AdjArgs a, int H, int W, StimArgs sa, float dt, float inv_dx2,
-              int n_pairs) {
+              int n_strips) {
   __shared__ AdjAxisTab tab[2][2];
   __shared__ float pair[3 * 64];
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int strip = blockIdx.x / n_pairs;
-  const int rs = 2 * (blockIdx.x - strip * n_pairs) + wave, cs = kRevOut * strip;
+  const int x = blockIdx.x % kXcds, q = gridDim.x / kXcds, r = gridDim.x % kXcds;
+  const int t = x * q + min(x, r) + blockIdx.x / kXcds;  // a die's pairs are neighbours
+  const int band = t / n_strips;
+  const int rs = 2 * band + wave, cs = kRevOut * (t - band * n_strips);
   const AdjStimList sv{sa};
   adj_tile_any<1>(c, a, H, W, sv, dt, inv_dx2, rs, cs,
                   (adj_edge_band(rs, 1, H) ? 1 : 0) | (adj_edge_strip(cs, W) ? 2 : 0), tab[wave],
@@ -152,7 +158,7 @@ static hipError_t launch_rev(const AdjLayout& L, char* wk, const Coef& c, const 
   const int tiles = strips * bands;
   if (tiles <= kRevRowTiles) {
     const int pairs = (H + 1) / 2;
-    k_adj_rev_row<<<strips * pairs, 128, 0, s>>>(c, a, H, W, sa, dt, inv_dx2, pairs);
+    k_adj_rev_row<<<strips * pairs, 128, 0, s>>>(c, a, H, W, sa, dt, inv_dx2, strips);
     return hipGetLastError();
   }
   k_adj_rev<kRevRows><<<(tiles + 3) / 4, 256, 0, s>>>(c, a, H, W, sa, dt, inv_dx2, bands, tiles);
