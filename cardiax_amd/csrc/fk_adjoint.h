@@ -456,7 +456,7 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
 // all run at once and an edge wave's rows, 1.2 us each, set the time. Forward and
 // backward over 200 steps, 2 rows per wave and one: 128^2 2.00 and 1.70 ms, 256^2
 // (640 bands) 2.05 and 1.76, 400^2 (1600) 2.47 and 2.30, 600^2 (3600) 3.39 and 3.56
-// (in plain order).
+// (in the order of strips).
 constexpr int kRevRowTiles = 2048;
 
 // Whether the band of R rows at rs, the strip at cs take the edge rules.
