@@ -151,11 +151,12 @@ __device__ __forceinline__ void lane_window(float y, float x[2 * n + 1]) {
 constexpr int kRevOut = 54;   // output columns per wave: 5 halo lanes on each side
 constexpr int kRevHalo = 5;   // what an edge's rules reach (4 away from the edges)
 
-// Tau accumulators: one triple of doubles per strip and pair of rows, so that
-// the sums do not depend on the band height.
+// Tau accumulators: one triple of doubles per strip and row. At most 54 terms are
+// added in float before a sum goes to its double, and the sums do not depend on
+// the band height.
 __host__ __device__ inline int adj_strips(int W) { return (W + kRevOut - 1) / kRevOut; }
 __host__ __device__ inline size_t adj_n_groups(int H, int W) {
-  return (size_t)adj_strips(W) * (size_t)((H + 1) / 2);
+  return (size_t)adj_strips(W) * (size_t)H;
 }
 
 // Stimulus fields of one step as an active list (count(), on(m), field(m)).
@@ -166,22 +167,33 @@ struct AdjStimList {
   __device__ const float* field(int m) const { return sa.f[m]; }
 };
 
-// Sum over the wave's 64 lanes, valid in lane 63: a fixed tree of DPP moves
-// (no LDS). The lanes without a source add 0.
-__device__ __forceinline__ float wave_sum63(float x) {
-  auto add = [](float a, auto ctrl, auto rows) {
-    const int m = __builtin_amdgcn_update_dpp(0, __float_as_int(a), decltype(ctrl)::value,
-                                              decltype(rows)::value, 0xf, false);
+// Sums over the wave of up to four values, each into its own 16 lanes, by lane
+// moves (no LDS): half the operations of a tree for each value.
+// x of the lanes 0-15 and 32-47 and y of the same, each with the 16 lanes above
+// it: x's sums go to the lower 16, y's to the upper.
+__device__ __forceinline__ float pair_sum16(float x, float y) {
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false,
+                                                  false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+// The same of the lower and the upper 32 lanes.
+__device__ __forceinline__ float pair_sum32(float x, float y) {
+  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false,
+                                                  false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+// Sum over each 16 lanes, in all of them.
+__device__ __forceinline__ float row_sum(float x) {
+  auto add = [](float a, auto ctrl) {
+    const int m = __builtin_amdgcn_update_dpp(0, __float_as_int(a), decltype(ctrl)::value, 0xf,
+                                              0xf, false);
     return a + __int_as_float(m);
   };
   using std::integral_constant;
-  x = add(x, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr:1
-  x = add(x, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});  // row_shr:2
-  x = add(x, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});  // row_shr:4
-  x = add(x, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});  // row_shr:8
-  x = add(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row_bcast:15
-  x = add(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row_bcast:31
-  return x;
+  x = add(x, integral_constant<int, 0x128>{});  // row_ror:8
+  x = add(x, integral_constant<int, 0x124>{});  // row_ror:4
+  x = add(x, integral_constant<int, 0x122>{});  // row_ror:2
+  return add(x, integral_constant<int, 0x121>{});  // row_ror:1
 }
 
 struct AdjArgs {
@@ -192,7 +204,7 @@ struct AdjArgs {
   const AdjAxisTab* tab;             // rows, columns
 };
 
-// One reverse step of the band of R rows (even) at rs of the strip at cs: one
+// One reverse step of the band of R rows at rs of the strip at cs: one
 // wave, lane l on column cs - 5 + l, rows walked as the forward streaming tile
 // walks them: windows of u, D and the cotangent L = lu + inj in registers,
 // column neighbours by DPP, no LDS. The fields that the transposed operators
@@ -202,7 +214,7 @@ struct AdjArgs {
 // rows). It replaced a kernel that kept seven derived fields in memory (104
 // bytes by design, 121-142 measured), two threads per cell:
 // 59.1 us before, 27.6 now per step of 12 problems of 128^2 to 512^2 (1.26 M
-// cells; 167 registers, three waves per SIMD); 61 us for 3.84 M cells (3.0 TB/s of
+// cells; 161 registers, three waves per SIMD); 61 us for 3.84 M cells (3.0 TB/s of
 // the 48 bytes); 7.05 and, a wave per row, 6.2 at 256^2, where a launch and an edge
 // wave's own instructions bound both.
 // XG, YG: a row within 13 of an edge, a column within 13 of a side. In such a
@@ -211,16 +223,14 @@ struct AdjArgs {
 // tab: the wave's LDS copy of the tables, filled here where they are used (read
 // from memory one row after another they were most of an edge wave's time: a
 // dozen dependent scalar loads, 33 us in place of 29 for the 12 problems).
-// R = 1: a wave per row, the even row of a pair and the odd one next to each
-// other in a block; every wave of the block calls it (a barrier). The even row
-// passes its tau terms on through `pair` (3 x 64 floats), the odd one adds.
+// The waves of a block may run different instantiations (an edge band next to an
+// inner one), so it holds no workgroup barrier.
 template <int R, bool XG, bool YG, class SV>
 __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H, int W,
                                          const SV& sv, float dt, float inv_dx2, int rs, int cs,
-                                         AdjAxisTab* tab, float* pair = nullptr) {
+                                         AdjAxisTab* tab) {
 #pragma clang fp contract(off)
-  static_assert(R == 1 || R % 2 == 0, "tau groups are pairs of rows");
-  constexpr int P = R == 1 ? 1 : R / 2;  // pairs of rows
+  static_assert(R == 1 || R == 2 || R == 4, "the tau sums of a band");
   constexpr int E = XG ? kRevHalo : 4;  // window rows above and below the band
   constexpr int NW = R + 2 * E, NG = NW - 4;  // window; its first differences
   const int lane = threadIdx.x & 63;
@@ -255,18 +265,15 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
 #pragma unroll
     for (int k = 0; k < NW; ++k) LL[k] = LL[k] + at(a.inj, rs - E + k);
   }
-  // The tau sums of the band's row pairs (lane 63 adds to them at the end; every
-  // lane loads the same words, so that they arrive with the rest: read where they
-  // are added to, they ended the wave with a trip to memory).
-  double* gt = a.g_tau + 3 * ((size_t)(cs / kRevOut) * ((H + 1) / 2) + rs / 2);
-  double g0[3 * P];
-#pragma unroll
-  for (int p = 0; p < P; ++p)
-#pragma unroll
-    for (int f = 0; f < 3; ++f)
-      g0[3 * p + f] = !XG || (rs & ~1) + 2 * p < H
-                          ? ((const double __attribute__((address_space(1)))*)gt)[3 * p + f]
-                          : 0.0;
+  // The tau sums of the band's rows: lane 16 k + f holds sum f of row k and loads
+  // it here, so that it arrives with the rest (read where it is added to, it
+  // ended the wave with a trip to memory).
+  const int tau_row = lane >> 4, tau_f = lane & 15;
+  const bool has_tau = tau_f < 3 && tau_row < (XG ? min(R, H - rs) : R);
+  double __attribute__((address_space(1)))* gt =
+      (double __attribute__((address_space(1)))*)a.g_tau +
+      3 * ((size_t)(cs / kRevOut) * H + rs + tau_row) + tau_f;
+  const double g0 = has_tau ? *gt : 0.0;
   float vv[R], ww[R], lvv[R], lww[R], gd[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) {
@@ -320,7 +327,7 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
     q1[k] = slope(dd, m, r, true) * LL[m];
   }
 
-  float ts[3];
+  float even[3], ts[3];  // tau terms of an even row; of the rows so far, by 16 lanes
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     const int i = rs + k, m = k + E, mf = m - 2;  // row, its entries in the windows
@@ -423,33 +430,20 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
     const float t_d = (q ? -vv[k] * a1 * c.inv_td : 0.0f) * lt;
     const float t_r = (q ? c.inv_tr * c.inv_tr * c.inv_cm : 0.0f) * lt;
     const float t_si = (-ww[k] * S * c.inv_tsi * c.inv_tsi * c.inv_cm) * lt;
-    if (R == 1) {
-      if ((rs & 1) == 0) {
-        pair[lane] = t_d;
-        pair[64 + lane] = t_r;
-        pair[128 + lane] = t_si;
-      }
-      lds_barrier();
-      if ((rs & 1) == 0) return;
+    const float t[3] = {t_d, t_r, t_si};
 #pragma unroll
-      for (int f = 0; f < 3; ++f) ts[f] = pair[64 * f + lane];
-    }
-    if (R > 1 && k % 2 == 0) {
-      ts[0] = t_d;
-      ts[1] = t_r;
-      ts[2] = t_si;
-    } else {
-      const float r0 = wave_sum63(ts[0] + t_d), r1 = wave_sum63(ts[1] + t_r),
-                  r2 = wave_sum63(ts[2] + t_si);
-      if (lane == 63 && (!XG || i - 1 < H)) {
-        double __attribute__((address_space(1)))* g =
-            (double __attribute__((address_space(1)))*)gt + 3 * (k / 2);
-        g[0] = g0[3 * (k / 2)] + (double)r0;
-        g[1] = g0[3 * (k / 2) + 1] + (double)r1;
-        g[2] = g0[3 * (k / 2) + 2] + (double)r2;
+    for (int f = 0; f < 3; ++f) {
+      if (R > 1 && k % 2 == 0) {
+        even[f] = t[f];
+      } else {
+        const float p = pair_sum16(R > 1 ? even[f] : t[f], t[f]);
+        ts[f] = k == 3 ? pair_sum32(ts[f], p) : p;
       }
     }
   }
+#pragma unroll
+  for (int f = 0; f < 3; ++f) ts[f] = row_sum(R == 4 ? ts[f] : pair_sum32(ts[f], ts[f]));
+  if (has_tau) *gt = g0 + (double)(tau_f == 0 ? ts[0] : tau_f == 1 ? ts[1] : ts[2]);
 }
 
 // Up to this many bands of 2 rows a reverse step runs a wave per row: the waves
@@ -471,12 +465,12 @@ __host__ __device__ inline bool adj_edge_strip(int cs, int W) {
 template <int R, class SV>
 __device__ __forceinline__ void adj_tile_any(const Coef& c, const AdjArgs& a, int H, int W,
                                              const SV& sv, float dt, float inv_dx2, int rs, int cs,
-                                             int flags, AdjAxisTab* tab, float* pair = nullptr) {
+                                             int flags, AdjAxisTab* tab) {
   switch (flags) {
-    case 0: adj_tile<R, false, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab, pair); break;
-    case 1: adj_tile<R, true, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab, pair); break;
-    case 2: adj_tile<R, false, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab, pair); break;
-    default: adj_tile<R, true, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab, pair); break;
+    case 0: adj_tile<R, false, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
+    case 1: adj_tile<R, true, false>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
+    case 2: adj_tile<R, false, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
+    default: adj_tile<R, true, true>(c, a, H, W, sv, dt, inv_dx2, rs, cs, tab); break;
   }
 }
 

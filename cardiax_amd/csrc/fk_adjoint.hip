@@ -86,16 +86,16 @@ __global__ void __launch_bounds__(128)
 k_adj_rev_row(Coef c, AdjArgs a, int H, int W, StimArgs sa, float dt, float inv_dx2,
               int n_strips) {
   __shared__ AdjAxisTab tab[2][2];
-  __shared__ float pair[3 * 64];
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int x = blockIdx.x % kXcds, q = gridDim.x / kXcds, r = gridDim.x % kXcds;
   const int t = x * q + min(x, r) + blockIdx.x / kXcds;  // a die's pairs are neighbours
   const int band = t / n_strips;
   const int rs = 2 * band + wave, cs = kRevOut * (t - band * n_strips);
+  if (rs >= H) return;  // an odd last row; the kernel has no barrier
   const AdjStimList sv{sa};
   adj_tile_any<1>(c, a, H, W, sv, dt, inv_dx2, rs, cs,
-                  (adj_edge_band(rs, 1, H) ? 1 : 0) | (adj_edge_strip(cs, W) ? 2 : 0), tab[wave],
-                  pair);
+                  (adj_edge_band(rs, 1, H) ? 1 : 0) | (adj_edge_strip(cs, W) ? 2 : 0),
+                  tab[wave]);
 }
 
 __global__ void k_adj_zero(float* a, size_t n) {

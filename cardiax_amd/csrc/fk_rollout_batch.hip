@@ -156,19 +156,18 @@ __device__ __forceinline__ const float* roll_inject(const RollDesc& S, int j, in
 }
 
 // Reverse of step c + k of segment `seg` (j = c + k + 1): cotangent set `cur`
-// (0 lam, 1 lam_alt) -> the other; x_j's frame cotangent enters first. R = 1: a
-// pair of rows per block of two waves.
+// (0 lam, 1 lam_alt) -> the other; x_j's frame cotangent enters first. R = 1: two
+// rows per block.
 template <int R>
 __global__ void __launch_bounds__(R == 1 ? 128 : 256)
 k_roll_rev(const RollDesc* __restrict__ sims, const RollTile* __restrict__ items, int n_items,
            const uint32_t* __restrict__ masks, int seg, int k, int j, int fe, int cur) {
   constexpr int kWaves = R == 1 ? 2 : 4;
   __shared__ AdjAxisTab tab[kWaves][2];
-  __shared__ float pair[R == 1 ? 3 * 64 : 1];
   const int it = __builtin_amdgcn_readfirstlane(blockIdx.x * kWaves + (int)(threadIdx.x >> 6));
   if (it >= n_items) return;
   RollTile item = items[it];
-  if (uni(item.sim) < 0) return;  // padding of the XCD order (of whole pairs)
+  if (uni(item.sim) < 0) return;  // padding of the XCD order
   item.sim = uni(item.sim);
   const RollDesc& S = sims[item.sim];
   const size_t n = S.cells;
@@ -188,7 +187,7 @@ k_roll_rev(const RollDesc* __restrict__ sims, const RollTile* __restrict__ items
   c.inv_t0 = uni(c.inv_t0); c.inv_tr = uni(c.inv_tr); c.inv_tsi = uni(c.inv_tsi);
   c.inv_cm = uni(c.inv_cm);
   adj_tile_any<R>(c, a, uni(S.H), uni(S.W), sv, uni(S.dt), uni(S.inv_dx2), uni(item.rs),
-                  uni(item.cs), uni(item.flags), tab[threadIdx.x >> 6], pair);
+                  uni(item.cs), uni(item.flags), tab[threadIdx.x >> 6]);
 }
 
 }  // namespace fk
@@ -297,7 +296,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
       default: append_block_items<Block32x2>(i, s.H, s.W, blocks); break;
     }
     for (int strip = 0; strip < adj_strips(s.W); ++strip)
-      for (int band = 0; band < (rows == 1 ? (s.H + 1) / 2 * 2 : (s.H + rows - 1) / rows); ++band) {
+      for (int band = 0; band < (s.H + rows - 1) / rows; ++band) {
         RollTile t;
         t.sim = i;
         t.cs = kRevOut * strip;
