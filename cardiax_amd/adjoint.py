@@ -4,9 +4,10 @@ frames with respect to the diffusivity map D and tau_d, tau_r, tau_si.
 ``rollout(...)`` runs cardiax/solve.py:92-100 on the GPU and returns the u
 fields after every ``frame_every`` steps. Its backward pass is the
 hand-written adjoint of the Euler step over the states of the forward pass.
-Those are kept when they take at most KEEP_BYTES, a small part of the GPU's
-memory (256 x 256 over 2000 steps: 1.6 GB, and 4.7 of 23.6 ms less than
-recomputing them). Longer or larger rollouts, and those that set
+Those are kept while all rollouts that await their backward pass keep at most
+KEEP_BYTES, a small part of the GPU's memory (256 x 256 over 2000 steps: 1.6 GB,
+and 4.7 of 23.6 ms less than recomputing them); they are given back with the
+graph. Longer or larger rollouts, and those that set
 ``checkpoint_every``, recompute them segment by segment from checkpoints every
 ~sqrt(N) steps (fk_forward_trajectory): O(sqrt(N)) states instead of N. Each
 segment is reversed by one fk_adjoint_segment call. Gates are fixed masks and the
@@ -17,17 +18,22 @@ from __future__ import annotations
 
 import ctypes
 import math
+import threading
 from typing import Sequence
 
 import torch
+from torch.multiprocessing.reductions import StorageWeakRef
 
 from . import _lib
 from ._device import on_device, require_gpu, stream_handle
 from .params import Params
 from .solve import State, _Stimuli, _scalar
 
-# Bytes of states that rollout keeps for its backward pass instead of recomputing them.
+# Bytes of states that the rollouts of one GPU keep for their backward passes instead of
+# recomputing them, over all whose backward pass is still to come.
 KEEP_BYTES = 4 << 30
+_kept: list = []  # (device, reference to the storage, bytes) of the kept states
+_kept_lock = threading.Lock()
 
 # Params fields that carry gradients, in the order of the returned gradients.
 GRAD_FIELDS = ("tau_d", "tau_r", "tau_si")
@@ -36,6 +42,22 @@ GRAD_FIELDS = ("tau_d", "tau_r", "tau_si")
 def _with_taus(params, tau_d, tau_r, tau_si) -> Params:
     p = Params(*[float(x) for x in params])
     return p._replace(tau_d=float(tau_d), tau_r=float(tau_r), tau_si=float(tau_si))
+
+
+def _keep_states(n: int, H: int, W: int, dev):
+    """Memory for the n + 1 states of a rollout, or None when it would take the
+    states kept at this time above KEEP_BYTES or the GPU has no room."""
+    nbytes = 12 * (n + 1) * H * W
+    with _kept_lock:
+        _kept[:] = [k for k in _kept if not k[1].expired()]
+        if nbytes + sum(b for d, _, b in _kept if d == dev) > KEEP_BYTES:
+            return None
+        try:
+            states = torch.empty((n + 1, 3, H, W), dtype=torch.float32, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            return None  # checkpoints take a fraction
+        _kept.append((dev, StorageWeakRef(states.untyped_storage()), nbytes))
+        return states
 
 
 class _Rollout(torch.autograd.Function):
@@ -57,23 +79,20 @@ class _Rollout(torch.autograd.Function):
         ctx.cfg = cfg
         ctx.prm = prm
         ctx.S = S
-        ctx.states = None
+        states = _keep_states(n, H, W, dev) if cfg["keep"] else None
+        if states is not None:
+            for f in range(3):
+                states[0, f].copy_(st[f])
+            if n > 0:
+                _lib.check(L.fk_forward_trajectory(
+                    ctypes.byref(p), D.data_ptr(), *(x.data_ptr() for x in states[0]), H, W,
+                    stim.pointer(), stim.n, float(t0), n, float(cfg["dt"]),
+                    float(cfg["dx"]), states[1:].data_ptr(), s))
+            ctx.S, ctx.ckpts = n, {0: st} if n else {}
+            # saved, not an attribute: released by the backward pass
+            ctx.save_for_backward(D, states)
+            return states[fe::fe, 2].clone(memory_format=torch.contiguous_format)
         ctx.save_for_backward(D)
-        if cfg["grad"] and cfg["checkpoint_every"] is None and 12 * (n + 1) * H * W <= KEEP_BYTES:
-            try:
-                states = torch.empty((n + 1, 3, H, W), dtype=torch.float32, device=dev)
-            except torch.cuda.OutOfMemoryError:
-                states = None  # checkpoints take a fraction
-            if states is not None:
-                for f in range(3):
-                    states[0, f].copy_(st[f])
-                if n > 0:
-                    _lib.check(L.fk_forward_trajectory(
-                        ctypes.byref(p), D.data_ptr(), *(x.data_ptr() for x in states[0]), H, W,
-                        stim.pointer(), stim.n, float(t0), n, float(cfg["dt"]),
-                        float(cfg["dx"]), states[1:].data_ptr(), s))
-                ctx.S, ctx.states, ctx.ckpts = n, states, {0: st} if n else {}
-                return states[fe::fe, 2].clone(memory_format=torch.contiguous_format)
         frames = torch.empty((n // fe, H, W), dtype=torch.float32, device=dev)
         # Each checkpoint interval runs through fk_forward_trajectory, the call
         # the backward pass uses to recompute it, so the backward linearises
@@ -100,7 +119,7 @@ class _Rollout(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_frames):
-        (D,) = ctx.saved_tensors
+        D, *kept = ctx.saved_tensors
         cfg, prm, S = ctx.cfg, ctx.prm, ctx.S
         dev = D.device
         H, W = D.shape
@@ -116,17 +135,18 @@ class _Rollout(torch.autograd.Function):
         lam = [torch.zeros((H, W), dtype=torch.float32, device=dev) for _ in range(3)]
         gD = torch.zeros((H, W), dtype=torch.float32, device=dev)
         # states x_c .. x_{e-1} of one segment, (v, w, u) planes per state
-        states = ctx.states
-        if states is None:
+        if kept:
+            states = kept[0]
+        else:
             states = torch.empty((S, 3, H, W), dtype=torch.float32, device=dev)
         for c in sorted(ctx.ckpts, reverse=True):
             e = min(n, c + S)
             x = ctx.ckpts[c]
-            if ctx.states is None:
+            if not kept:
                 states[0, 0].copy_(x.v)
                 states[0, 1].copy_(x.w)
                 states[0, 2].copy_(x.u)
-            if ctx.states is None and e - c > 1:  # recompute x_{c+1} .. x_{e-1}
+            if not kept and e - c > 1:  # recompute x_{c+1} .. x_{e-1}
                 _lib.check(L.fk_forward_trajectory(
                     ctypes.byref(p), D.data_ptr(), x.v.data_ptr(), x.w.data_ptr(),
                     x.u.data_ptr(), H, W, stim.pointer(), stim.n, float(t0 + c), e - c - 1,
@@ -178,7 +198,12 @@ def rollout(D: torch.Tensor, tau_d, tau_r, tau_si, state0, params, stimuli: Sequ
            "t0": _scalar(t0), "n_steps": int(n_steps), "frame_every": int(frame_every),
            "dt": float(dt), "dx": float(dx), "checkpoint_every": checkpoint_every,
            "tau_host": host,
-           "grad": torch.is_grad_enabled() and any(x.requires_grad for x in [D] + taus)}
+           # under saved-tensor hooks (offloading, torch.utils.checkpoint) the states are
+           # recomputed: the caller is short of memory, and a second forward has to save
+           # the same tensors as the first
+           "keep": checkpoint_every is None and torch.is_grad_enabled()
+           and any(x.requires_grad for x in [D] + taus)
+           and torch._C._autograd._top_saved_tensors_default_hooks(True) is None}
     return _Rollout.apply(D, taus[0], taus[1], taus[2], cfg)
 
 
