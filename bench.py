@@ -471,7 +471,8 @@ def bench_slab(seed, n_steps, size=1024, n_parts=8, depths=(1, 4, 8), tune=True)
         D = torch.from_numpy(np.ascontiguousarray(sim.D[r0:r1])).to(dev)
         stims = [(s.protocol, torch.from_numpy(np.ascontiguousarray(s.field[r0:r1])).to(dev))
                  for s in sim.stimuli]
-        variant = autotune.tune(shape, n_steps=300)["best"] if tune else autotune.resolved(shape)
+        variant = (autotune.tune(shape, n_steps=300)["best"] if tune
+                   else autotune.solve_variant(shape))
         st0 = solve.init(shape)
         solve._forward_euler(st0, 0, 200, sim.params, D, stims, sim.dt, sim.dx)  # warm-up
         torch.cuda.synchronize()
@@ -703,7 +704,7 @@ def main():
         tuned["state_at_step"] = t_mid
         del mid
         log("autotune %dx%d: %s" % (H, W, json.dumps(tuned)))
-    variant = autotune.resolved((H, W))
+    variant = autotune.solve_variant((H, W))
 
     def run():
         return solve._forward_euler(st0, sim.t0, sim.t1, sim.params, D, stims, sim.dt, sim.dx)

@@ -84,6 +84,8 @@ _SIGNATURES = {
                                           ctypes.POINTER(c_i32)]),
     "fk_autotune_lookup": (c_i32, [c_i32, c_i32]),
     "fk_forward_variant_for": (c_i32, [c_i32, c_i32]),
+    "fk_solve_variant_for": (c_i32, [c_i32, c_i32]),
+    "fk_step_variant_for": (c_i32, [c_i32, c_i32]),
     "fk_autotune_reset": (None, []),
     "fk_init": (c_i32, [c_vp, c_vp, c_vp, c_i64, c_vp]),
     "fk_check_finite": (c_i32, [ctypes.POINTER(c_vp), c_i32, c_i64, c_vp, c_vp]),

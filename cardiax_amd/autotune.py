@@ -66,14 +66,32 @@ def lookup(shape) -> str:
     return NAMES[int(_lib.lib().fk_autotune_lookup(H, W))]
 
 
-def resolved(shape) -> str:
-    """Name of the variant that forward solves of ``shape`` run now: the
-    process-wide setting, else the tuned one, else the size-based default."""
+def _name_of(query, shape) -> str:
     H, W = (int(x) for x in shape)
-    v = int(_lib.lib().fk_forward_variant_for(H, W))
+    v = int(query(H, W))
     if v < 0:
         _lib.check(v)
     return NAMES[v]
+
+
+def resolved(shape) -> str:
+    """Name of the variant set for ``shape``: the process-wide setting, else the
+    tuned one, else the size-based default of single steps. Where other kernels
+    of the same bits run in its place, ``solve_variant`` and ``step_variant``
+    name them."""
+    return _name_of(_lib.lib().fk_forward_variant_for, shape)
+
+
+def solve_variant(shape) -> str:
+    """Name of the variant whose kernel forward solves of several steps on
+    ``shape`` run now."""
+    return _name_of(_lib.lib().fk_solve_variant_for, shape)
+
+
+def step_variant(shape) -> str:
+    """Name of the variant whose kernel single steps (``solve.step``,
+    ``solve.step_euler``) on ``shape`` run now."""
+    return _name_of(_lib.lib().fk_step_variant_for, shape)
 
 
 def reset() -> None:

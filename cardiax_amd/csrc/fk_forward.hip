@@ -410,8 +410,6 @@ static int default_variant(int H, int W) {
   if (stream_t_fits<16>(H, W)) return kStreamT16;
   return n <= 8 * 1024 * 1024 ? (int)kStream4 : (int)kTile16;
 }
-static int resolve_variant(int v) { return v == kAuto ? (int)kStream2 : v; }
-
 // The variant an automatic solve of several steps runs when the shape was not
 // tuned: block tiles, which equal the streaming kernels of default_variant bit
 // for bit, in the tiling that LeastRounds finds. Against the best streaming
@@ -429,18 +427,32 @@ static int auto_variant(int H, int W) {
   return r.best;
 }
 
-// The variant of a solve of several steps.
-static int resolve_solve(int v, int H, int W) {
-  if (v != kAuto) return v;
-  const int t = tuned_variant(H, W);
-  return t != kAuto ? t : auto_variant(H, W);
+// The variant whose kernel a grid takes in place of v.
+static int on_grid(int v, int H, int W) {
+  if (W % 2 && v == kPair2) return kStream2;
+  if (W % 2 && v == kPair4) return kStream4;
+  if (is_two_step(v) && !two_step_fits(v, H, W)) return kStream2;
+  return v;
 }
 
-// The variant an automatic launch of one step on an H x W grid uses.
+// The variant of a solve of several steps.
+static int resolve_solve(int v, int H, int W) {
+  if (v == kAuto) v = tuned_variant(H, W);
+  return on_grid(v != kAuto ? v : auto_variant(H, W), H, W);
+}
+
+// The setting, else the tuned variant, else the streaming default.
 static int resolve_for(int v, int H, int W) {
-  if (v != kAuto) return v;
-  const int t = tuned_variant(H, W);
-  return t != kAuto ? t : default_variant(H, W);
+  if (v == kAuto) v = tuned_variant(H, W);
+  return on_grid(v != kAuto ? v : default_variant(H, W), H, W);
+}
+
+// The one-step variant that runs a single step in place of v.
+static int step_variant(int v) {
+  if (is_pc(v)) return pc_base(v);  // no coefficient precompute to amortise
+  if (is_two_step(v)) return kStream2;
+  if (is_block(v)) return kStream8;
+  return v;
 }
 
 template <int R>
@@ -503,7 +515,7 @@ static hipError_t launch_step(int variant, bool euler, const Coef& c, const floa
                               const float* v, const float* w, const float* u, int H, int W,
                               const StimArgs& sa, float dt, float inv_dx2, float* ov,
                               float* ow, float* ou, hipStream_t s) {
-  switch (resolve_variant(variant)) {
+  switch (step_variant(on_grid(variant, H, W))) {
     case kPlain: {
       const dim3 block(64, 4), grid((W + 63) / 64, (H + 3) / 4);
       if (euler)
@@ -516,24 +528,11 @@ static hipError_t launch_step(int variant, bool euler, const Coef& c, const floa
     case kTile16: launch_tile<16>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
     case kTile32: launch_tile<32>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
     case kStream32: launch_stream<32>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
-    case kStreamC16:  // single steps: no coefficient precompute to amortise
     case kStream16: launch_stream<16>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
-    case kStreamC4:
     case kStream4: launch_stream<4>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
-    case kStreamC2:
     case kStream2: launch_stream<2>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
-    case kPair2:
-      if (W % 2 == 0) launch_stream2<2>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s);
-      else launch_stream<2>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s);
-      break;
-    case kPair4:
-      if (W % 2 == 0) launch_stream2<4>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s);
-      else launch_stream<4>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s);
-      break;
-    case kStreamT8:  // single steps of the two-step variants: the 2-row bands
-    case kStreamT12:
-    case kStreamT16:
-    case kStreamT24: launch_stream<2>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
+    case kPair2: launch_stream2<2>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
+    case kPair4: launch_stream2<4>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
     case kStream8:
     default: launch_stream<8>(euler, c, D, v, w, u, H, W, sa, dt, inv_dx2, ov, ow, ou, s); break;
   }
@@ -673,7 +672,6 @@ int32_t forward_loop(int variant, const fk_params* params, const float* D, const
   int v = resolve_solve(variant, H, W);
   // nothing to amortise, or no room for the coefficients
   if (is_pc(v) && (steps < 2 || state_only)) v = pc_base(v);
-  if (is_two_step(v) && !two_step_fits(v, H, W)) v = kStream2;
   float4* cf = nullptr;
   if (is_pc(v)) {
     cf = (float4*)((char*)work + coef_offset(H, W));
@@ -822,7 +820,7 @@ using namespace fk;
 
 extern "C" {
 
-int32_t fk_abi_version(void) { return 3; }
+int32_t fk_abi_version(void) { return 4; }
 
 int32_t fk_set_forward_variant(int32_t variant) {
   ErrorScope es;
@@ -1000,11 +998,19 @@ void fk_autotune_reset(void) {
 int32_t fk_forward_variant_for(int32_t H, int32_t W) {
   ErrorScope es;
   if (H < 3 || W < 3) return set_error(FK_ERR_ARG, "grid %d x %d: H, W must be >= 3", H, W);
-  const int v = resolve_for(g_variant.load(), H, W);
-  if (W % 2 && v == kPair2) return kStream2;
-  if (W % 2 && v == kPair4) return kStream4;
-  if (is_two_step(v) && !two_step_fits(v, H, W)) return kStream2;
-  return v;
+  return resolve_for(g_variant.load(), H, W);
+}
+
+int32_t fk_solve_variant_for(int32_t H, int32_t W) {
+  ErrorScope es;
+  if (!check_grid(H, W)) return last_code();
+  return resolve_solve(g_variant.load(), H, W);
+}
+
+int32_t fk_step_variant_for(int32_t H, int32_t W) {
+  ErrorScope es;
+  if (!check_grid(H, W)) return last_code();
+  return step_variant(resolve_for(g_variant.load(), H, W));
 }
 
 int32_t fk_forward_trajectory(const fk_params* params, const float* D, const float* v0,

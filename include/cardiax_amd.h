@@ -132,12 +132,23 @@ int32_t fk_autotune_lookup(int32_t H, int32_t W);
 /* Forgets every tuned shape. */
 void fk_autotune_reset(void);
 
-/* The variant fk_forward_euler runs on an H x W grid under the current
- * setting: the fk_set_forward_variant choice when it is not 0, else the tuned
- * one, else the single-step default listed there (whose bits the block tiles of
- * an automatic solve reproduce); 17 / 18 on an odd W report the 15 / 13 they
- * run. No reference counterpart. FK_ERR_ARG for H or W below 3. */
+/* The current setting on an H x W grid: the fk_set_forward_variant choice when
+ * it is not 0, else the tuned variant, else the default that is listed there
+ * for single steps; 17 / 18 on an odd W report 15 / 13, and 19-22 on a grid too
+ * small for them 15. Solves and single steps that run another kernel of the
+ * same bits in its place are reported by the two calls below. No reference
+ * counterpart. FK_ERR_ARG for H or W below 3. */
 int32_t fk_forward_variant_for(int32_t H, int32_t W);
+
+/* The variant whose kernel fk_forward_euler runs on an H x W grid now over
+ * several steps (a single last step of 7-10 and 19-22 runs 15).
+ * fk_forward_trajectory runs the same of 7-10, and the one-step kernel of any
+ * other. No reference counterpart. FK_ERR_ARG for a grid that a solve refuses. */
+int32_t fk_solve_variant_for(int32_t H, int32_t W);
+
+/* The variant whose kernel fk_step and fk_step_euler run on an H x W grid now.
+ * No reference counterpart. FK_ERR_ARG for a grid that they refuse. */
+int32_t fk_step_variant_for(int32_t H, int32_t W);
 
 /* cardiax/solve.py:18-23 -- v = w = 1, u = 0 over n_cells cells. */
 int32_t fk_init(float* v, float* w, float* u, int64_t n_cells, void* stream);

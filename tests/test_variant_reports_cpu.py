@@ -1,0 +1,50 @@
+"""Host logic only: the kernel that a solve of several steps and a single step of
+a shape run, as the library reports it. The launches take the same functions."""
+import pytest
+
+from cardiax_amd import _lib, autotune
+
+BLOCKS = ("tb64x2", "tb64x4", "tb32x2", "tb32x4")
+
+
+@pytest.fixture
+def variant():
+    L = _lib.lib()
+    prev = L.fk_set_forward_variant(0)
+    yield lambda name: L.fk_set_forward_variant(_lib.VARIANTS[name])
+    L.fk_set_forward_variant(prev)
+
+
+@pytest.mark.parametrize("shape,solve", [
+    ((3, 3), "tb32x4"), ((128, 128), "tb32x4"),       # 32 rows, 4 steps
+    ((500, 500), "tb64x4"), ((4096, 4096), "tb64x4"),  # 48 rows, 3 steps
+    ((700, 600), "tb32x2"),                            # 64 rows, 3 steps
+    ((2048, 2048), "tb64x2"),                          # 32 rows, 2 steps
+    ((100000, 100), "tile16")])
+def test_automatic_solves(variant, shape, solve):
+    assert autotune.solve_variant(shape) == solve
+
+
+@pytest.mark.parametrize("name,shape,solve,step", [
+    ("auto", (1024, 1024), None, "stream2"), ("auto", (2048, 2048), None, "stream2"),
+    ("auto", (40000, 100), None, "stream4"), ("auto", (100000, 100), "tile16", "tile16"),
+    ("stream16", (64, 64), "stream16", "stream16"),
+    ("streamc8", (64, 64), "streamc8", "stream8"), ("streamc2", (64, 64), "streamc2", "stream2"),
+    ("pair2", (64, 64), "pair2", "pair2"), ("pair2", (64, 63), "stream2", "stream2"),
+    ("pair4", (64, 63), "stream4", "stream4"),
+    ("streamt12", (1024, 1024), "streamt12", "stream2"),
+    ("streamt12", (39, 1024), "stream2", "stream2")])
+def test_solves_and_single_steps(variant, name, shape, solve, step):
+    variant(name)
+    if solve is None:
+        assert autotune.solve_variant(shape) in BLOCKS
+    else:
+        assert autotune.solve_variant(shape) == solve
+    assert autotune.step_variant(shape) == step
+
+
+def test_refused_grids(variant):
+    for query in (autotune.solve_variant, autotune.step_variant):
+        for shape in ((2, 64), (64, 2), ((1 << 18) + 1, 64)):
+            with pytest.raises(ValueError):
+                query(shape)
