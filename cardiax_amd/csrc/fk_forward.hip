@@ -447,11 +447,13 @@ static int resolve_for(int v, int H, int W) {
   return on_grid(v != kAuto ? v : default_variant(H, W), H, W);
 }
 
-// The one-step variant that runs a single step in place of v.
+// The one-step variant that runs a single step in place of v. Of the variants
+// with several steps per launch that is the 2-row bands, the single step of an
+// untuned shape too (1024^2 6.7 us a step and 9.2 with 8-row bands, 2048^2 24.0
+// and 31.7).
 static int step_variant(int v) {
   if (is_pc(v)) return pc_base(v);  // no coefficient precompute to amortise
-  if (is_two_step(v)) return kStream2;
-  if (is_block(v)) return kStream8;
+  if (is_two_step(v) || is_block(v)) return kStream2;
   return v;
 }
 
@@ -1048,9 +1050,8 @@ int32_t fk_forward_trajectory(const fk_params* params, const float* D, const flo
       k += ns;
       continue;
     }
-    HIP_CHECK(launch_step(is_block(v) ? (int)kStream2 : v, true, c, D, src[0], src[1], src[2], H,
-                          W, sched.at(t + (double)k), dt, inv_dx2, d, d + n, d + 2 * n,
-                          (hipStream_t)stream));
+    HIP_CHECK(launch_step(v, true, c, D, src[0], src[1], src[2], H, W, sched.at(t + (double)k),
+                          dt, inv_dx2, d, d + n, d + 2 * n, (hipStream_t)stream));
     src[0] = d;
     src[1] = d + n;
     src[2] = d + 2 * n;

@@ -94,8 +94,8 @@ int32_t fk_abi_version(void);
  *    19-22  two Euler steps per launch on streaming bands of 8 / 12 / 16 / 24
  *           rows, bit-identical to two steps of 15 (grids below 2R + 16 rows
  *           or 112 columns run 15; an odd last step runs 15)
- * fk_step and fk_step_euler run 4 in place of 7-11, 5 in place of 12, 13 in
- * place of 14 and 15 in place of 16 and 19-22. */
+ * fk_step and fk_step_euler run 4 in place of 11, 5 in place of 12, 13 in place
+ * of 14 and 15 in place of 7-10, 16 and 19-22. */
 int32_t fk_set_forward_variant(int32_t variant);
 
 /* Autotuner of the forward step kernel. No reference counterpart (the

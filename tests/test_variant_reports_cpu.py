@@ -48,3 +48,12 @@ def test_refused_grids(variant):
         for shape in ((2, 64), (64, 2), ((1 << 18) + 1, 64)):
             with pytest.raises(ValueError):
                 query(shape)
+
+
+@pytest.mark.parametrize("name", BLOCKS)
+def test_single_steps_of_block_variants(variant, name):
+    """A shape whose tuned solve runs block tiles takes the 2-row bands for single
+    steps, as the last step of such a solve does."""
+    variant(name)
+    assert autotune.solve_variant((1024, 1024)) == name
+    assert autotune.step_variant((1024, 1024)) == "stream2"
