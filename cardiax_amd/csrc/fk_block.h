@@ -470,7 +470,7 @@ __device__ __forceinline__ BlockPlace block_place(int b, const BlockOrder& o, co
   const int last = o.per_xcd - (x < o.extra ? 0 : 1);
   const int t = x * o.per_xcd + min(x, o.extra) + (o.back ? last - k : k);
   const int per = kBlockGroup * ca.n;
-  // t / per: the float quotient is within one of it (t < 2^24)
+  // t / per: the float quotient is within one of it (below 2^15, t below 2^24)
   int g = __builtin_amdgcn_readfirstlane((int)((float)t * o.inv_group));
   g -= g * per > t;
   g += (g + 1) * per <= t;

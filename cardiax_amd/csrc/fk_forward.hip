@@ -427,8 +427,11 @@ static int auto_variant(int H, int W) {
   return r.best;
 }
 
-// The variant whose kernel a grid takes in place of v.
+// The variant whose kernel a grid takes in place of v. A launch holds fewer than
+// 2^32 threads: 32 rows and 4 steps take 4 per cell (48 rows and 3 steps 0.6).
 static int on_grid(int v, int H, int W) {
+  if (v == kBlock32x4 && block_tiles<Block32x4>(H, W) * (Block32x4::waves * 64) > UINT32_MAX)
+    return kBlock48x3;
   if (W % 2 && v == kPair2) return kStream2;
   if (W % 2 && v == kPair4) return kStream4;
   if (is_two_step(v) && !two_step_fits(v, H, W)) return kStream2;

@@ -84,7 +84,8 @@ int32_t fk_abi_version(void);
  *    4-6    streaming wavefront bands of 8 / 16 / 32 rows
  *    7-10   temporal blocking: tiles of 64 columns by 32 rows with 2 steps per
  *           launch, 48 rows with 3, 64 rows with 3 and 32 rows with 4,
- *           bit-identical to as many steps of 15 (a single last step runs 15)
+ *           bit-identical to as many steps of 15 (a single last step runs 15;
+ *           above about 1e9 cells 8 runs in place of 10)
  *    11, 12 streaming bands of 8 / 16 rows with the static diffusion
  *           coefficients precomputed once per fk_forward_euler call
  *    13, 15 streaming bands of 4 / 2 rows

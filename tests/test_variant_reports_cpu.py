@@ -57,3 +57,12 @@ def test_single_steps_of_block_variants(variant, name):
     variant(name)
     assert autotune.solve_variant((1024, 1024)) == name
     assert autotune.step_variant((1024, 1024)) == "stream2"
+
+
+def test_a_launch_stays_below_2_32_threads(variant):
+    """1024 threads per 8 x 32 cells of a 32-row tile of 4 steps: above 1.07e9 cells
+    they would exceed what a launch may hold."""
+    variant("tb32x4")
+    assert autotune.solve_variant((32768, 32000)) == "tb32x4"  # 4.19e9 threads
+    assert autotune.solve_variant((32768, 33000)) == "tb64x4"
+    assert autotune.solve_variant((1 << 18, 8192)) == "tb64x4"
