@@ -170,6 +170,7 @@ def bench_batched(n_sims, n_steps, seed, per_sim_steps=64):
     with Batch(bs) as b:
         tuned = b.autotune(32)
         log("batch autotune: %s" % json.dumps(tuned))
+        option, per_launch = b.option, b.steps_per_launch
         b.run(64)  # warm-up: records the graph
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -179,13 +180,10 @@ def bench_batched(n_sims, n_steps, seed, per_sim_steps=64):
         n_bad = sum(int(not bool(torch.isfinite(x.u).all().item())) for x in b.states)
         umax = max(float(x.u.abs().max().item()) for x in b.states)
     batched = cells * n_steps / el / 1e9
-    # the tuned work list: one Euler step per launch, or block tiles of 32 rows (2 steps, for
-    # a batch this size) or 48 rows (3)
-    per_launch = 1
-    kernel = "k_batch_step<%d>" % tuned["rows"]
-    if tuned["two_step"]:
-        per_launch, kernel = {8: (2, "k_batch_block<4, 8, 2>"),
-                              16: (3, "k_batch_block<4, 12, 3>")}[tuned["rows"]]
+    # the work list in use: one Euler step per launch, or block tiles of 32 rows (4 steps, 2
+    # for a batch of many tiles) or 48 rows (3)
+    kernel = {4: "k_batch_block<2, 16, 4>", 3: "k_batch_block<4, 12, 3>",
+              2: "k_batch_block<4, 8, 2>", 1: "k_batch_step<%s>" % option}[per_launch]
     # per-simulation launches: the same simulations, one call each
     for x in bs[:4]:
         solve._forward_euler(x.state, 0, 4, x.params, x.diffusivity, x.stimuli, x.dt, x.dx)

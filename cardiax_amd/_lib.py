@@ -150,6 +150,7 @@ _SIGNATURES = {
     "fk_batch_autotune": (c_i32, [c_vp, c_i32, c_vp, ctypes.POINTER(c_f),
                                   ctypes.POINTER(c_i32)]),
     "fk_batch_set_rows": (c_i32, [c_vp, c_i32]),
+    "fk_batch_option": (c_i32, [c_vp, ctypes.POINTER(c_i32)]),
     "fk_batch_n_items": (c_i32, [c_vp]),
     "fk_batch_destroy": (c_i32, [c_vp]),
 }

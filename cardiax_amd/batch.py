@@ -96,15 +96,35 @@ class Batch:
     def n_tiles(self) -> int:
         return int(_lib.lib().fk_batch_n_items(self._h))
 
+    def _option(self):
+        if self._h is None:
+            raise RuntimeError("batch is closed")
+        steps = ctypes.c_int32(0)
+        r = int(_lib.lib().fk_batch_option(self._h, ctypes.byref(steps)))
+        if r < 0:
+            _lib.check(r)
+        two = r & _lib.FK_BATCH_TWO_STEP
+        return ("t" if two else "") + str(r & ~_lib.FK_BATCH_TWO_STEP), int(steps.value)
+
+    @property
+    def option(self) -> str:
+        """The work-list option in use: "2", "4", "8", "16", "t8" or "t16"."""
+        return self._option()[0]
+
+    @property
+    def steps_per_launch(self) -> int:
+        """Euler steps that one launch advances the batch with that option."""
+        return self._option()[1]
+
     def autotune(self, n_steps: int = 64) -> dict:
         """Time every available work-list option (bands of 2, 4, 8 or 16 rows
         advanced one step per launch; block tiles of 32 or 48 rows, "t8" and
         "t16", advanced 2 to 4 steps per launch when every simulation fits) and
-        keep the fastest for later
-        runs (fk_batch_autotune); the simulations' states are not touched.
-        Returns ``{"rows": R, "two_step": bool, "times_ms": {option: ms}}``
-        with options "2", "4", "8", "16", "t8", "t16" (unavailable ones left
-        out)."""
+        keep the fastest for later runs (fk_batch_autotune); the simulations'
+        states are not touched. Returns ``{"rows": R, "two_step": bool,
+        "times_ms": {option: ms}, "option": name}``: the fastest of the options
+        that ``set_rows`` takes, the times of those, and the option left in use,
+        which may be faster block tiles that the sizes rule out there."""
         if self._h is None:
             raise RuntimeError("batch is closed")
         times = (ctypes.c_float * _lib.FK_BATCH_N_OPTIONS)()
@@ -115,7 +135,8 @@ class Batch:
         return {"rows": r & ~_lib.FK_BATCH_TWO_STEP,
                 "two_step": bool(r & _lib.FK_BATCH_TWO_STEP),
                 "times_ms": {name: round(float(t), 4)
-                             for name, t in zip(BATCH_OPTIONS, times) if t >= 0}}
+                             for name, t in zip(BATCH_OPTIONS, times) if t >= 0},
+                "option": self.option}
 
     def set_rows(self, rows: int, two_step: bool = False) -> None:
         """Pin the work-list option of later runs (fk_batch_set_rows): a band

@@ -400,6 +400,13 @@ int32_t fk_batch_destroy(fk_batch* b) {
 
 int32_t fk_batch_n_items(const fk_batch* b) { return b ? b->n_items_opt[b->opt] : 0; }
 
+int32_t fk_batch_option(const fk_batch* b, int32_t* steps_per_launch) {
+  ErrorScope es;
+  if (b == nullptr) return set_error(FK_ERR_ARG, "batch is null");
+  if (steps_per_launch) *steps_per_launch = batch_steps(b->block[b->opt]);
+  return kBatchRows[b->opt] | (kBatchTwo[b->opt] ? FK_BATCH_TWO_STEP : 0);
+}
+
 // Stimulus masks of the next n_rel (<= kGraphSteps) steps from the counter.
 static hipError_t batch_masks(fk_batch* b, int n_rel, hipStream_t s) {
   const int total = b->n_sims * n_rel;

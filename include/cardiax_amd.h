@@ -374,7 +374,7 @@ int32_t fk_batch_run(fk_batch* b, int64_t n_steps, int32_t use_graph, void* stre
  * state. times_ms (FK_BATCH_N_OPTIONS floats in the order 2, 4, 8, 16 rows,
  * then the two of FK_BATCH_TWO_STEP; -1 for one that is not offered; may be
  * NULL) and best_rows (may be NULL) receive the timings and the fastest option
- * offered. */
+ * offered; fk_batch_option tells the one left in use. */
 int32_t fk_batch_autotune(fk_batch* b, int32_t n_steps, void* stream, float* times_ms,
                           int32_t* best_rows);
 
@@ -384,7 +384,13 @@ int32_t fk_batch_autotune(fk_batch* b, int32_t n_steps, void* stream, float* tim
  * launch); waits for the device first. */
 int32_t fk_batch_set_rows(fk_batch* b, int32_t rows);
 
-/* Number of (simulation, strip, band) tiles of one batch step. */
+/* The work-list option that fk_batch_run uses now, as fk_batch_set_rows names
+ * it, and in steps_per_launch (may be NULL) the Euler steps of one of its
+ * launches. An untuned batch, and one whose tuner found nothing faster, may be
+ * on block tiles that the size rule does not offer. FK_ERR_ARG for NULL. */
+int32_t fk_batch_option(const fk_batch* b, int32_t* steps_per_launch);
+
+/* Number of tiles of one launch over the batch. */
 int32_t fk_batch_n_items(const fk_batch* b);
 
 /* Waits for the device and releases the batch. */
