@@ -53,16 +53,18 @@ __device__ __forceinline__ bool inside_polygon(const double* __restrict__ rp,
   return in;
 }
 
-// One wave per image row. An edge's part of the test at row y is the column
-// where the edge crosses y, the same for every pixel of the row: the wave
-// collects a polygon's crossings once (a ballot per 64 edges), and a pixel is
-// inside when an odd number of them lie to its right. A pixel then costs a
-// comparison per crossing (two to six on the generator's contours) instead of
-// one per vertex: 47 us before, 18 us now for 5 contours of 101 vertices at
-// 1200 x 1200. A polygon with more crossings than the list has room for is
+// One wave per row and kRasterCols columns of it. An edge's part of the test at
+// row y is the column where the edge crosses y, the same for every pixel of the
+// row: the wave collects a polygon's crossings once (a ballot per 64 edges), and a
+// pixel is inside when an odd number of them lie to its right. A pixel then costs
+// a comparison per crossing (two to six on the generator's contours) instead of
+// one per vertex: 47 us before, 13 us now for 5 contours of 101 vertices at
+// 1200 x 1200. Columns per wave: 64 take 27 us there, 128 18, 512 14, and a
+// whole row 19 (and 4 x 100000 up to 800, where 256 take 10). A polygon with more crossings than the list has room for is
 // tested pixel by pixel; polygons beyond kRasterPolys are a second pass over
 // the row.
 constexpr int kRasterCross = 256, kRasterPolys = 32;
+constexpr int kRasterCols = 256;
 
 __global__ void __launch_bounds__(256)
 k_raster_polygons(float* __restrict__ mask, int H, int W, const double* __restrict__ rp,
@@ -105,7 +107,10 @@ k_raster_polygons(float* __restrict__ mask, int H, int W, const double* __restri
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the wave's own LDS writes
     __builtin_amdgcn_wave_barrier();
-    for (int cb = 0; cb < W; cb += 64) {
+    // this block's columns, run by run (one run unless W exceeds 65535 of them)
+    for (int64_t x = (int64_t)blockIdx.y * kRasterCols; x < W;
+         x = (x + 64) % kRasterCols ? x + 64 : x + 64 + (int64_t)(gridDim.y - 1) * kRasterCols) {
+      const int cb = (int)x;
       const int c = cb + lane;
       bool on = false;
       for (int p = 0; p < np; ++p) {
@@ -483,7 +488,8 @@ int32_t fk_rasterize_polygons(float* mask, int32_t H, int32_t W, const double* r
     HIP_CHECK(hipMemcpyAsync(d_box, boxes.data(), n_polys * sizeof(PolyBox),
                              hipMemcpyHostToDevice, s));
   }
-  k_raster_polygons<<<(H + 3) / 4, 256, 0, s>>>(mask, H, W, d_r, d_c, d_box, n_polys);
+  const dim3 grid((H + 3) / 4, std::min((W - 1) / kRasterCols + 1, 65535));
+  k_raster_polygons<<<grid, 256, 0, s>>>(mask, H, W, d_r, d_c, d_box, n_polys);
   HIP_CHECK(hipGetLastError());
   // the host-side staging of boxes must outlive the copy
   HIP_CHECK(hipStreamSynchronize(s));
