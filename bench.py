@@ -612,7 +612,7 @@ def bench_scar(seed, size=1200, reps=5):
             "roofline": {"bound": "fp64", "achieved": round(achieved, 2),
                          "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
-                         "kernel": "k_conv_cols + k_conv_rows", "flops_per_launch": int(flops)},
+                         "kernel": "k_conv_first + k_conv_last", "flops_per_launch": int(flops)},
             "D_range": [float(D.min()), float(D.max())],
             "cpu_oracle_ms": {"raster": round(t_mask * 1e3, 1),
                               "fft_blur_and_rescale": round(t_fft * 1e3, 1), "cores": 1}}

@@ -137,9 +137,9 @@ k_raster_polygons(float* __restrict__ mask, int H, int W, const double* __restri
 // within a chunk, every tap column q: R input values (one load each, reused
 // by up to R outputs; the chunk's rows stay in L1 across q) and the chunk's
 // 2R - 1 taps of column q, contiguous and wave-uniform in the padded,
-// transposed copy of the kernel (k_pad_kernel: zeros outside [0, kh), so no
+// transposed copy of the kernel (k_conv_prepare: zeros outside [0, kh), so no
 // test per tap). The inputs come from a zero-padded copy of the image
-// (k_pad_image) wide enough for every row and column a thread reaches, so
+// (pad_image) wide enough for every row and column a thread reaches, so
 // the loads need no clamp and no select. Per output the sum runs over
 // chunks, then q, then d, in double; rounded once.
 constexpr int kConvRows = 8;
@@ -167,6 +167,8 @@ __host__ __device__ inline ConvPad conv_pad(int H, int W, int kh, int kw) {
 // order the passes walk them, last tap first.
 constexpr int kSepR = 8;  // outputs per thread of a pass
 
+constexpr int kConvFlags = 64;  // blocks of k_conv_prepare, and a flag of each
+
 struct ConvWork {  // offsets of the workspace, bytes
   size_t taps, col, row, flag, image, total;
 };
@@ -179,47 +181,53 @@ inline ConvWork conv_work(int H, int W, int kh, int kw) {
   w.col = up((size_t)kw * conv_padded_rows(kh) * sizeof(double));
   w.row = w.col + up((size_t)kh * sizeof(double));
   w.flag = w.row + up((size_t)kw * sizeof(double));
-  w.image = w.flag + 256;
+  w.image = w.flag + up(kConvFlags * sizeof(int));
   // the padded image, or the column pass's result in double
   w.total = w.image + std::max((size_t)pd.Hp * pd.Wp * sizeof(float),
                                (size_t)H * W * sizeof(double));
   return w;
 }
 
+// The padded, transposed taps, the factors, and whether the kernel is the outer
+// product of them: every tap c[p] r[q] within `tol` of itself (flags all 1). The
+// direct sum of n taps rounds n times, 2^-53 of the result each at most; tol is
+// half of that, and 2^-48 at most, which keeps the passes' error below its (at most
+// 2^-50.8 of the result and 2^-49.0 with 10 to 19 taps a side, 2^-49.9 and 2^-46.4
+// with 40 to 69). The Gaussian's taps are exp(-(x^2 + y^2) / 2 s^2), whose argument
+// (at most 16 before the tail is cut) carries a few roundings of 2^-53 of itself:
+// over 1400 draws of the generator's width at sides from 4 to 130 no tap was off by
+// more than 2^-48.7. A zero or non-finite centre tap fails (its row is not finite),
+// and so does a tap cut to zero.
 __global__ void __launch_bounds__(256)
-k_pad_kernel(const double* __restrict__ k, int kh, int kw, double* __restrict__ kt,
-             double* __restrict__ col, double* __restrict__ row, int* __restrict__ outer) {
+k_conv_prepare(const double* __restrict__ k, int kh, int kw, double tol,
+               double* __restrict__ kt, double* __restrict__ col, double* __restrict__ row,
+               int* __restrict__ flags) {
   const int kp = conv_padded_rows(kh);
-  const int idx = blockIdx.x * 256 + threadIdx.x;
   const int pc = (kh - 1) / 2, qc = (kw - 1) / 2;
-  if (idx == 0) *outer = 1;
-  if (idx < kh) col[idx] = k[(size_t)(kh - 1 - idx) * kw + qc];
-  if (idx < kw) row[idx] = k[(size_t)pc * kw + kw - 1 - idx] / k[(size_t)pc * kw + qc];
-  if (idx >= kw * kp) return;
-  const int q = idx / kp, p = idx % kp - kConvPadFront;
-  kt[idx] = (p >= 0 && p < kh) ? k[(size_t)p * kw + q] : 0.0;
+  const int64_t t0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = 256 * kConvFlags;
+  bool outer = true;
+  for (int64_t t = t0; t < (int64_t)kw * kp; t += step) {
+    const int q = (int)(t / kp), p = (int)(t - (int64_t)q * kp) - kConvPadFront;
+    const bool in = p >= 0 && p < kh;
+    const double x = in ? k[(size_t)p * kw + q] : 0.0;
+    kt[t] = x;
+    if (!in) continue;
+    const double c = k[(size_t)p * kw + qc], r = k[(size_t)pc * kw + q] / k[(size_t)pc * kw + qc];
+    outer = outer && fabs(x - c * r) <= tol * fabs(x) && isfinite(x);
+    if (q == qc) col[kh - 1 - p] = c;
+    if (p == pc) row[kw - 1 - q] = r;
+  }
+  outer = __syncthreads_and(outer);
+  if (threadIdx.x == 0) flags[blockIdx.x] = outer;
 }
 
-// *outer stays 1 when every tap is c[p] r[q] within 2^-46 of itself. The
-// Gaussian's taps are exp(-(x^2 + y^2) / 2 s^2), whose argument (at most 16
-// before the tail is cut) carries a rounding of 2^-53 of itself, so products
-// of two of them agree within 2^-48; the blurred value then agrees to 2^-46,
-// against the 2^-24 of its rounding to float32. A zero or non-finite centre
-// tap fails (its row is not finite), and so does a tap cut to zero.
-__global__ void __launch_bounds__(256)
-k_check_outer(const double* __restrict__ k, int kh, int kw, const double* __restrict__ col,
-              const double* __restrict__ row, int* __restrict__ outer) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)kh * kw) return;
-  const int p = (int)(idx / kw), q = (int)(idx - (int64_t)p * kw);
-  const double x = k[idx], y = col[kh - 1 - p] * row[kw - 1 - q];
-  if (!(fabs(x - y) <= 0x1p-46 * fabs(x)) || !isfinite(x)) *outer = 0;
+__device__ __forceinline__ bool is_outer(const int* __restrict__ flags) {
+  static_assert(kConvFlags == 64, "a flag per lane");
+  return __builtin_amdgcn_ballot_w64(flags[threadIdx.x & 63] != 0) == ~0ull;
 }
 
-__global__ void __launch_bounds__(256)
-k_pad_image(const float* __restrict__ src, int H, int W, ConvPad pd, float* __restrict__ pad,
-            const int* __restrict__ outer) {
-  if (*outer) return;  // the two passes run
+__device__ __forceinline__ void pad_image(const float* __restrict__ src, int H, int W, ConvPad pd,
+                                          float* __restrict__ pad) {
   const size_t n = (size_t)pd.Hp * pd.Wp;
   for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < n;
        idx += (size_t)gridDim.x * 256) {
@@ -228,14 +236,14 @@ k_pad_image(const float* __restrict__ src, int H, int W, ConvPad pd, float* __re
   }
 }
 
-__global__ void __launch_bounds__(256)
-k_convolve_same(const float* __restrict__ pad, int H, int W, ConvPad pd,
-                const double* __restrict__ kt, int kh, int kw, float* __restrict__ dst,
-                const int* __restrict__ outer) {
-  if (*outer) return;  // the two passes run
+// Block b of the direct sum.
+__device__ __forceinline__ void convolve_same(const float* __restrict__ pad, int H, int W,
+                                              ConvPad pd, const double* __restrict__ kt, int kh,
+                                              int kw, float* __restrict__ dst, int b) {
   constexpr int R = kConvRows;
-  const int j = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int i0 = __builtin_amdgcn_readfirstlane((blockIdx.y * 4 + (int)(threadIdx.x >> 6)) * R);
+  const int bx = (W + 63) / 64;
+  const int j = b % bx * 64 + (threadIdx.x & 63);
+  const int i0 = __builtin_amdgcn_readfirstlane((b / bx * 4 + (int)(threadIdx.x >> 6)) * R);
   if (i0 >= H) return;  // wave-uniform
   const int oi = (kh - 1) / 2, oj = (kw - 1) / 2;
   const int kp = conv_padded_rows(kh);
@@ -298,14 +306,14 @@ __device__ __forceinline__ void sep_fma(double acc[kSepR], const double x[kSepR]
 // in double, kSepR outputs down a column per thread. Walking input rows
 // m = 0 .. kh + kSepR - 2 from i0 + oi - (kh - 1), output r takes tap m - r of
 // the reversed column: one coalesced load per row feeds kSepR multiply-adds
-// with wave-uniform taps.
-__global__ void __launch_bounds__(256)
-k_conv_cols(const float* __restrict__ src, int H, int W, const double* __restrict__ col, int kh,
-            double* __restrict__ tmp, const int* __restrict__ outer) {
-  if (!*outer) return;
+// with wave-uniform taps. Block b of (W + 63) / 64 across.
+__device__ __forceinline__ void conv_cols(const float* __restrict__ src, int H, int W,
+                                          const double* __restrict__ col, int kh,
+                                          double* __restrict__ tmp, int b) {
   constexpr int R = kSepR;
-  const int j = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int i0 = __builtin_amdgcn_readfirstlane((blockIdx.y * 4 + (int)(threadIdx.x >> 6)) * R);
+  const int bx = (W + 63) / 64;
+  const int j = b % bx * 64 + (threadIdx.x & 63);
+  const int i0 = __builtin_amdgcn_readfirstlane((b / bx * 4 + (int)(threadIdx.x >> 6)) * R);
   if (i0 >= H) return;  // wave-uniform
   const uint32_t cb = (uint32_t)min(j, W - 1) * 4u;
   const int top = i0 + (kh - 1) / 2 - (kh - 1);
@@ -340,14 +348,14 @@ k_conv_cols(const float* __restrict__ src, int H, int W, const double* __restric
 constexpr int kSepSeg = 64 * kSepR;
 constexpr int kSepSpan = 256;
 
-__global__ void __launch_bounds__(256)
-k_conv_rows(const double* __restrict__ tmp, int H, int W, const double* __restrict__ row, int kw,
-            float* __restrict__ dst, const int* __restrict__ outer) {
-  if (!*outer) return;
+__device__ __forceinline__ void conv_rows(const double* __restrict__ tmp, int H, int W,
+                                          const double* __restrict__ row, int kw,
+                                          float* __restrict__ dst, int b) {
   constexpr int R = kSepR, N = kSepSeg + kSepSpan;
   __shared__ double s[4][N + N / R];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = blockIdx.x * 4 + wave, j0 = blockIdx.y * kSepSeg;
+  const int bx = (H + 3) / 4;
+  const int i = b % bx * 4 + wave, j0 = b / bx * kSepSeg;
   const int left = j0 + (kw - 1) / 2 - (kw - 1);  // column of input m = 0 of output j0
   const double* src = tmp + (size_t)min(i, H - 1) * W;
   double acc[R];
@@ -374,6 +382,33 @@ k_conv_rows(const double* __restrict__ tmp, int H, int W, const double* __restri
       const int j = j0 + R * lane + r;
       if (j < W) dst[(size_t)i * W + j] = (float)acc[r];
     }
+  }
+}
+
+// Either route's first launch (the column pass; the padded image) and second one
+// (the row pass; the direct sum), each in the blocks it needs. With a launch for
+// each, those not wanted cost 10 us a call: 12 x 12 taps at 128 x 128 take 32 us as
+// an outer product and 40 directly, before 38 and 51.
+__global__ void __launch_bounds__(256)
+k_conv_first(const float* __restrict__ src, int H, int W, ConvPad pd,
+             const double* __restrict__ col, int kh, float* __restrict__ pad,
+             double* __restrict__ tmp, int n_cols, const int* __restrict__ flags) {
+  if (!is_outer(flags))
+    pad_image(src, H, W, pd, pad);
+  else if ((int)blockIdx.x < n_cols)
+    conv_cols(src, H, W, col, kh, tmp, blockIdx.x);
+}
+
+__global__ void __launch_bounds__(256)
+k_conv_last(const float* __restrict__ pad, const double* __restrict__ tmp, int H, int W,
+            ConvPad pd, const double* __restrict__ kt, const double* __restrict__ row, int kh,
+            int kw, float* __restrict__ dst, int n_rows, int n_direct,
+            const int* __restrict__ flags) {
+  const int b = blockIdx.x;
+  if (is_outer(flags)) {  // uniform over the block, as is b: conv_rows has barriers
+    if (b < n_rows) conv_rows(tmp, H, W, row, kw, dst, b);
+  } else if (b < n_direct) {
+    convolve_same(pad, H, W, pd, kt, kh, kw, dst, b);
   }
 }
 
@@ -545,24 +580,21 @@ int32_t fk_convolve_same(const float* src, int32_t H, int32_t W, const double* k
   const ConvPad pd = conv_pad(H, W, kh, kw);
   char* wk = (char*)work;
   double *kt = (double*)wk, *col = (double*)(wk + wo.col), *row = (double*)(wk + wo.row);
-  int* outer = (int*)(wk + wo.flag);
+  int* flags = (int*)(wk + wo.flag);
   float* pad = (float*)(wk + wo.image);
   double* tmp = (double*)(wk + wo.image);
-  const int n_pad = kw * conv_padded_rows(kh);  // >= kh and kw
-  k_pad_kernel<<<(n_pad + 255) / 256, 256, 0, s>>>(kernel, kh, kw, kt, col, row, outer);
-  k_check_outer<<<(unsigned)(((size_t)kh * kw + 255) / 256), 256, 0, s>>>(kernel, kh, kw, col,
-                                                                          row, outer);
-  // The host does not know the kernel's values: both routes are queued, and
-  // the kernels of the one not taken leave at once.
-  k_conv_cols<<<dim3((W + 63) / 64, (H + 4 * kSepR - 1) / (4 * kSepR)), 256, 0, s>>>(
-      src, H, W, col, kh, tmp, outer);
-  k_conv_rows<<<dim3((H + 3) / 4, (W + kSepSeg - 1) / kSepSeg), 256, 0, s>>>(tmp, H, W, row, kw,
-                                                                            dst, outer);
-  const size_t n_img = (size_t)pd.Hp * pd.Wp;
-  k_pad_image<<<(int)std::min<size_t>((n_img + 255) / 256, 4096), 256, 0, s>>>(src, H, W, pd,
-                                                                              pad, outer);
-  const dim3 grid((W + 63) / 64, (H + 4 * kConvRows - 1) / (4 * kConvRows));
-  k_convolve_same<<<grid, 256, 0, s>>>(pad, H, W, pd, kt, kh, kw, dst, outer);
+  const double tol = std::min(0x1p-48, 0x1p-54 * kh * kw);
+  k_conv_prepare<<<kConvFlags, 256, 0, s>>>(kernel, kh, kw, tol, kt, col, row, flags);
+  // The host does not know the kernel's values: a launch holds both routes, by the
+  // flags.
+  const int64_t nc = (int64_t)((W + 63) / 64) * ((H + 4 * kSepR - 1) / (4 * kSepR));
+  const int64_t np = std::min<int64_t>(((int64_t)pd.Hp * pd.Wp + 1023) / 1024, 4096);
+  k_conv_first<<<(unsigned)std::max(nc, np), 256, 0, s>>>(src, H, W, pd, col, kh, pad, tmp, (int)nc,
+                                                          flags);
+  const int64_t nr = (int64_t)((H + 3) / 4) * ((W + kSepSeg - 1) / kSepSeg);
+  const int64_t nd = (int64_t)((W + 63) / 64) * ((H + 4 * kConvRows - 1) / (4 * kConvRows));
+  k_conv_last<<<(unsigned)std::max(nr, nd), 256, 0, s>>>(pad, tmp, H, W, pd, kt, row, kh, kw, dst,
+                                                         (int)nr, (int)nd, flags);
   HIP_CHECK(hipGetLastError());
   return FK_OK;
 }
