@@ -11,8 +11,8 @@
 // steps; for each segment, in reverse, the states are recomputed from its
 // checkpoint and the steps are reversed one by one, frame cotangents entering
 // lam_u at the frame steps. Every launch covers all problems through a work
-// list (forward steps a block per block tile, two to four steps; reverse steps a
-// wave per tile), and the tiles run the same device code as the per-grid
+// list (forward steps a block per block tile, two to four steps, or a wave per
+// streaming tile for a single one; reverse steps a wave per tile), and the tiles run the same device code as the per-grid
 // kernels: the results are bitwise those of the per-grid path.
 //
 // Reference: there is no counterpart in the reference, whose inverse problem
@@ -34,6 +34,17 @@
 #include "fk_stream.h"
 
 namespace fk {
+
+__device__ __forceinline__ Coef uni(const Coef& a) {
+  Coef c = a;
+  c.V_c = uni(c.V_c); c.V_v = uni(c.V_v); c.V_csi = uni(c.V_csi); c.kk = uni(c.kk);
+  c.kk_off = uni(c.kk_off);
+  c.inv_tvp = uni(c.inv_tvp); c.inv_tv1m = uni(c.inv_tv1m); c.inv_tv2m = uni(c.inv_tv2m);
+  c.inv_twp = uni(c.inv_twp); c.inv_twm = uni(c.inv_twm); c.inv_td = uni(c.inv_td);
+  c.inv_t0 = uni(c.inv_t0); c.inv_tr = uni(c.inv_tr); c.inv_tsi = uni(c.inv_tsi);
+  c.inv_cm = uni(c.inv_cm);
+  return c;
+}
 
 // Block tiling of the forward steps.
 enum RollBlock { kRoll32x4, kRoll48x3, kRoll32x2 };
@@ -97,13 +108,7 @@ k_roll_block(const RollDesc* __restrict__ sims, const BlockItem* __restrict__ it
   if (sim < 0) return;  // padding of the XCD order: the whole block leaves
   const RollDesc& S = sims[sim];
   const BatchBlockStim sv{S.stim, pack_masks(masks + sim, n, n_lev)};
-  Coef c = S.c;
-  c.V_c = uni(c.V_c); c.V_v = uni(c.V_v); c.V_csi = uni(c.V_csi); c.kk = uni(c.kk);
-  c.kk_off = uni(c.kk_off);
-  c.inv_tvp = uni(c.inv_tvp); c.inv_tv1m = uni(c.inv_tv1m); c.inv_tv2m = uni(c.inv_tv2m);
-  c.inv_twp = uni(c.inv_twp); c.inv_twm = uni(c.inv_twm); c.inv_td = uni(c.inv_td);
-  c.inv_t0 = uni(c.inv_t0); c.inv_tr = uni(c.inv_tr); c.inv_tsi = uni(c.inv_tsi);
-  c.inv_cm = uni(c.inv_cm);
+  const Coef c = uni(S.c);
   const size_t cells = S.cells;
   float* out = uni(S.traj + (size_t)k * 3 * cells);
   const BlockIO io{uni(S.D), uni(roll_state(S, seg, k, 0)), uni(roll_state(S, seg, k, 1)),
@@ -113,6 +118,50 @@ k_roll_block(const RollDesc* __restrict__ sims, const BlockItem* __restrict__ it
   const BlockSpan q{uni(it.c.o), uni(it.c.a), uni(it.c.b)};
   block_tile_any<Cfg, false>(c, io, uni(S.H), uni(S.W), sv, n_lev, uni(S.dt), uni(S.inv_dx2), r,
                              q, lds);
+}
+
+// One Euler step: x_{c+k} -> trajectory slot k, on streaming tiles of kRollRows
+// rows, a wave each: the step that whole launches of the block tiles leave over, and
+// every step of segments of one. A block tile's halo is made for several steps.
+// Forward, us per step with segments of one and of three, on block tiles only and
+// so: 1.05 M cells 18.6 and 11.2, 17.2 and 10.3; 3.1 M cells 38.9 and 24.5, 35.0
+// and 22.9.
+constexpr int kRollRows = 4;
+
+__global__ void __launch_bounds__(256)
+k_roll_step(const RollDesc* __restrict__ sims, const RollTile* __restrict__ items, int n_items,
+            const uint32_t* __restrict__ masks, int seg, int k) {
+  constexpr int R = kRollRows;
+  const int it = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x >> 6));
+  if (it >= n_items) return;
+  const RollTile item = items[it];
+  const int sim = uni(item.sim), rs = uni(item.rs), cs = uni(item.cs);
+  if (sim < 0) return;  // padding of the XCD order
+  const RollDesc& S = sims[sim];
+  const uint32_t mask = (uint32_t)uni((int)masks[sim]);
+  const BatchStimView sv{S.stim, uni(S.n_stim), mask};
+  const Coef c = uni(S.c);
+  const size_t cells = S.cells;
+  const float *D = uni(S.D), *v = uni(roll_state(S, seg, k, 0)), *w = uni(roll_state(S, seg, k, 1)),
+              *u = uni(roll_state(S, seg, k, 2));
+  float* out = uni(S.traj + (size_t)k * 3 * cells);
+  const int H = uni(S.H), W = uni(S.W);
+  const float dt = uni(S.dt), inv_dx2 = uni(S.inv_dx2);
+#define FK_RS(X, Y, ST)                                                                     \
+  stream_tile<R, true, X, Y, ST, BatchStimView, false, true>(c, D, nullptr, v, w, u, H, W, sv, \
+                                                             dt, inv_dx2, out, out + cells,    \
+                                                             out + 2 * cells, rs, cs)
+  switch (uni(item.flags) | (mask ? 4 : 0)) {
+    case 0: FK_RS(false, false, false); break;
+    case 1: FK_RS(true, false, false); break;
+    case 2: FK_RS(false, true, false); break;
+    case 3: FK_RS(true, true, false); break;
+    case 4: FK_RS(false, false, true); break;
+    case 5: FK_RS(true, false, true); break;
+    case 6: FK_RS(false, true, true); break;
+    default: FK_RS(true, true, true); break;
+  }
+#undef FK_RS
 }
 
 // After forward segment `seg` (steps c .. c + len - 1): the frames it holds
@@ -179,13 +228,7 @@ k_roll_rev(const RollDesc* __restrict__ sims, const RollTile* __restrict__ items
                   uni(S.part), uni(S.tab)};
   const uint32_t mask = uni((int)masks[item.sim]);
   const BatchStimView sv{S.stim, mask ? uni(S.n_stim) : 0, mask};
-  Coef c = S.c;
-  c.V_c = uni(c.V_c); c.V_v = uni(c.V_v); c.V_csi = uni(c.V_csi); c.kk = uni(c.kk);
-  c.kk_off = uni(c.kk_off);
-  c.inv_tvp = uni(c.inv_tvp); c.inv_tv1m = uni(c.inv_tv1m); c.inv_tv2m = uni(c.inv_tv2m);
-  c.inv_twp = uni(c.inv_twp); c.inv_twm = uni(c.inv_twm); c.inv_td = uni(c.inv_td);
-  c.inv_t0 = uni(c.inv_t0); c.inv_tr = uni(c.inv_tr); c.inv_tsi = uni(c.inv_tsi);
-  c.inv_cm = uni(c.inv_cm);
+  const Coef c = uni(S.c);
   adj_tile_any<R>(c, a, uni(S.H), uni(S.W), sv, uni(S.dt), uni(S.inv_dx2), uni(item.rs),
                   uni(item.cs), uni(item.flags), tab[threadIdx.x >> 6]);
 }
@@ -203,9 +246,10 @@ struct fk_rollout_batch {
   size_t dev_bytes = 0;
   RollDesc* d_sims = nullptr;
   BlockItem* d_tiles = nullptr;  // forward
+  RollTile* d_step = nullptr;    // forward, single steps
   RollTile* d_rev = nullptr;     // reverse
   uint32_t* d_masks = nullptr;  // n_steps x n
-  int n_tiles = 0, n_rev = 0;
+  int n_tiles = 0, n_step = 0, n_rev = 0;
   int block = kRoll32x4;  // RollBlock of the forward steps
   int rev_rows = 4;       // band rows of the reverse tiles
   size_t max_cells = 0;
@@ -287,7 +331,11 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   // adjacent reverse tiles (which share halo rows), whole on one die each
   constexpr int kRunTiles = 16;
   std::vector<BlockItem> blocks;
-  std::vector<std::vector<RollTile>> rev_runs;
+  std::vector<std::vector<RollTile>> step_runs, rev_runs;
+  // whether some segment, or its recomputation, leaves a single step over
+  const int per = roll_steps(b->block), last = n_steps - (b->n_seg - 1) * b->S;
+  bool single = false;
+  for (int len : {b->S, b->S - 1, last, last - 1}) single = single || len % per == 1;
   for (int i = 0; i < n; ++i) {
     const fk_rollout_spec& s = specs[i];
     switch (b->block) {
@@ -295,6 +343,18 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
       case kRoll48x3: append_block_items<Block48x3>(i, s.H, s.W, blocks); break;
       default: append_block_items<Block32x2>(i, s.H, s.W, blocks); break;
     }
+    const StreamGeom g = make_stream_geom<kRollRows>(s.H, s.W);
+    for (int strip = 0; single && strip < g.n_strips; ++strip)
+      for (int band = 0; band < g.n_bands; ++band) {
+        RollTile t;
+        t.sim = i;
+        t.cs = std::min(kStripOut * strip, g.cs_last);
+        t.rs = std::min(kRollRows * band, g.rs_last);
+        const bool yg = t.cs < 3 || t.cs + kStripOut + 3 > s.W;
+        t.flags = (edge_band(t.rs, kRollRows, s.H, s.W) ? 1 : 0) | (yg ? 2 : 0);
+        if (band % kRunTiles == 0) step_runs.emplace_back();
+        step_runs.back().push_back(t);
+      }
     for (int strip = 0; strip < adj_strips(s.W); ++strip)
       for (int band = 0; band < (s.H + rows - 1) / rows; ++band) {
         RollTile t;
@@ -308,8 +368,10 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
       }
   }
   const std::vector<BlockItem> tiles = block_work_list(blocks);
+  const std::vector<RollTile> steps = xcd_order(step_runs, 4, RollTile{-1, 0, 0, 0});
   const std::vector<RollTile> rev = xcd_order(rev_runs, rows == 1 ? 2 : 4, RollTile{-1, 0, 0, 0});
   b->n_tiles = (int)tiles.size();
+  b->n_step = (int)steps.size();
   b->n_rev = (int)rev.size();
   // stimulus activity of every step, as the per-grid path evaluates it
   std::vector<uint32_t> masks((size_t)n_steps * n);
@@ -328,6 +390,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   };
   const size_t o_sims = take(sizeof(RollDesc) * n);
   const size_t o_tiles = take(sizeof(BlockItem) * tiles.size());
+  const size_t o_step = take(sizeof(RollTile) * steps.size());
   const size_t o_rev = take(sizeof(RollTile) * rev.size());
   const size_t o_masks = take(sizeof(uint32_t) * masks.size());
   std::vector<size_t> o_ckpt(n), o_traj(n), o_lam(n);
@@ -350,6 +413,7 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   }
   b->d_sims = (RollDesc*)(b->dev + o_sims);
   b->d_tiles = (BlockItem*)(b->dev + o_tiles);
+  b->d_step = (RollTile*)(b->dev + o_step);
   b->d_rev = (RollTile*)(b->dev + o_rev);
   b->d_masks = (uint32_t*)(b->dev + o_masks);
   std::vector<RollDesc> desc(n);
@@ -388,6 +452,8 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   if (e == hipSuccess)
     e = hipMemcpy(b->d_tiles, tiles.data(), sizeof(BlockItem) * tiles.size(),
                   hipMemcpyHostToDevice);
+  if (e == hipSuccess && !steps.empty())
+    e = hipMemcpy(b->d_step, steps.data(), sizeof(RollTile) * steps.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(b->d_rev, rev.data(), sizeof(RollTile) * rev.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess)
@@ -406,13 +472,18 @@ size_t fk_rollout_batch_device_bytes(const fk_rollout_batch* b) { return b ? b->
 // Steps c .. c + n_steps - 1 of segment `seg` (c = seg S) into the trajectory.
 static void roll_steps_of(fk_rollout_batch* b, int seg, int n_steps, hipStream_t s) {
   const int per = roll_steps(b->block);
+  auto masks = [&](int k) { return b->d_masks + (size_t)(seg * b->S + k) * b->n; };
   auto go = [&](auto cfg, int k, int n_lev) {
     typedef decltype(cfg) Cfg;
-    k_roll_block<Cfg><<<b->n_tiles, Cfg::waves * 64, 0, s>>>(
-        b->d_sims, b->d_tiles, b->n, b->d_masks + (size_t)(seg * b->S + k) * b->n, seg, k, n_lev);
+    k_roll_block<Cfg><<<b->n_tiles, Cfg::waves * 64, 0, s>>>(b->d_sims, b->d_tiles, b->n, masks(k),
+                                                            seg, k, n_lev);
   };
   for (int k = 0; k < n_steps; k += per) {
     const int n_lev = std::min(per, n_steps - k);
+    if (n_lev == 1) {
+      k_roll_step<<<b->n_step / 4, 256, 0, s>>>(b->d_sims, b->d_step, b->n_step, masks(k), seg, k);
+      continue;
+    }
     switch (b->block) {
       case kRoll32x4: go(Block32x4{}, k, n_lev); break;
       case kRoll48x3: go(Block48x3{}, k, n_lev); break;
