@@ -179,7 +179,6 @@ __device__ __forceinline__ void copy_cells(float* __restrict__ dst, const float*
 // 1.85 ms; 26.1 M cells now take 0.15 ms). blockIdx.y strides over the
 // fields: LOAD callers -> pool 0 and resets the step counter; else pool
 // `parity` -> callers and moves every simulation's time on by n_steps.
-constexpr int kCopyBlocks = 16;  // blocks per field and launch row
 
 template <bool LOAD>
 __global__ void __launch_bounds__(256)
@@ -190,9 +189,9 @@ k_batch_copy(SimDesc* __restrict__ sims, int n, int parity, int64_t* __restrict_
     const int f = (int)(y % 3);
     const size_t cells = (size_t)S.H * S.W;
     if (LOAD)
-      copy_cells(S.buf[0][f], S.user[f], cells, blockIdx.x, kCopyBlocks);
+      copy_cells(S.buf[0][f], S.user[f], cells, blockIdx.x, gridDim.x);
     else
-      copy_cells(S.user[f], S.buf[parity][f], cells, blockIdx.x, kCopyBlocks);
+      copy_cells(S.user[f], S.buf[parity][f], cells, blockIdx.x, gridDim.x);
     if (!LOAD && f == 0 && blockIdx.x == 0 && threadIdx.x == 0) S.t0 += (double)n_steps;
   }
   if (LOAD && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *step_base = 0;
@@ -220,6 +219,7 @@ struct fk_batch {
   std::vector<fk_sim> host_sims;   // caller's descriptors (state pointers)
   std::vector<size_t> offset;      // per-sim cell offset in the pools
   size_t total_cells = 0;
+  int copy_blocks = 0;             // blocks per field of k_batch_copy
   char* dev = nullptr;             // one allocation: descriptors, items, counter, pools
   SimDesc* d_sims = nullptr;
   char* d_items[kNumRowOpts] = {};  // TileItem (one step) or BlockItem
@@ -300,6 +300,13 @@ int32_t fk_batch_create(const fk_sim* sims, int32_t n, fk_batch** out) {
         }
     }
   }
+  // blocks of a field's copy: 4096 cells each in the largest simulation, 16 at least,
+  // about 2^16 in all. With 16 whatever the sizes, one step of a batch of one 4096^2
+  // simulation took 1130 us (290 so), of one 2048^2 180 (60).
+  size_t largest = 0;
+  for (int i = 0; i < n; ++i) largest = std::max(largest, (size_t)sims[i].H * sims[i].W);
+  b->copy_blocks =
+      (int)std::max<size_t>(16, std::min<size_t>(largest / 4096, 65536 / (3 * (size_t)n)));
   // 32 rows: 4 steps per launch for batches of few tiles, else 2
   LeastRounds by32((int64_t)b->total_cells), least((int64_t)b->total_cells);
   by32.offer(kBatch32x4, Block32x4{}, n32x4);
@@ -569,7 +576,7 @@ int32_t fk_batch_run(fk_batch* b, int64_t n_steps, int32_t use_graph, void* stre
   for (int i = 0; i < b->n_sims; ++i)
     if (!check_time(b->host_sims[i].t, b->host_sims[i].t + (double)n_steps)) return last_code();
   hipStream_t s = (hipStream_t)stream;
-  const dim3 cg(kCopyBlocks, (unsigned)std::min<int64_t>(3 * (int64_t)b->n_sims, 65535));
+  const dim3 cg(b->copy_blocks, (unsigned)std::min<int64_t>(3 * (int64_t)b->n_sims, 65535));
   k_batch_copy<true><<<cg, 256, 0, s>>>(b->d_sims, b->n_sims, 0, b->d_step, 0);
   HIP_CHECK(hipGetLastError());
   int64_t k = 0;

@@ -12,8 +12,9 @@
 // checkpoint and the steps are reversed one by one, frame cotangents entering
 // lam_u at the frame steps. Every launch covers all problems through a work
 // list (forward steps a block per block tile, two to four steps, or a wave per
-// streaming tile for a single one; reverse steps a wave per tile), and the tiles run the same device code as the per-grid
-// kernels: the results are bitwise those of the per-grid path.
+// streaming tile for a single one; reverse steps a wave per tile), and the tiles
+// run the same device code as the per-grid kernels: the results are bitwise those
+// of the per-grid path.
 //
 // Reference: there is no counterpart in the reference, whose inverse problem
 // is learnt by a network (deepx); the forward step follows
@@ -320,8 +321,8 @@ int32_t fk_rollout_batch_create(const fk_rollout_spec* specs, int32_t n, int32_t
   least.offer(kRoll48x3, Block48x3{}, n48x3);
   least.offer(kRoll32x2, Block32x2{}, n32x2);
   b->block = least.best;
-  // A row per wave as in the per-grid step; bands of 2 rows while the waves are few and a wave's rows, one after
-  // the other, set the time (2 problems 64 to 200 wide, 100 steps: 1.07 ms, 1.33 with
+  // A row per wave as in the per-grid step; bands of 2 rows while the waves are few
+  // and a wave's rows, one after the other, set the time (2 problems 64 to 200 wide, 100 steps: 1.07 ms, 1.33 with
   // 4; 10 of 128 to 480: 3.33 and 3.40); 4 rows for more (12 of 128 to 512: 4.63 and
   // 4.69; one reverse step of 3.84 M cells 60 and 68 us, 67 with 8). The bits do not
   // depend on it.

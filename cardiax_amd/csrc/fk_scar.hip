@@ -60,9 +60,9 @@ __device__ __forceinline__ bool inside_polygon(const double* __restrict__ rp,
 // a comparison per crossing (two to six on the generator's contours) instead of
 // one per vertex: 47 us before, 13 us now for 5 contours of 101 vertices at
 // 1200 x 1200. Columns per wave: 64 take 27 us there, 128 18, 512 14, and a
-// whole row 19 (and 4 x 100000 up to 800, where 256 take 10). A polygon with more crossings than the list has room for is
-// tested pixel by pixel; polygons beyond kRasterPolys are a second pass over
-// the row.
+// whole row 19 (and 4 x 100000 up to 800, where 256 take 10). A polygon with more
+// crossings than the list has room for is tested pixel by pixel; polygons beyond
+// kRasterPolys are a second pass over the row.
 constexpr int kRasterCross = 256, kRasterPolys = 32;
 constexpr int kRasterCols = 256;
 
