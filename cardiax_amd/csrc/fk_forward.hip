@@ -343,6 +343,19 @@ static bool is_block(int v) { return v >= kBlock32x2 && v <= kBlock32x4; }
 
 static int block_steps(int v) { return v == kBlock32x2 ? 2 : v == kBlock32x4 ? 4 : 3; }
 
+// Steps of the next launch of block variant v with `left` to go, and in *v the
+// variant that runs them. Where a step's fields exceed the 256 MB cache (`streams`),
+// a tile of three steps takes as long for two of them as for three, so a solve of
+// 3 a + 1 or 3 a + 2 steps ends in two launches or one of two steps on 32 rows
+// (4096^2: two steps 140 us in place of 189, four 278 in place of 353).
+static int block_launch(int* v, int64_t left, bool streams) {
+  if (streams && *v == kBlock48x3 && (left == 2 || left == 4)) {
+    *v = kBlock32x2;
+    return 2;
+  }
+  return (int)std::min<int64_t>(block_steps(*v), left);
+}
+
 static bool is_two_step(int v) { return v >= kStreamT8 && v <= kStreamT24; }
 
 // Whether the two-step variant v fits an H x W grid (else stream2 runs).
@@ -674,7 +687,7 @@ int32_t forward_loop(int variant, const fk_params* params, const float* D, const
   const float inv_dx2 = (float)(1.0 / ((double)dx * (double)dx));
   float* wk = (float*)work;
   float* bufs[2][3] = {{v_out, w_out, u_out}, {wk, wk + n, wk + 2 * n}};
-  int v = resolve_solve(variant, H, W);
+  int v = steps < 2 ? resolve_for(variant, H, W) : resolve_solve(variant, H, W);
   // nothing to amortise, or no room for the coefficients
   if (is_pc(v) && (steps < 2 || state_only)) v = pc_base(v);
   float4* cf = nullptr;
@@ -692,12 +705,11 @@ int32_t forward_loop(int variant, const fk_params* params, const float* D, const
   StimSchedule sched(stimuli, n_stimuli);
   BlockStim st{};
   for (int i = 0; i < n_stimuli; ++i) st.f[i] = stimuli[i].field;
-  for (int64_t k = 0; k < steps; k += depth) {
+  for (int64_t k = 0, ns = depth; k < steps; k += ns) {
     float** d = bufs[dst];
     if (is_two_step(v)) {
-      const int ns = (int)std::min<int64_t>(2, steps - k);
       const StimArgs s1 = sched.at(t + (double)k);  // copies: at() reuses its storage
-      if (ns == 2) {
+      if (steps - k >= 2) {
         const StimArgs s2 = sched.at(t + (double)(k + 1));
         HIP_CHECK(launch_two_step(v, c, D, src[0], src[1], src[2], H, W, s1, s2, dt, inv_dx2,
                                   d[0], d[1], d[2], s));
@@ -706,10 +718,11 @@ int32_t forward_loop(int variant, const fk_params* params, const float* D, const
                               inv_dx2, d[0], d[1], d[2], s));
       }
     } else if (is_block(v) && steps - k > 1) {
-      const int ns = (int)std::min<int64_t>(depth, steps - k);
-      block_stim(sched, t + (double)k, ns, st);
+      int bv = v;
+      ns = block_launch(&bv, steps - k, LeastRounds((int64_t)n).streams);
+      block_stim(sched, t + (double)k, (int)ns, st);
       const BlockIO io{D, src[0], src[1], src[2], d[0], d[1], d[2], 0, false};
-      HIP_CHECK(launch_block(v, c, io, H, W, st, ns, dt, inv_dx2, dst == 1, s));
+      HIP_CHECK(launch_block(bv, c, io, H, W, st, (int)ns, dt, inv_dx2, dst == 1, s));
     } else if (is_block(v)) {  // a single last step
       HIP_CHECK(launch_step(kStream2, true, c, D, src[0], src[1], src[2], H, W,
                             sched.at(t + (double)k), dt, inv_dx2, d[0], d[1], d[2], s));

@@ -142,7 +142,8 @@ void fk_autotune_reset(void);
 int32_t fk_forward_variant_for(int32_t H, int32_t W);
 
 /* The variant whose kernel fk_forward_euler runs on an H x W grid now over
- * several steps (a single last step of 7-10 and 19-22 runs 15).
+ * several steps (a single last step of 7-10 and 19-22 runs 15, and large grids
+ * may end a solve by 8 in launches of 7; the bits are the same).
  * fk_forward_trajectory runs the same of 7-10, and the one-step kernel of any
  * other. No reference counterpart. FK_ERR_ARG for a grid that a solve refuses. */
 int32_t fk_solve_variant_for(int32_t H, int32_t W);
