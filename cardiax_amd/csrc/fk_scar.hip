@@ -18,7 +18,7 @@
 // out[i, j] = sum_{p, q} k[p, q] in[i + (kh-1)/2 - p, j + (kw-1)/2 - q]
 // (integer halves), zero outside the image; products and sums in double. A
 // kernel that is an outer product (the generator's Gaussian, unless its tail
-// was cut) runs as a column pass and a row pass.
+// was cut) and not small runs as a column pass and a row pass.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -167,7 +167,9 @@ __host__ __device__ inline ConvPad conv_pad(int H, int W, int kh, int kw) {
 // order the passes walk them, last tap first.
 constexpr int kSepR = 8;  // outputs per thread of a pass
 
-constexpr int kConvFlags = 64;  // blocks of k_conv_prepare, and a flag of each
+// Blocks of k_conv_prepare, and a flag of each; then one that is set when the image
+// holds a value that is not finite.
+constexpr int kConvFlags = 64;
 
 struct ConvWork {  // offsets of the workspace, bytes
   size_t taps, col, row, flag, image, total;
@@ -181,44 +183,49 @@ inline ConvWork conv_work(int H, int W, int kh, int kw) {
   w.col = up((size_t)kw * conv_padded_rows(kh) * sizeof(double));
   w.row = w.col + up((size_t)kh * sizeof(double));
   w.flag = w.row + up((size_t)kw * sizeof(double));
-  w.image = w.flag + up(kConvFlags * sizeof(int));
+  w.image = w.flag + up((kConvFlags + 1) * sizeof(int));
   // the padded image, or the column pass's result in double
   w.total = w.image + std::max((size_t)pd.Hp * pd.Wp * sizeof(float),
                                (size_t)H * W * sizeof(double));
   return w;
 }
 
-// The padded, transposed taps, the factors, and whether the kernel is the outer
-// product of them: every tap c[p] r[q] within `tol` of itself (flags all 1). The
-// direct sum of n taps rounds n times, 2^-53 of the result each at most; tol is
-// half of that, and 2^-48 at most, which keeps the passes' error below its (at most
-// 2^-50.8 of the result and 2^-49.0 with 10 to 19 taps a side, 2^-49.9 and 2^-46.4
-// with 40 to 69). The Gaussian's taps are exp(-(x^2 + y^2) / 2 s^2), whose argument
-// (at most 16 before the tail is cut) carries a few roundings of 2^-53 of itself:
-// over 1400 draws of the generator's width at sides from 4 to 130 no tap was off by
-// more than 2^-48.7. A zero or non-finite centre tap fails (its row is not finite),
-// and so does a tap cut to zero.
+// Whether an outer-product kernel takes the two passes: from kMinPasses units of the
+// direct sum on, a unit being one tap column of one chunk of rows. Direct and passes,
+// us a call: 10 x 10 taps (30 units) 22.7 and 22.0 at 1000 x 700, 18.7 and 14.2 at 64^2;
+// 9 x 9 (18) 18.2 and 19.9, 16.1 and 12.5; 60 x 2 (18) 20.0 and 25.6; 3 x 3 13.7 and 19.5.
+constexpr int kMinPasses = 24;
+
+// The padded, transposed taps and, with `passes`, the factors and whether the kernel
+// is the outer product of them: every tap c[p] r[q] within 2^-48 of itself (flags all
+// 1). The passes' error is then below the direct sum's: at most 2^-50.8 of the result
+// and 2^-49.0 with 10 to 19 taps a side, 2^-49.9 and 2^-46.4 with 40 to 69. The
+// Gaussian's taps are exp(-(x^2 + y^2) / 2 s^2), whose argument (at most 16 before the
+// tail is cut) carries a few roundings of 2^-53 of itself: over 1400 draws of the
+// generator's width at sides from 4 to 130 no tap was off by more than 2^-48.7. A zero
+// or non-finite centre tap fails (its row is not finite), and so does a tap cut to zero.
 __global__ void __launch_bounds__(256)
-k_conv_prepare(const double* __restrict__ k, int kh, int kw, double tol,
+k_conv_prepare(const double* __restrict__ k, int kh, int kw, bool passes,
                double* __restrict__ kt, double* __restrict__ col, double* __restrict__ row,
                int* __restrict__ flags) {
   const int kp = conv_padded_rows(kh);
   const int pc = (kh - 1) / 2, qc = (kw - 1) / 2;
   const int64_t t0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = 256 * kConvFlags;
-  bool outer = true;
+  bool outer = passes;
   for (int64_t t = t0; t < (int64_t)kw * kp; t += step) {
     const int q = (int)(t / kp), p = (int)(t - (int64_t)q * kp) - kConvPadFront;
     const bool in = p >= 0 && p < kh;
     const double x = in ? k[(size_t)p * kw + q] : 0.0;
     kt[t] = x;
-    if (!in) continue;
+    if (!passes || !in) continue;
     const double c = k[(size_t)p * kw + qc], r = k[(size_t)pc * kw + q] / k[(size_t)pc * kw + qc];
-    outer = outer && fabs(x - c * r) <= tol * fabs(x) && isfinite(x);
+    outer = outer && fabs(x - c * r) <= 0x1p-48 * fabs(x) && isfinite(x);
     if (q == qc) col[kh - 1 - p] = c;
     if (p == pc) row[kw - 1 - q] = r;
   }
   outer = __syncthreads_and(outer);
   if (threadIdx.x == 0) flags[blockIdx.x] = outer;
+  if (t0 == 0) flags[kConvFlags] = 0;
 }
 
 __device__ __forceinline__ bool is_outer(const int* __restrict__ flags) {
@@ -227,16 +234,31 @@ __device__ __forceinline__ bool is_outer(const int* __restrict__ flags) {
 }
 
 __device__ __forceinline__ void pad_image(const float* __restrict__ src, int H, int W, ConvPad pd,
-                                          float* __restrict__ pad) {
-  const size_t n = (size_t)pd.Hp * pd.Wp;
-  for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < n;
-       idx += (size_t)gridDim.x * 256) {
-    const int r = (int)(idx / pd.Wp) - pd.PT, c = (int)(idx % pd.Wp) - pd.PL;
-    pad[idx] = (r >= 0 && r < H && c >= 0 && c < W) ? src[(size_t)r * W + c] : 0.0f;
+                                          float* __restrict__ pad, int* __restrict__ nonfinite) {
+  const size_t n = (size_t)pd.Hp * pd.Wp, step = (size_t)gridDim.x * 256;
+  const size_t first = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const int dr = (int)(step / pd.Wp), dc = (int)(step - (size_t)dr * pd.Wp);
+  int r = (int)(first / pd.Wp), c = (int)(first - (size_t)r * pd.Wp);
+  bool bad = false;
+  for (size_t idx = first; idx < n; idx += step) {
+    const int i = r - pd.PT, j = c - pd.PL;
+    const float x = (i >= 0 && i < H && j >= 0 && j < W) ? src[(size_t)i * W + j] : 0.0f;
+    pad[idx] = x;
+    bad = bad || !isfinite(x);
+    r += dr;
+    c += dc;
+    if (c >= pd.Wp) {
+      c -= pd.Wp;
+      ++r;
+    }
   }
+  if (bad) *nonfinite = 1;
 }
 
-// Block b of the direct sum.
+// Block b of the direct sum. FINITE: the zero taps around the kernel may be
+// multiplied by any input; else they are left out, so that an infinite input
+// reaches the outputs of its window only.
+template <bool FINITE>
 __device__ __forceinline__ void convolve_same(const float* __restrict__ pad, int H, int W,
                                               ConvPad pd, const double* __restrict__ kt, int kh,
                                               int kw, float* __restrict__ dst, int b) {
@@ -268,7 +290,11 @@ __device__ __forceinline__ void convolve_same(const float* __restrict__ pad, int
       for (int m = 0; m < R; ++m)    // d = d0 + m
 #pragma unroll
         for (int r = 0; r < R; ++r)  // p = r - d: tap index r - m + R - 1
-          acc[r] = fma(t[r - m + R - 1], x[m], acc[r]);
+        {
+          const double a = fma(t[r - m + R - 1], x[m], acc[r]);
+          const int p = r - d0 - m;
+          acc[r] = FINITE || (p >= 0 && p < kh) ? a : acc[r];
+        }
     }
   }
   if (j < W) {
@@ -387,14 +413,14 @@ __device__ __forceinline__ void conv_rows(const double* __restrict__ tmp, int H,
 
 // Either route's first launch (the column pass; the padded image) and second one
 // (the row pass; the direct sum), each in the blocks it needs. With a launch for
-// each, those not wanted cost 10 us a call: 12 x 12 taps at 128 x 128 take 32 us as
-// an outer product and 40 directly, before 38 and 51.
+// each, those not wanted cost 4 to 10 us a call: 12 x 12 taps at 128 x 128 take 14
+// us as an outer product, 18 then.
 __global__ void __launch_bounds__(256)
 k_conv_first(const float* __restrict__ src, int H, int W, ConvPad pd,
              const double* __restrict__ col, int kh, float* __restrict__ pad,
-             double* __restrict__ tmp, int n_cols, const int* __restrict__ flags) {
-  if (!is_outer(flags))
-    pad_image(src, H, W, pd, pad);
+             double* __restrict__ tmp, bool passes, int n_cols, int* __restrict__ flags) {
+  if (!passes || !is_outer(flags))
+    pad_image(src, H, W, pd, pad, flags + kConvFlags);
   else if ((int)blockIdx.x < n_cols)
     conv_cols(src, H, W, col, kh, tmp, blockIdx.x);
 }
@@ -402,13 +428,16 @@ k_conv_first(const float* __restrict__ src, int H, int W, ConvPad pd,
 __global__ void __launch_bounds__(256)
 k_conv_last(const float* __restrict__ pad, const double* __restrict__ tmp, int H, int W,
             ConvPad pd, const double* __restrict__ kt, const double* __restrict__ row, int kh,
-            int kw, float* __restrict__ dst, int n_rows, int n_direct,
+            int kw, float* __restrict__ dst, bool passes, int n_rows, int n_direct,
             const int* __restrict__ flags) {
   const int b = blockIdx.x;
-  if (is_outer(flags)) {  // uniform over the block, as is b: conv_rows has barriers
+  if (passes && is_outer(flags)) {  // uniform over the block, as is b: conv_rows has barriers
     if (b < n_rows) conv_rows(tmp, H, W, row, kw, dst, b);
   } else if (b < n_direct) {
-    convolve_same(pad, H, W, pd, kt, kh, kw, dst, b);
+    if (flags[kConvFlags] == 0)
+      convolve_same<true>(pad, H, W, pd, kt, kh, kw, dst, b);
+    else
+      convolve_same<false>(pad, H, W, pd, kt, kh, kw, dst, b);
   }
 }
 
@@ -583,18 +612,18 @@ int32_t fk_convolve_same(const float* src, int32_t H, int32_t W, const double* k
   int* flags = (int*)(wk + wo.flag);
   float* pad = (float*)(wk + wo.image);
   double* tmp = (double*)(wk + wo.image);
-  const double tol = std::min(0x1p-48, 0x1p-54 * kh * kw);
-  k_conv_prepare<<<kConvFlags, 256, 0, s>>>(kernel, kh, kw, tol, kt, col, row, flags);
+  const bool passes = (int64_t)kw * ((kh + 2 * kConvRows - 2) / kConvRows) >= kMinPasses;
+  k_conv_prepare<<<kConvFlags, 256, 0, s>>>(kernel, kh, kw, passes, kt, col, row, flags);
   // The host does not know the kernel's values: a launch holds both routes, by the
   // flags.
   const int64_t nc = (int64_t)((W + 63) / 64) * ((H + 4 * kSepR - 1) / (4 * kSepR));
   const int64_t np = std::min<int64_t>(((int64_t)pd.Hp * pd.Wp + 1023) / 1024, 4096);
-  k_conv_first<<<(unsigned)std::max(nc, np), 256, 0, s>>>(src, H, W, pd, col, kh, pad, tmp, (int)nc,
-                                                          flags);
+  k_conv_first<<<(unsigned)std::max(nc, np), 256, 0, s>>>(src, H, W, pd, col, kh, pad, tmp, passes,
+                                                          (int)nc, flags);
   const int64_t nr = (int64_t)((H + 3) / 4) * ((W + kSepSeg - 1) / kSepSeg);
   const int64_t nd = (int64_t)((W + 63) / 64) * ((H + 4 * kConvRows - 1) / (4 * kConvRows));
   k_conv_last<<<(unsigned)std::max(nr, nd), 256, 0, s>>>(pad, tmp, H, W, pd, kt, row, kh, kw, dst,
-                                                         (int)nr, (int)nd, flags);
+                                                         passes, (int)nr, (int)nd, flags);
   HIP_CHECK(hipGetLastError());
   return FK_OK;
 }

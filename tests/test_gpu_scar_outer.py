@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from cardiax_amd import scars
+from oracle import scar_oracle as so
 
 pytestmark = pytest.mark.gpu
 
@@ -29,20 +30,27 @@ def test_taps_are_kept(gpu, n):
     assert np.array_equal(out[inner], np.broadcast_to(expect, out.shape)[inner])
 
 
-@pytest.mark.parametrize("side", [3, 7, 8, 9])
-def test_sides_around_the_rule(gpu, side):
-    """Below and above the 64 taps up to which the bound on a tap grows, a kernel that is an outer product and one that is
-    not, against float64: at most 81 products of values below 1, within 2^-24 of
-    the result's rounding and 2^-46 of the sum."""
-    rng = np.random.default_rng(side)
+@pytest.mark.parametrize("kh,kw", [(3, 3), (9, 9), (2, 24), (3, 11), (3, 12), (10, 8), (60, 2)])
+def test_around_the_rule(gpu, kh, kw):
+    """Kernels below and above the size from which an outer product runs as passes,
+    one that is one and one that is not, against float64: the result's rounding and
+    at most 264 double roundings (2^-44 of the sum)."""
+    rng = np.random.default_rng(kh)
     img = rng.uniform(size=(37, 45)).astype(np.float32)
-    for k in (scars.gauss_kernel(side, 2.0), rng.uniform(size=(side, side))):
+    for k in (np.outer(rng.uniform(0.5, 1.5, kh), rng.uniform(0.5, 1.5, kw)),
+              rng.uniform(size=(kh, kw))):
         out = scars.convolve_same(torch.from_numpy(img).to(gpu), k).cpu().numpy()
-        pad = np.pad(img.astype(np.float64), side)
-        ref = np.zeros(img.shape)
-        o = (side - 1) // 2
-        for p in range(side):
-            for q in range(side):
-                i, j = side + o - p, side + o - q
-                ref += k[p, q] * pad[i:i + img.shape[0], j:j + img.shape[1]]
-        assert np.abs(out - ref).max() <= (2.0 ** -24 + 2.0 ** -46) * np.abs(ref).max()
+        ref = so.convolve_same(img, k)
+        assert np.abs(out - ref).max() <= (2.0 ** -23 + 2.0 ** -44) * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("kh,kw", [(3, 3), (6, 9), (17, 6), (30, 20)])
+@pytest.mark.parametrize("outer", [True, False])
+def test_non_finite_values_stay_in_their_windows(gpu, kh, kw, outer):
+    rng = np.random.default_rng(kw)
+    img = rng.uniform(size=(70, 80)).astype(np.float32)
+    img[0, 3], img[35, 40], img[60, 79] = -np.inf, np.nan, np.inf
+    k = (np.outer(rng.uniform(0.5, 1.5, kh), rng.uniform(0.5, 1.5, kw)) if outer
+         else rng.uniform(0.1, 1.0, size=(kh, kw)))
+    got = scars.convolve_same(torch.from_numpy(img).to(gpu), k).cpu().numpy()
+    np.testing.assert_allclose(got, so.convolve_same(img, k), rtol=2 ** -22, atol=0)
