@@ -451,11 +451,12 @@ def bench_slab(seed, n_steps, size=1024, n_parts=8, depths=(1, 4, 8), tune=True)
     halo exchange every k steps needs (the stencil reaches 4 rows per step).
     The slab's rows come from the middle of the single-tissue workload. GCUPS
     count owned cells only; the ghost rows are the recomputation that k steps
-    between exchanges cost. No exchange is made: there is one GPU."""
+    between exchanges cost. A launch may not pass an exchange, so the kernel is the
+    fastest whose steps per launch divide k. No exchange is made: there is one GPU."""
     import numpy as np
     import torch
 
-    from cardiax_amd import autotune, solve, workloads
+    from cardiax_amd import _lib, autotune, solve, workloads
 
     sim = workloads.c2_inputs(seed, shape=(size, size), steps=n_steps)
     dev = torch.device("cuda", 0)
@@ -469,17 +470,24 @@ def bench_slab(seed, n_steps, size=1024, n_parts=8, depths=(1, 4, 8), tune=True)
         D = torch.from_numpy(np.ascontiguousarray(sim.D[r0:r1])).to(dev)
         stims = [(s.protocol, torch.from_numpy(np.ascontiguousarray(s.field[r0:r1])).to(dev))
                  for s in sim.stimuli]
-        variant = (autotune.tune(shape, n_steps=300)["best"] if tune
-                   else autotune.solve_variant(shape))
+        if tune:
+            times = autotune.tune(shape, n_steps=300)["times_ms"]
+            variant = min((v for v in times if k % KERNELS[v][1] == 0), key=times.get)
+        else:
+            variant = autotune.step_variant(shape) if k % 4 else "tb32x4"
         st0 = solve.init(shape)
-        solve._forward_euler(st0, 0, 200, sim.params, D, stims, sim.dt, sim.dx)  # warm-up
-        torch.cuda.synchronize()
-        stream = torch.cuda.current_stream()
-        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        e0.record(stream)
-        solve._forward_euler(st0, 0, n_steps, sim.params, D, stims, sim.dt, sim.dx)
-        e1.record(stream)
-        torch.cuda.synchronize()
+        prev = _lib.lib().fk_set_forward_variant(_lib.VARIANTS[variant])
+        try:
+            solve._forward_euler(st0, 0, 200, sim.params, D, stims, sim.dt, sim.dx)  # warm-up
+            torch.cuda.synchronize()
+            stream = torch.cuda.current_stream()
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record(stream)
+            solve._forward_euler(st0, 0, n_steps, sim.params, D, stims, sim.dt, sim.dx)
+            e1.record(stream)
+            torch.cuda.synchronize()
+        finally:
+            _lib.lib().fk_set_forward_variant(prev)
         us = e0.elapsed_time(e1) * 1e3 / n_steps
         res["slabs"].append({"steps_per_exchange": k, "rows": shape[0], "variant": variant,
                              "us_per_step": round(us, 3),
