@@ -213,9 +213,9 @@ struct AdjArgs {
 // cotangent 12 in and 12 out, D 4, dL/dD 8: 48 per cell, and the windows' halo
 // rows). It replaced a kernel that kept seven derived fields in memory (104
 // bytes by design, 121-142 measured), two threads per cell:
-// 59.1 us before, 27.6 now per step of 12 problems of 128^2 to 512^2 (1.26 M
+// 59.1 us before, 27.3 now per step of 12 problems of 128^2 to 512^2 (1.26 M
 // cells; 161 registers, three waves per SIMD); 61 us for 3.84 M cells (3.0 TB/s of
-// the 48 bytes); 7.05 and, a wave per row, 6.2 at 256^2, where a launch and an edge
+// the 48 bytes); 7.05 and, a wave per row, 5.7 to 6.0 at 256^2, where a launch and an edge
 // wave's own instructions bound both.
 // XG, YG: a row within 13 of an edge, a column within 13 of a side. In such a
 // band each row, and in such a strip each lane, takes the table or the central
@@ -448,9 +448,9 @@ __device__ __forceinline__ void adj_tile(const Coef& c, const AdjArgs& a, int H,
 
 // Up to this many bands of 2 rows a reverse step runs a wave per row: the waves
 // all run at once and an edge wave's rows, 1.2 us each, set the time. Forward and
-// backward over 200 steps, 2 rows per wave and one: 128^2 2.00 and 1.70 ms, 256^2
-// (640 bands) 2.05 and 1.76, 400^2 (1600) 2.47 and 2.30, 600^2 (3600) 3.39 and 3.56
-// (in the order of strips).
+// backward over 200 steps, 2 rows per wave and one: 128^2 1.79 and 1.54 ms, 256^2
+// (640 bands) 1.83 and 1.61, 400^2 (1600) 2.23 and 2.16, 460^2 (2070) 2.28 and 2.34,
+// 600^2 (3600) 2.96 and 2.99.
 constexpr int kRevRowTiles = 2048;
 
 // Whether the band of R rows at rs, the strip at cs take the edge rules.

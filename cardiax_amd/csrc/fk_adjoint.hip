@@ -79,8 +79,9 @@ k_adj_rev(Coef c, AdjArgs a, int H, int W, StimArgs sa, float dt, float inv_dx2,
 
 // The same with a wave per row, a pair of rows per block. A die takes a run of
 // whole bands across the strips, so that neighbours' windows come from its L2 and
-// the edge strips spread over all dies; forward and backward over 200 steps,
-// strips first in plain order and so: 256^2 1.88 and 1.76 ms, 350^2 2.33 and 2.16,
+// the edge strips spread over all dies; forward and backward over 200 steps
+// (with the rows of a pair still adding their tau terms together), strips first
+// in plain order and so: 256^2 1.88 and 1.76 ms, 350^2 2.33 and 2.16,
 // 400^2 2.32 and 2.30 (runs along a strip: 1.82, 2.19 and 2.46).
 __global__ void __launch_bounds__(128)
 k_adj_rev_row(Coef c, AdjArgs a, int H, int W, StimArgs sa, float dt, float inv_dx2,
