@@ -25,7 +25,9 @@ FK_ERR_NONFINITE = -4
 FK_MAX_STIMULI = 32
 FK_NOALLOC_MAX_CELLS = 1 << 20
 
-# Forward kernel variants (fk_set_forward_variant).
+# Forward kernel variants (fk_set_forward_variant). The block tiles keep the names of the
+# tiles that had these numbers before them: "tb64x2" is 32 rows and 2 steps per launch,
+# "tb64x4" 48 rows and 3, "tb32x2" 64 rows and 3, "tb32x4" 32 rows and 4.
 VARIANTS = {"auto": 0, "plain": 1, "tile16": 2, "tile32": 3, "stream8": 4, "stream16": 5,
             "stream32": 6, "tb64x2": 7, "tb64x4": 8, "tb32x2": 9, "tb32x4": 10,
             "streamc8": 11, "streamc16": 12, "stream4": 13, "streamc4": 14,
